@@ -231,7 +231,7 @@ int sgk_batch_create(int nrep, const SimParams *params, const sgk_config *cfgIn,
     if (cfg.cell_capacity > 64 || cfg.cell_capacity % 8)
         return bfail(nullptr, SGK_E_UNSUPPORTED, "cell capacity must be a multiple of 8 up to 64");
     if (cfg.close_capacity % 8) return bfail(nullptr, SGK_E_UNSUPPORTED, "close capacity must be a multiple of 8");
-    long long sumMe = 0;
+    long long sumAtoms = 0;
     for (int r = 0; r < nrep; ++r) {
         const SimParams &s = params[r];
         if (s.nMol <= 0 || s.nMolMe < 0 || s.nMolMe > s.nMol || s.nMol >= (1 << 24))
@@ -243,7 +243,7 @@ int sgk_batch_create(int nrep, const SimParams *params, const sgk_config *cfgIn,
         if (s.sizeHistRdf <= 0 || s.sizeHistRdf > 8192) return bfail(nullptr, SGK_E_ARG, "RDF bins must be 1..8192");
         if (const char *m = mismatch(s0, s))
             return bfail(nullptr, SGK_E_ARG, "replica " + std::to_string(r) + " differs from replica 0 in " + m);
-        sumMe += s.nMolMe;
+        sumAtoms += s.nMol;
     }
     int ndev = 0;
     if (hipGetDeviceCount(&ndev) != hipSuccess || ndev == 0) return bfail(nullptr, SGK_E_HIP, "no HIP device");
@@ -271,7 +271,7 @@ int sgk_batch_create(int nrep, const SimParams *params, const sgk_config *cfgIn,
     const int G = cfg.metal_lanes;
     const bool fixedG = G == 1 || G == 2 || G == 4 || G == 8 || G == 16;
     for (int r = 0; r < nrep; ++r) b->repLanes.push_back(fixedG ? G : default_lanes(params[r].nMolMe));
-    (void)sumMe;
+    b->nlNine = sumAtoms <= sgk::kNlNineAtoms;
     // replica table and block tables; per-replica workgroup decomposition as in sgk_ctx
     std::vector<int2> atomTab, metalTab, nlTab, nlTabC;
     long long atomOff = 0, metalOff = 0, carbonOff = 0, cellOff = 0, ordOff = 0;
@@ -288,12 +288,15 @@ int sgk_batch_create(int nrep, const SimParams *params, const sgk_config *cfgIn,
         R.cellOff = cellOff;
         const int nbAtom = (s.nMol + 255) / 256;
         const int nbMetal = (s.nMolMe + 255) / 256;
-        const int nbC = (R.p.nC + 255) / 256;
         for (int k = 0; k < nbAtom; ++k) atomTab.push_back(make_int2(r, k));
         for (int k = 0; k < nbMetal; ++k) metalTab.push_back(make_int2(r, k));
-        // cell-ordered list build: kNlMetalLanes lanes per metal atom, then one lane per carbon;
-        // every replica's metal workgroups (the long walks) are dispatched before any carbon one
-        R.nbNlM = (int)(((long long)s.nMolMe * sgk::kNlMetalLanes + 255) / 256);
+        // cell-ordered list build: kNlMetalLanes lanes per metal atom, then one lane per carbon (or
+        // nine lanes for either); every replica's metal workgroups (the long walks) are dispatched
+        // before any carbon one
+        const int nine = sgk::kNineAtoms;
+        R.nbNlM = b->nlNine ? (s.nMolMe + nine - 1) / nine
+                            : (int)(((long long)s.nMolMe * sgk::kNlMetalLanes + 255) / 256);
+        const int nbC = b->nlNine ? (R.p.nC + nine - 1) / nine : (R.p.nC + 255) / 256;
         for (int k = 0; k < R.nbNlM; ++k) nlTab.push_back(make_int2(r, k));
         for (int k = 0; k < nbC; ++k) nlTabC.push_back(make_int2(r, R.nbNlM + k));
         R.ordOff = (int)ordOff;

@@ -95,6 +95,13 @@ namespace sgk {
 // Lanes per metal atom of the cell-ordered list build (each takes two of every 2G candidates; 8
 // measured no faster on the batch and 1.5 % slower on the 1.1 M-atom system).
 constexpr int kNlMetalLanes = 4;
+// Atoms per workgroup of the nine-lane list build (four waves of seven atoms), and the largest system
+// (or batch, atoms of all replicas) that uses it.  The nine-lane build is shorter in latency, the
+// one-lane build in instructions; whole steps at 900-1,000 K, one-lane / nine-lane (us): 1,161 atoms
+// 39.3 / 34.6, 44,353 49.8 / 41.0, 129,120 53.1 / 48.0, 275,880 85.7 / 84.8, 440,000 107.7 / 114.9,
+// 1.1 M 224 / 248; batches of 373,577 atoms 112.9 / 113.0, of 448,542 125.0 / 127.4.
+constexpr int kNineAtoms = 4 * 7;
+constexpr int kNlNineAtoms = 1 << 18;
 }
 
 // Force-pass workgroups of nMe metal atoms at G lanes each.  With the density or force pass
@@ -121,6 +128,7 @@ struct sgk_batch {
     sgk::BatchRep *dReps = nullptr;
     int2 *atomTab = nullptr, *forceTab = nullptr, *metalTab = nullptr, *nlTab = nullptr;
     int nAtomBlocks = 0, nForceBlocks = 0, nMetalBlocks = 0, nNlBlocks = 0;
+    bool nlNine = false;  // nl_scheme 3 with nine lanes per atom (nlTab counts its workgroups)
     // cell-ordered list build (nl_scheme 3): the order of every replica from one counting sort
     int *order = nullptr, *ordCnt = nullptr, *ordKey = nullptr, *ordSlot = nullptr, *ordBlock = nullptr;
     long long nOrdBuckets = 0;

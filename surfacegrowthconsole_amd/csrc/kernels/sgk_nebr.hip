@@ -830,6 +830,305 @@ __device__ __forceinline__ void nlc_body(const DevParams &p, int blk, const type
                    fullNBL);
 }
 
+// ---- nine lanes per atom (nl_scheme 3, systems that do not fill the chip) ----------------------------
+// One lane per carbon and four per metal atom leave a small system waiting on each lane's chain of
+// loads: 9 columns one after another, each its cell counts and then its candidates (per rebuild 62 us
+// for 1,161 atoms on 8 workgroups, 74 us for 44,353, 79 us for 137,940; here 14, 25 and 52).  Nine lanes share an atom, one per column of its
+// 27 cells, seven atoms to a wave.  Each lane tests its column's candidates and keeps the hits as bit
+// masks; a scan over the atom's nine lanes gives the list position of each column's first entry (the
+// columns in table order, so the lists are those of the walks above, bit for bit); each lane then
+// writes its own entries.  The columns' setup and the scans are paid per nine lanes instead of once,
+// so the walks above keep the sizes where the chip is full (kNlNineAtoms).  Bound by its two rounds
+// of dependent loads below ~50 k atoms and by VALU issue above.
+
+// A lane's column: three cells back to back; candidate v is entry v + o of the cell-ordered positions.
+struct NlColumn {
+    int o0, o1, o2, n0, n01, tot;
+    float shx, shy, sz0, sz1, sz2;
+};
+
+// Column q (0..8) of cell c: the offsets 3q, 3q+1 and 3q+2 of the table.
+__device__ __forceinline__ NlColumn nl_column(const DevParams &p, int c, int q, const int *__restrict__ cnt) {
+    const int ccz = c / (p.cx * p.cy);
+    const int ccy = (c - ccz * p.cx * p.cy) / p.cx;
+    const int ccx = c - (ccz * p.cy + ccy) * p.cx;
+    NlColumn k;
+    float tx, ty;
+    const int C0 = stencil_cell<float>(p, ccx, ccy, ccz, 3 * q, k.shx, k.shy, k.sz0);
+    const int C1 = stencil_cell<float>(p, ccx, ccy, ccz, 3 * q + 1, tx, ty, k.sz1);
+    const int C2 = stencil_cell<float>(p, ccx, ccy, ccz, 3 * q + 2, tx, ty, k.sz2);
+    const int cap = p.cellCap;
+    const int n0 = min(cnt[C0], cap), n1 = min(cnt[C1], cap), n2 = min(cnt[C2], cap);
+    k.n0 = n0;
+    k.n01 = n0 + n1;
+    k.tot = n0 + n1 + n2;
+    k.o0 = C0 * cap;  // indices fit 32 bits (ncell * cellCap < 2^31 is checked at set-up)
+    k.o1 = C1 * cap - n0;
+    k.o2 = C2 * cap - k.n01;
+    return k;
+}
+
+// The value of the cell that holds candidate v of a column (cells end at n0, n01 and the column's end).
+template <class T>
+__device__ __forceinline__ T pick3(int v, int n0, int n01, T a, T b, T c) {
+    const T hi = v < n01 ? b : c;
+    return v < n0 ? a : hi;
+}
+
+// Whether candidate (position e, index in e.w) is a neighbour of atom i at A: its index and r^2.
+__device__ __forceinline__ bool nine_test(const float3 &A, int i, float rrN, const float4 &e, float shx, float shy,
+                                          float shz, int &k, float &rr) {
+    k = __float_as_int(e.w);
+    rr = shifted_rr(A, make_float3(e.x, e.y, e.z), shx, shy, shz);
+    return rr < rrN && k != i;
+}
+
+// Inclusive sum over the lanes of an atom up to this one (q = place of the lane among its nine).
+__device__ __forceinline__ int nine_scan(int x, int q) {
+#pragma unroll
+    for (int d = 1; d < 9; d <<= 1) {
+        const int y = __shfl_up(x, d, 64);
+        if (q >= d) x += y;
+    }
+    return x;
+}
+
+// Bit masks of a column's candidates: 32 bits where no column of the wave holds more (the sheet's
+// hold ~12), else 64.
+__device__ __forceinline__ int mask_count(unsigned m) { return __popc(m); }
+__device__ __forceinline__ int mask_count(unsigned long long m) { return __popcll(m); }
+__device__ __forceinline__ int mask_first(unsigned m) { return __ffs((int)m) - 1; }
+__device__ __forceinline__ int mask_first(unsigned long long m) { return __ffsll((long long)m) - 1; }
+__device__ __forceinline__ int mask_last(unsigned m) { return 31 - __clz((int)m); }
+__device__ __forceinline__ int mask_last(unsigned long long m) { return 63 - __clzll((long long)m); }
+
+// Takes the lowest four set bits of m: their places in v (0 past the last), their number returned.
+template <class MASK>
+__device__ __forceinline__ int mask_take4(MASK &m, int (&v)[4]) {
+    int n = 0;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+        v[s] = m ? mask_first(m) : 0;
+        n += m ? 1 : 0;
+        m &= m - MASK(1);
+    }
+    return n;
+}
+
+// Lists of the atom whose column q (candidates described by K) this lane holds; wave-collective.
+// i < 0: no atom.  Candidates past MASK's bits (crowded cells) are counted one by one and tested again when they
+// are written.
+template <bool METAL, bool KEEP, class MASK>
+__device__ __forceinline__ void nine_lists(const DevParams &p, int i, int q, const float3 A, const NlColumn K,
+                                           const float4 *__restrict__ cpos, DevState *st, int *__restrict__ nlM,
+                                           int *__restrict__ nnM, unsigned *__restrict__ lj, int *__restrict__ nlj,
+                                           unsigned *__restrict__ cl, int *__restrict__ ncl, int *__restrict__ fullNN,
+                                           int *__restrict__ fullNBL) {
+    constexpr int BITS = 8 * (int)sizeof(MASK);
+    const int ic = i - p.nMolMe;
+    const float rrN = p.rrNebr, rrC = p.closeR2;
+    const int nMe = p.nMolMe, nlCap = p.nlCap;
+    // plain values: a select between members of the struct would be made in memory
+    const int o0 = K.o0, o1 = K.o1, o2 = K.o2, n0 = K.n0, n01 = K.n01, tot = K.tot;
+    const float shx = K.shx, shy = K.shy, sz0 = K.sz0, sz1 = K.sz1, sz2 = K.sz2;
+#define SGK_ENTRY(v) ((unsigned)((v) + pick3((v), n0, n01, o0, o1, o2)))
+#define SGK_TEST(v) nine_test(A, i, rrN, cpos[SGK_ENTRY(v)], shx, shy, pick3((v), n0, n01, sz0, sz1, sz2), k, rr)
+    // hits among the first BITS candidates; metal and close partners among them (carbons)
+    MASK hit = 0, met = 0, near = 0;
+    const int totM = min(tot, BITS);
+    for (int base = 0; base < totM; base += 4) {
+        float4 P[4];
+        float sz[4];
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            const int v = min(base + s, tot - 1);
+            sz[s] = pick3(v, n0, n01, sz0, sz1, sz2);
+            P[s] = cpos[SGK_ENTRY(v)];
+        }
+        unsigned hb = 0, mb = 0, nb = 0;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            int k;
+            float rr;
+            const bool h = nine_test(A, i, rrN, P[s], shx, shy, sz[s], k, rr) && base + s < tot;
+            hb |= h ? 1u << s : 0u;
+            if (!METAL) {
+                mb |= k < nMe ? 1u << s : 0u;
+                nb |= rr < rrC ? 1u << s : 0u;
+            }
+        }
+        hit |= (MASK)hb << base;
+        if (!METAL) {
+            met |= (MASK)(mb & hb) << base;
+            near |= (MASK)(nb & hb) << base;
+        }
+    }
+    int more = 0;
+    for (int v = BITS; v < tot; ++v) {
+        int k;
+        float rr;
+        if (SGK_TEST(v)) ++more;
+    }
+    const int mine = mask_count(hit) + more;
+    const int upto = nine_scan(mine, q);
+    const int first = upto - mine;  // list position of the column's first hit
+    // a list is cut at its capacity: hits past it are not entries
+    for (int drop = first + mask_count(hit) - nlCap; drop > 0 && hit; --drop) hit &= ~(MASK(1) << mask_last(hit));
+    int err = 0;
+    if (METAL) {
+        int *row = nlM + (size_t)(i < 0 ? 0 : i) * nlCap;
+        int at = first;
+        for (MASK m = hit; m;) {  // four entries a round: their indices are loaded together
+            int v[4], k[4];
+            const int n = mask_take4(m, v);
+#pragma unroll
+            for (int s = 0; s < 4; ++s) k[s] = __float_as_int(cpos[SGK_ENTRY(v[s])].w);
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+                if (s < n) {
+                    row[at + s] = k[s];
+                    if (KEEP) fullNBL[(size_t)(at + s) * p.nMol + i] = k[s];
+                }
+            at += n;
+        }
+        for (int v = BITS; v < tot; ++v) {
+            int k;
+            float rr;
+            if (!SGK_TEST(v)) continue;
+            if (at < nlCap) {
+                row[at] = k;
+                if (KEEP) fullNBL[(size_t)at * p.nMol + i] = k;
+            }
+            ++at;
+        }
+        if (i >= 0 && q == 8) {
+            if (upto > nlCap) err |= SGK_FLAG_NL_OVERFLOW;
+            nl_finish(p, i, true, ic, upto, 0, 0, err, nnM, nullptr, nullptr, fullNN, st);
+        }
+        return;
+    }
+    met &= hit;
+    near &= hit;
+    int moreM = 0, moreN = 0;
+    if (tot > BITS) {
+        int at = first + mask_count(hit);
+        for (int v = BITS; v < tot && at < nlCap; ++v) {
+            int k;
+            float rr;
+            if (!SGK_TEST(v)) continue;
+            ++at;
+            moreM += k < nMe ? 1 : 0;
+            moreN += rr < rrC ? 1 : 0;
+        }
+    }
+    const int mineL = mask_count(met) + moreM, mineN = mask_count(near) + moreN;
+    const int both = nine_scan(mineL | (mineN << 16), q);
+    int atL = (both & 0xffff) - mineL, atN = (both >> 16) - mineN;
+    unsigned *row = cl + (size_t)(i < 0 ? 0 : ic) * p.clCap;
+    for (MASK m = near; m; atN += 4) {
+        int v[4], k[4];
+        const int n = mask_take4(m, v);
+#pragma unroll
+        for (int s = 0; s < 4; ++s) k[s] = __float_as_int(cpos[SGK_ENTRY(v[s])].w);
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+            if (s < n && atN + s < p.clCap)
+                row[atN + s] = ((unsigned)k[s] << 8) | (unsigned)(first + mask_count(hit & ((MASK(1) << v[s]) - MASK(1))));
+    }
+    for (MASK m = met; m; atL += 4) {
+        int v[4], k[4];
+        const int n = mask_take4(m, v);
+#pragma unroll
+        for (int s = 0; s < 4; ++s) k[s] = __float_as_int(cpos[SGK_ENTRY(v[s])].w);
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+            if (s < n && atL + s < p.ljCap)
+                lj[(size_t)(atL + s) * p.nC + ic] =
+                    ((unsigned)k[s] << 8) | (unsigned)(first + mask_count(hit & ((MASK(1) << v[s]) - MASK(1))));
+    }
+    if (tot > BITS) {
+        atL = (both & 0xffff) - moreM;
+        atN = (both >> 16) - moreN;
+        int at = first + mask_count(hit);
+        for (int v = BITS; v < tot && at < nlCap; ++v) {
+            int k;
+            float rr;
+            if (!SGK_TEST(v)) continue;
+            const unsigned ent = ((unsigned)k << 8) | (unsigned)at;
+            if (k < nMe) {
+                if (atL < p.ljCap) lj[(size_t)atL * p.nC + ic] = ent;
+                ++atL;
+            }
+            if (rr < rrC) {
+                if (atN < p.clCap) row[atN] = ent;
+                ++atN;
+            }
+            ++at;
+        }
+    }
+    if (KEEP) {  // reference layout: every hit
+        int at = first;
+        for (int v = 0; v < tot && at < nlCap; ++v) {
+            int k;
+            float rr;
+            if (!SGK_TEST(v)) continue;
+            fullNBL[(size_t)at * p.nMol + i] = k;
+            ++at;
+        }
+    }
+    if (i >= 0 && q == 8) {
+        if (upto > nlCap) err |= SGK_FLAG_NL_OVERFLOW;
+        if ((both & 0xffff) > p.ljCap) err |= SGK_FLAG_LJ_OVERFLOW;
+        if ((both >> 16) > p.clCap) err |= SGK_FLAG_CLOSE_OVERFLOW;
+        nl_finish(p, i, false, ic, upto, both & 0xffff, both >> 16, err, nullptr, nlj, ncl, fullNN, st);
+    }
+#undef SGK_TEST
+#undef SGK_ENTRY
+}
+
+template <bool M, bool METAL, bool KEEP>
+__device__ __forceinline__ void nl9_body(const DevParams &p, int blk, const typename Prec<M>::P4 *__restrict__ pos,
+                                         const CellBufs &bufs, int b, DevState *st, const int *__restrict__ order,
+                                         int *__restrict__ nlM, int *__restrict__ nnM, unsigned *__restrict__ lj,
+                                         int *__restrict__ nlj, unsigned *__restrict__ cl, int *__restrict__ ncl,
+                                         int *__restrict__ fullNN, int *__restrict__ fullNBL) {
+    const int lane = threadIdx.x & 63, g = lane / 9, q = lane - 9 * g;
+    const int t = (blk * 4 + (int)(threadIdx.x >> 6)) * 7 + g;
+    int i = -1;
+    float3 A = make_float3(0.f, 0.f, 0.f);
+    NlColumn K = {0, 0, 0, 0, 0, 0, 0.f, 0.f, 0.f, 0.f, 0.f};
+    if (g < 7 && t < (METAL ? p.nMolMe : p.nC)) {
+        i = METAL ? (order ? order[p.nC + t] : t) : (order ? order[t] : p.nMolMe + t);
+        const int c = bufs.cellOfB(b)[i];
+        if (c >= 0) {  // not binned: empty lists
+            A = f3(pos[i]);
+            K = nl_column(p, c, q, bufs.cntB(b));
+        }
+    }
+    if (__any(K.tot > 32))
+        nine_lists<METAL, KEEP, unsigned long long>(p, i, q, A, K, bufs.cellPos, st, nlM, nnM, lj, nlj, cl, ncl, fullNN,
+                                                    fullNBL);
+    else
+        nine_lists<METAL, KEEP, unsigned>(p, i, q, A, K, bufs.cellPos, st, nlM, nnM, lj, nlj, cl, ncl, fullNN, fullNBL);
+}
+
+template <bool M, bool KEEP>
+__global__ __launch_bounds__(256) void k_nl9(DevParams p, int nbM, const typename Prec<M>::P4 *__restrict__ pos,
+                                             CellBufs bufs, DevState *st, int force, int fromNext,
+                                             const int *__restrict__ order, int *__restrict__ nlM,
+                                             int *__restrict__ nnM, unsigned *__restrict__ lj,
+                                             int *__restrict__ nlj, unsigned *__restrict__ cl,
+                                             int *__restrict__ ncl, int *__restrict__ fullNN,
+                                             int *__restrict__ fullNBL) {
+    if (!force && !st->nebrNow) return;
+    const int b = fromNext ? (st->cellbuf ^ 1) : st->cellbuf;
+    const int bb = blockIdx.x;
+    if (bb < nbM)
+        nl9_body<M, true, KEEP>(p, bb, pos, bufs, b, st, order, nlM, nnM, lj, nlj, cl, ncl, fullNN, fullNBL);
+    else
+        nl9_body<M, false, KEEP>(p, bb - nbM, pos, bufs, b, st, order, nlM, nnM, lj, nlj, cl, ncl, fullNN, fullNBL);
+}
+
 template <bool M, bool KEEP>
 __global__ __launch_bounds__(256) void k_nlc(DevParams p, int nbM, const typename Prec<M>::P4 *__restrict__ pos,
                                              CellBufs bufs, DevState *st, int force, int fromNext,
@@ -1026,6 +1325,26 @@ __global__ __launch_bounds__(256) void kb_nlc(BatchArgs a) {
     else
         nlc_body<M, false>(p, e.y - B.nbNlM, pos, rep_cells(a, B), b, st, order, a.lj + B.carbonOff * p.ljCap,
                            a.nlj + B.carbonOff, a.cl + B.carbonOff * p.clCap, a.ncl + B.carbonOff, nullptr, nullptr);
+}
+
+// Batched, nine lanes per atom: nlTab counts workgroups of kNineAtoms atoms.
+template <bool M>
+__global__ __launch_bounds__(256) void kb_nl9(BatchArgs a) {
+    const int2 e = a.nlTab[blockIdx.x];
+    DevState *st = a.state + e.x;
+    if (!st->nebrNow) return;
+    const BatchRep &B = a.reps[e.x];
+    const DevParams &p = B.p;
+    const int b = st->cellbuf ^ 1;
+    const typename Prec<M>::P4 *pos = (const typename Prec<M>::P4 *)a.pos + B.atomOff;
+    const int *order = a.order ? a.order + B.atomOff : nullptr;
+    if (e.y < B.nbNlM)
+        nl9_body<M, true, false>(p, e.y, pos, rep_cells(a, B), b, st, order, a.nlM + B.metalOff * p.nlCap,
+                                 a.nnM + B.metalOff, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr);
+    else
+        nl9_body<M, false, false>(p, e.y - B.nbNlM, pos, rep_cells(a, B), b, st, order, nullptr, nullptr,
+                                  a.lj + B.carbonOff * p.ljCap, a.nlj + B.carbonOff, a.cl + B.carbonOff * p.clCap,
+                                  a.ncl + B.carbonOff, nullptr, nullptr);
 }
 
 // Make the freshly built buffer current (API path; the step path does this in its reduction).
@@ -1269,19 +1588,28 @@ void launch_nl(sgk_ctx *c, bool force) {
     const unsigned g = blocks_for(c->dp.nMol, 256);
     const int fromNext = force ? 0 : 1;  // step path: build from the new buffer before the commit
     if (c->dp.nlScheme == 3) {
-        const int nbM = (int)blocks_for((long long)c->dp.nMolMe * kNlMetalLanes, 256);
-        const unsigned gc = (unsigned)nbM + blocks_for(c->dp.nC, 256);
+        const bool nine = c->dp.nMol <= kNlNineAtoms;
+        const int nbM = nine ? (int)blocks_for(c->dp.nMolMe, kNineAtoms)
+                             : (int)blocks_for((long long)c->dp.nMolMe * kNlMetalLanes, 256);
+        const unsigned gc = (unsigned)nbM + blocks_for(c->dp.nC, nine ? kNineAtoms : 256);
         const int *order = c->orderValid ? c->nlOrder : nullptr;
-#define SGK_NLC(MM, KK, P4)                                                                                      \
-    hipLaunchKernelGGL((k_nlc<MM, KK>), dim3(gc), dim3(256), 0, c->stream, c->dp, nbM, (const P4 *)c->pos,           \
+#define SGK_NLC(K, MM, KK, P4)                                                                                     \
+    hipLaunchKernelGGL((K<MM, KK>), dim3(gc), dim3(256), 0, c->stream, c->dp, nbM, (const P4 *)c->pos,           \
                        cell_bufs(c), c->state, (int)force, fromNext, order, c->nlM, c->nnM, c->lj, c->nlj, c->cl,  \
                        c->ncl, c->fullNN, c->fullNBL)
-        const bool keep = c->dp.keepFull != 0;
-        if (c->mixed) {
-            if (keep) SGK_NLC(true, true, double4); else SGK_NLC(true, false, double4);
-        } else {
-            if (keep) SGK_NLC(false, true, float4); else SGK_NLC(false, false, float4);
-        }
+#define SGK_NLC_KEEP(MM, P4)                                                                                       \
+    do {                                                                                                           \
+        if (c->dp.keepFull) {                                                                                      \
+            if (nine) SGK_NLC(k_nl9, MM, true, P4); else SGK_NLC(k_nlc, MM, true, P4);                             \
+        } else {                                                                                                   \
+            if (nine) SGK_NLC(k_nl9, MM, false, P4); else SGK_NLC(k_nlc, MM, false, P4);                           \
+        }                                                                                                          \
+    } while (0)
+        if (c->mixed)
+            SGK_NLC_KEEP(true, double4);
+        else
+            SGK_NLC_KEEP(false, float4);
+#undef SGK_NLC_KEEP
 #undef SGK_NLC
         profile_end(c, "nl");
         return;
@@ -1350,10 +1678,17 @@ void build_batch_nl_order(sgk_batch *b) {
 
 void launch_batch_nl(sgk_batch *b) {
     if (b->cfg.nl_scheme == 3 && b->nlTab) {
-        if (b->mixed)
-            hipLaunchKernelGGL(kb_nlc<true>, dim3(b->nNlBlocks), dim3(256), 0, b->stream, b->args());
-        else
-            hipLaunchKernelGGL(kb_nlc<false>, dim3(b->nNlBlocks), dim3(256), 0, b->stream, b->args());
+        const dim3 g(b->nNlBlocks), t(256);
+        if (b->nlNine) {
+            if (b->mixed)
+                hipLaunchKernelGGL(kb_nl9<true>, g, t, 0, b->stream, b->args());
+            else
+                hipLaunchKernelGGL(kb_nl9<false>, g, t, 0, b->stream, b->args());
+        } else if (b->mixed) {
+            hipLaunchKernelGGL(kb_nlc<true>, g, t, 0, b->stream, b->args());
+        } else {
+            hipLaunchKernelGGL(kb_nlc<false>, g, t, 0, b->stream, b->args());
+        }
         return;
     }
     const bool tiled = b->cfg.nl_scheme == 2;
