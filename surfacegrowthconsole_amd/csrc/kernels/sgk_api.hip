@@ -67,7 +67,7 @@ int check_flags(sgk_ctx *c) {
     if (e != hipSuccess) return hip_fail(c, e, "hipMemcpyAsync(state)");
     e = hipStreamSynchronize(c->stream);
     if (e != hipSuccess) return hip_fail(c, e, "hipStreamSynchronize");
-    const int f = c->hostState->errors & kFatal;
+    const int f = (c->hostState->errors | c->hostState->errPrev) & kFatal;
     if (f) return fail(c, (f & SGK_FLAG_DISPLACEMENT) ? SGK_E_DISPLACEMENT : SGK_E_OVERFLOW, "device:" + flag_text(f));
     return SGK_OK;
 }
@@ -385,7 +385,11 @@ int sgk_create(const SimParams *sp, const sgk_config *cfgIn, sgk_ctx **out) {
         SGK_TRY(dalloc(c, &c->rdfSlot, nMe, false));
         SGK_TRY(dalloc(c, &c->rdfPos, nMe, false));
     }
+    SGK_TRY(dalloc(c, (char **)&c->partialsAlt, (nParts + nParts / 64 + 2) * sgk::partial_bytes(c), true));
+    SGK_TRY(dalloc(c, (char **)&c->partVmax, nParts * R, true));
+    SGK_TRY(dalloc(c, (char **)&c->partVmaxAlt, nParts * R, true));
     SGK_TRY(dalloc(c, &c->state, 1, true));
+    SGK_TRY(dalloc(c, &c->stateAlt, 1, true));
     SGK_TRY(dalloc(c, &c->records, (size_t)cfg.records_capacity, true));
     SGK_TRY(dalloc(c, &c->hist, (size_t)p.sizeHistRdf, true));
     if (hipHostMalloc((void **)&c->hostState, sizeof(DevState), 0) != hipSuccess) {
@@ -422,7 +426,7 @@ int sgk_destroy(sgk_ctx *c) {
         if (g.second.exec) (void)hipGraphExecDestroy(g.second.exec);
     void *ptrs[] = {c->pos, c->posAlt, c->vel, c->acc, c->rho, c->embF, c->embDF, c->fric, c->cellOf[0], c->cellOf[1],
                     c->cnt[0], c->cnt[1], c->slots[0], c->slots[1], c->slotOf, c->cellPos, c->nlM, c->nnM, c->lj, c->nlj, c->cl,
-                    c->ncl, c->bondC, c->bondA, c->fullNN, c->fullNBL, c->partials, c->state, c->records, c->hist,
+                    c->ncl, c->bondC, c->bondA, c->fullNN, c->fullNBL, c->partials, c->partialsAlt, c->partVmax, c->partVmaxAlt, c->state, c->stateAlt, c->records, c->hist,
                     c->nlOrder, c->ordCnt, c->ordKey, c->ordSlot, c->ordBlock, c->rdfCnt, c->rdfBlock, c->rdfKey,
                     c->rdfSlot, c->rdfPos};
     for (void *q : ptrs)
@@ -919,33 +923,54 @@ static void enqueue_steps(sgk_ctx *c, const std::string &flags) {
         pre[k] = c->dp.iRegime != 1 && !(b & 3) && k + 1 < n;
         nPre += pre[k];
     }
-    bool unfuseFirst = (nPre & 1) != 0;
-    bool kicked = false, drifted = false;
+    // A fused step with nothing else behind it has no closing launches either: the next step's first
+    // kernel and its force launch close it (StepClose, sgk_reduce.h).  Its state advances into the
+    // other DevState, the next step's partials go to the other array, and an even number of such steps ends the chunk on the state it started from.
+    bool unfuse = (nPre & 1) != 0;
+    std::vector<char> fuse(n, 0), fold(n, 0);
+    int nFold = 0;
+    for (size_t k = 0; k < n; ++k) {
+        if (!pre[k] || !c->posAlt) continue;
+        fuse[k] = !unfuse;
+        unfuse = false;
+        fold[k] = fuse[k] && flags[k] == 'a' && c->stateAlt && c->partVmax;
+        nFold += fold[k];
+    }
+    for (size_t k = 0; (nFold & 1) && k < n; ++k)
+        if (fold[k]) {
+            fold[k] = 0;
+            break;
+        }
+    bool kicked = false, drifted = false, folded = false;
     for (size_t k = 0; k < n; ++k) {
         const int b = flags[k] - 'a';
-        bool fuse = false;
-        if (pre[k] && c->posAlt) {
-            fuse = !unfuseFirst;
-            unfuseFirst = false;
-        }
         sgk::launch_insert(c);  // regime 1 only
-        if (drifted)
+        if (folded)
+            sgk::launch_bin_next(c);
+        else if (drifted)
             sgk::launch_bin(c, false);
         else
             sgk::launch_lf1(c, true, kicked);
         sgk::launch_sortcells(c, false);
         sgk::launch_nl(c, false);
         sgk::launch_rho(c);
-        sgk::launch_force(c, true, true, pre[k], fuse ? c->posAlt : nullptr);
+        sgk::launch_force(c, true, !fold[k], pre[k], fuse[k] ? c->posAlt : nullptr, folded);
+        if (fold[k]) sgk::launch_reduce_chunks(c);
         kicked = pre[k];
-        drifted = fuse;
+        drifted = fuse[k];
+        folded = fold[k];
         if (b & 1) sgk::launch_thermostat(c, 0, 0.0, 0);
         if (b & 2) sgk::launch_shear(c);
         // the samples below read this step's positions, still in pos
         if (b & 4) sgk::launch_rdf(c);
         if (b & 16) sgk::launch_diffuse(c);
         if (b & 8) sgk::launch_adh_obs(c, c->adj->d.part, c->adj->d.adh, 1);
-        if (fuse) std::swap(c->pos, c->posAlt);
+        if (fuse[k]) std::swap(c->pos, c->posAlt);
+        if (fold[k]) {
+            std::swap(c->state, c->stateAlt);
+            std::swap(c->partials, c->partialsAlt);
+            std::swap(c->partVmax, c->partVmaxAlt);
+        }
     }
 }
 

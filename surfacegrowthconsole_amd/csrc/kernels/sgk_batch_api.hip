@@ -69,7 +69,7 @@ int check_batch_flags(sgk_batch *b) {
     const int fatal = SGK_FLAG_CELL_OVERFLOW | SGK_FLAG_NL_OVERFLOW | SGK_FLAG_LJ_OVERFLOW | SGK_FLAG_CLOSE_OVERFLOW |
                       SGK_FLAG_DISPLACEMENT;
     for (int r = 0; r < b->nrep; ++r) {
-        const int f = b->hostState[r].errors & fatal;
+        const int f = (b->hostState[r].errors | b->hostState[r].errPrev) & fatal;
         if (f)
             return bfail(b, (f & SGK_FLAG_DISPLACEMENT) ? SGK_E_DISPLACEMENT : SGK_E_OVERFLOW,
                          "replica " + std::to_string(r) + ": device flags " + std::to_string(f));
@@ -470,6 +470,7 @@ int sgk_batch_set_run_state(sgk_batch *b, int rep, int stepCount, int nebrNow, d
     s.nebrNow = nebrNow ? 1 : 0;
     s.dispHi = dispHi;
     s.errors = 0;
+    s.errPrev = 0;
     s.rec = 0;
     BHIP(b, hipMemcpy(b->state + rep, &s, sizeof(DevState), hipMemcpyHostToDevice));
     if (rep == 0) b->hostStep = stepCount;

@@ -22,19 +22,18 @@ inline CellBufs cell_bufs(sgk_ctx *c) {
 
 // Cell of atom n (position q, float) with the reference's FP32 formula
 // c = VLinear(int((r + L/2) * invWidth)) (SurfaceGrowth.cu:594-600), truncation toward zero, and
-// its slot in the new buffer (cellbuf ^ 1) by atomicAdd.  Slot order is arbitrary; k_sortcells
+// its slot in the new buffer b (cellbuf ^ 1) by atomicAdd.  Slot order is arbitrary; k_sortcells
 // sorts.  Called by every active lane of a wave together (wave-collective).
-__device__ __forceinline__ void bin_atom(const DevParams &p, int n, float3 q, const CellBufs &bufs, DevState *st) {
+__device__ __forceinline__ void bin_atom(const DevParams &p, int n, float3 q, const CellBufs &bufs, int b, int *errors) {
 #pragma clang fp contract(off)
     const float sx = q.x + 0.5f * p.Lx;
     const float sy = q.y + 0.5f * p.Ly;
     const float sz = q.z + 0.5f * p.Lz;
     const int cx = (int)(sx * p.iwx), cy = (int)(sy * p.iwy), cz = (int)(sz * p.iwz);
     const int c = (cz * p.cy + cy) * p.cx + cx;
-    const int b = st->cellbuf ^ 1;
     if (c < 0 || c >= p.ncell) {  // no reference block has this index: the atom is not binned
         bufs.cellOfB(b)[n] = -1;
-        atomicOr(&st->errors, SGK_FLAG_UNBINNED);
+        atomicOr(errors, SGK_FLAG_UNBINNED);
         return;
     }
     bufs.cellOfB(b)[n] = c;
@@ -64,7 +63,7 @@ __device__ __forceinline__ void bin_atom(const DevParams &p, int n, float3 q, co
     if (slot < p.cellCap)
         bufs.slotsB(b)[(size_t)c * p.cellCap + slot] = n;
     else
-        atomicOr(&st->errors, SGK_FLAG_CELL_OVERFLOW);
+        atomicOr(errors, SGK_FLAG_CELL_OVERFLOW);
 }
 
 }  // namespace sgk

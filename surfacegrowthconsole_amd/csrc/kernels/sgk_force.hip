@@ -601,7 +601,7 @@ __device__ __forceinline__ void force_block(const DevParams &p, int b, int nbM, 
                                             float *__restrict__ fric, const unsigned *__restrict__ lj,
                                             const int *__restrict__ nlj, const uint4 *__restrict__ bondC,
                                             const uint4 *__restrict__ bondA, Partial<typename Prec<M>::A> *part,
-                                            int integrate) {
+                                            typename Prec<M>::A *vmax, int integrate) {
     using A = typename Prec<M>::A;
     // Each branch reduces and stores on its own: a Partial merged across the two branches keeps
     // both bodies' registers live at once (154 VGPRs in the FP64 form against 120 apart).
@@ -609,12 +609,18 @@ __device__ __forceinline__ void force_block(const DevParams &p, int b, int nbM, 
         const Partial<A> q = metal_body<M, T, G>(p, xm ? xcd_block(b, nbM) : b, pos, posOut, vel, acc, nlM, nnM, embF,
                                                  embDF, fric, integrate);
         const Partial<A> r = block_reduce_partial<true>(q);
-        if (threadIdx.x == 0) part[b] = r;
+        if (threadIdx.x == 0) {
+            part[b] = r;
+            if (vmax) vmax[b] = r.vmax;
+        }
     } else {
         const Partial<A> q = carbon_body<M, T>(p, xm ? xcd_block(b - nbM, nb - nbM) : b - nbM, pos, posOut, vel, acc,
                                                lj, nlj, bondC, bondA, integrate);
         const Partial<A> r = block_reduce_partial<false>(q);
-        if (threadIdx.x == 0) part[b] = r;
+        if (threadIdx.x == 0) {
+            part[b] = r;
+            if (vmax) vmax[b] = r.vmax;
+        }
     }
 }
 
@@ -627,10 +633,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
                                                float *__restrict__ fric, const unsigned *__restrict__ lj,
                                                const int *__restrict__ nlj, const uint4 *__restrict__ bondC,
                                                const uint4 *__restrict__ bondA, Partial<typename Prec<M>::A> *part,
-                                               int integrate) {
+                                               typename Prec<M>::A *vmax, int integrate,
+                                               StepClose<typename Prec<M>::A> close) {
+    // With a step to close, the first workgroup does that and the others follow it: hardware index
+    // b + 1 runs on XCD (b + 1) % 8, so the ranges below still take whole XCDs (relabelled by one).
+    const int first = close.on ? 1 : 0;
+    if (close.on && blockIdx.x == 0) {
+        close_body(p, close);
+        return;
+    }
     // nbM is a multiple of 8: both ranges keep the XCD of each block
-    force_block<M, T, G>(p, blockIdx.x, nbM, gridDim.x, p.xcdMap & 4, pos, posOut, vel, acc, nlM, nnM, embF, embDF,
-                         fric, lj, nlj, bondC, bondA, part, integrate);
+    force_block<M, T, G>(p, blockIdx.x - first, nbM, gridDim.x - first, p.xcdMap & 4, pos, posOut, vel, acc, nlM, nnM, embF, embDF,
+                         fric, lj, nlj, bondC, bondA, part, vmax, integrate);
 }
 
 // Batched: each replica's workgroups write into its own range of partials (kb_finalize reduces).
@@ -646,7 +660,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
                          (R *)a.vel + 3 * B.atomOff, (R *)a.acc + 3 * B.atomOff, a.nlM + B.metalOff * p.nlCap,
                          a.nnM + B.metalOff, a.embF + B.metalOff, a.embDF + B.metalOff, a.fric + B.metalOff,
                          a.lj + B.carbonOff * p.ljCap, a.nlj + B.carbonOff, a.bondC + B.carbonOff,
-                         a.bondA + B.carbonOff, (Partial<A> *)a.partials + B.partOff, integrate);
+                         a.bondA + B.carbonOff, (Partial<A> *)a.partials + B.partOff, nullptr, integrate);
 }
 
 // ---- launchers ---------------------------------------------------------------------------------
@@ -671,12 +685,25 @@ static void rho_dispatch(sgk_ctx *c) {
 }
 
 template <bool M, class T>
-static void force_dispatch(sgk_ctx *c, int integrate, void *posOut) {
+static void force_dispatch(sgk_ctx *c, int integrate, void *posOut, bool closePrev) {
     using P4 = typename Prec<M>::P4;
     using R = typename Prec<M>::R;
     using A = typename Prec<M>::A;
     const int G = c->metalLanes;
-    const unsigned g = (unsigned)(c->nbM + c->nbC);
+    const int nParts = c->nbM + c->nbC;
+    const unsigned g = (unsigned)nParts + (closePrev ? 1u : 0u);
+    StepClose<A> close = {};
+    if (closePrev) {
+        const bool direct = nParts <= kCloseDirectParts;
+        close.part = (const Partial<A> *)c->partialsAlt + (direct ? 0 : c->part2Off);
+        close.n = direct ? nParts : (nParts + kPartChunk - 1) / kPartChunk;
+        close.direct = direct;
+        close.old = c->stateAlt;
+        close.st = c->state;
+        close.records = c->records;
+        close.recCap = c->cfg.records_capacity;
+        close.on = 1;
+    }
     P4 *pos = (P4 *)c->pos;
     R *vel = (R *)c->vel;
     Partial<A> *part = (Partial<A> *)c->partials;
@@ -684,7 +711,7 @@ static void force_dispatch(sgk_ctx *c, int integrate, void *posOut) {
     hipLaunchKernelGGL((k_force<M, T, GG>), dim3(g), dim3(256), 0, c->stream, c->dp, c->nbM, pos, (P4 *)posOut,  \
                        vel, (R *)c->acc,                                                                        \
                        c->nlM, c->nnM, c->embF, c->embDF, c->fric, c->lj, c->nlj, c->bondC, c->bondA, part,     \
-                       integrate)
+                       (A *)c->partVmax, integrate, close)
     switch (G) {
         case 1: SGK_F(1); break;
         case 2: SGK_F(2); break;
@@ -753,17 +780,17 @@ void launch_batch_rho(sgk_batch *b) { batch_launch(b, false, 0); }
 void launch_batch_force(sgk_batch *b, bool prekick, void *posOut) { batch_launch(b, true, prekick ? 2 : 1, posOut); }
 void launch_batch_force_eval(sgk_batch *b) { batch_launch(b, true, 0); }
 
-void launch_force(sgk_ctx *c, bool integrate, bool finalize, bool prekick, void *posOut) {
+void launch_force(sgk_ctx *c, bool integrate, bool finalize, bool prekick, void *posOut, bool closePrev) {
     if (c->nbM + c->nbC == 0) return;
     profile_begin(c);
     const int mode = integrate ? (prekick ? 2 : 1) : 0;
     if (mode != 2) posOut = nullptr;  // the drift follows the next step's half-kick only
     if (!c->mixed)
-        force_dispatch<false, float>(c, mode, posOut);
+        force_dispatch<false, float>(c, mode, posOut, closePrev);
     else if (c->cfg.pair_fp64)
-        force_dispatch<true, double>(c, mode, posOut);
+        force_dispatch<true, double>(c, mode, posOut, closePrev);
     else
-        force_dispatch<true, float>(c, mode, posOut);
+        force_dispatch<true, float>(c, mode, posOut, closePrev);
     profile_end(c, "force");
     if (finalize) launch_finalize(c, 0);
 }

@@ -64,7 +64,10 @@ struct sgk_ctx {
     int orderAge = 0;                                   // steps run since the order was built
     // reductions and run state
     void *partials = nullptr;
+    void *partVmax = nullptr;                           // v^2 maximum of every force-pass workgroup
+    void *partialsAlt = nullptr, *partVmaxAlt = nullptr;  // swapped with state, below
     sgk::DevState *state = nullptr;
+    sgk::DevState *stateAlt = nullptr;                  // swapped with state inside a chunk of steps, never across one
     sgk_record *records = nullptr;
     unsigned int *hist = nullptr;
     sgk::DevState *hostState = nullptr;                 // pinned mirror
@@ -208,6 +211,8 @@ int prepare_ctx(const SimParams *sp, const sgk_config *cfg, sgk_ctx *c, std::str
 
 // sgk_nebr.hip
 void launch_bin(sgk_ctx *c, bool force);
+// The previous step's closing decision (its state in c->stateAlt), then the binning of a rebuild step.
+void launch_bin_next(sgk_ctx *c);
 void launch_batch_sortcells(sgk_batch *b);
 void launch_batch_nl(sgk_batch *b);
 void build_batch_nl_order(sgk_batch *b);
@@ -228,7 +233,9 @@ void launch_batch_force_eval(sgk_batch *b);  // forces, energies and partials on
 // prekick: the force pass also applies the next step's first half-kick (the caller guarantees that
 // nothing touches velocities or accelerations before that step's launch_lf1(kicked = true)).
 // posOut (with prekick): also drift the positions of the next step into posOut (sgk_force.hip).
-void launch_force(sgk_ctx *c, bool integrate, bool finalize, bool prekick = false, void *posOut = nullptr);
+// closePrev: one more workgroup closes the previous step (its state and partials in the Alt buffers).
+void launch_force(sgk_ctx *c, bool integrate, bool finalize, bool prekick = false, void *posOut = nullptr,
+                  bool closePrev = false);
 // sgk_step.hip
 void launch_lf1(sgk_ctx *c, bool bin, bool kicked = false);
 void launch_insert(sgk_ctx *c);
@@ -241,6 +248,7 @@ void launch_batch_reset_records(sgk_batch *b);
 void launch_lf2(sgk_ctx *c);
 void launch_props(sgk_ctx *c);
 void launch_finalize(sgk_ctx *c, int mode);          // 0 step, 1 evaluate only
+void launch_reduce_chunks(sgk_ctx *c);
 void launch_thermostat(sgk_ctx *c, int stepOverride, double vvOverride, int useOverride);
 void launch_shear(sgk_ctx *c);
 void launch_reset_records(sgk_ctx *c);

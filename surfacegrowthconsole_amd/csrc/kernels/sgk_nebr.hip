@@ -23,6 +23,7 @@
 #include "sgk_cells.h"
 #include "sgk_device.h"
 #include "sgk_internal.h"
+#include "sgk_reduce.h"
 
 namespace sgk {
 
@@ -87,7 +88,44 @@ __global__ void k_bin(DevParams p, const typename Prec<M>::P4 *__restrict__ pos,
     if (!force && !st->nebrNow) return;
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= p.nMol) return;
-    bin_atom(p, i, f3(pos[i]), bufs, st);
+    bin_atom(p, i, f3(pos[i]), bufs, st->cellbuf ^ 1, &st->errors);
+}
+
+// First kernel of a step whose positions the previous force pass drifted and whose previous step has
+// no closing launches (StepClose): every workgroup takes the v^2 maximum of the force pass (its
+// per-workgroup maxima, or the chunk totals: n values `stride` apart) and decides from the old state
+// whether this step rebuilds; the first one writes the advanced state.  Then the binning, on a
+// rebuild.  The launch lasts about as long as k_bin's (4-5 us under the profiler, latency of the
+// maxima and the state); what goes away is the two closing launches.
+template <bool M>
+__global__ __launch_bounds__(256) void k_bin_next(DevParams p, const typename Prec<M>::P4 *__restrict__ pos,
+                                                  CellBufs bufs, const typename Prec<M>::A *__restrict__ vmax, int n,
+                                                  int stride, const DevState *old, DevState *st) {
+    using A = typename Prec<M>::A;
+    __shared__ A sh[4];
+    A v = A(0);
+    for (int k = threadIdx.x; k < n; k += 256) v = OpMax::f(v, vmax[(size_t)k * stride]);
+    v = wave_reduce63<OpMax>(v);
+    if ((threadIdx.x & 63) == 63) sh[threadIdx.x >> 6] = v;
+    __syncthreads();
+    v = OpMax::f(OpMax::f(sh[0], sh[1]), OpMax::f(sh[2], sh[3]));
+    const StepNext<A> s = step_next(p, old, v);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {  // all but errors, which this launch's binning may raise
+        st->step = s.step;
+        st->nebrNow = s.nebrNow;
+        st->cellbuf = s.cellbuf;
+        st->rec = old->rec + 1;
+        st->rebuilds = s.rebuilds;
+        st->dispHi = s.dispHi;
+        st->shear = old->shear;
+        st->shearCount = old->shearCount;
+        st->nMolDeposited = old->nMolDeposited;
+        st->errPrev = old->errPrev | old->errors | (s.displaced ? SGK_FLAG_DISPLACEMENT : 0);
+    }
+    if (!s.nebrNow) return;
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= p.nMol) return;
+    bin_atom(p, i, f3(pos[i]), bufs, s.cellbuf ^ 1, &st->errors);
 }
 
 // Coordinate of the padding entries of the cell-ordered positions: its squared distance to any atom
@@ -1566,6 +1604,26 @@ void launch_bin(sgk_ctx *c, bool force) {
     else
         hipLaunchKernelGGL(k_bin<false>, dim3(g), dim3(256), 0, c->stream, c->dp, (const float4 *)c->pos, cell_bufs(c),
                            c->state, (int)force);
+    profile_end(c, "bin");
+}
+
+void launch_bin_next(sgk_ctx *c) {
+    if (c->dp.nMol == 0) return;
+    profile_begin(c);
+    const unsigned g = blocks_for(c->dp.nMol, 256);
+    const int nParts = c->nbM + c->nbC, nChunks = (nParts + kPartChunk - 1) / kPartChunk;
+    const bool direct = nParts <= kCloseDirectParts;
+#define SGK_BN(MM, P4, A)                                                                                              \
+    hipLaunchKernelGGL(k_bin_next<MM>, dim3(g), dim3(256), 0, c->stream, c->dp, (const P4 *)c->pos, cell_bufs(c),     \
+                       direct ? (const A *)c->partVmaxAlt                                                               \
+                              : &((const Partial<A> *)c->partialsAlt + c->part2Off)->vmax,                             \
+                       direct ? nParts : nChunks, direct ? 1 : (int)(sizeof(Partial<A>) / sizeof(A)), c->stateAlt,  \
+                       c->state)
+    if (c->mixed)
+        SGK_BN(true, double4, double);
+    else
+        SGK_BN(false, float4, float);
+#undef SGK_BN
     profile_end(c, "bin");
 }
 

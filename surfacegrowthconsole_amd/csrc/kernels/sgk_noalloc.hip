@@ -108,6 +108,8 @@ __global__ __launch_bounds__(256) void k_noalloc_init(InitArgs a) {
         s.step = a.step;
         s.nebrNow = 1;
         s.errors = 0;
+        s.errPrev = 0;
+        s.pad = 0;
         s.cellbuf = 0;
         s.rec = 0;
         s.rebuilds = 0;
@@ -122,7 +124,7 @@ __global__ __launch_bounds__(256) void k_noalloc_init(InitArgs a) {
     }
 }
 
-__global__ void k_noalloc_flags(const sgk::DevState *state, int *flags) { *flags = state->errors; }
+__global__ void k_noalloc_flags(const sgk::DevState *state, int *flags) { *flags = state->errors | state->errPrev; }
 
 }  // namespace
 

@@ -65,11 +65,13 @@ struct Partial {
     T vir;  // pair virial 1/2 sum f_ik |d_ik|^2 of the EAM and LJ terms (force pass only)
 };
 
-// Device-resident run state (one per context).
+// Device-resident run state.  A context has two: a step whose closing is folded into the next step
+// leaves its state as it is, and the next step's first kernel writes the advanced state into the
+// other one (k_bin_next), because all of its workgroups still read the old one.
 struct DevState {
     int step;              // stepCount after the last finished step
     int nebrNow;           // rebuild at the next step
-    int errors;            // SGK_FLAG_* bits
+    int errors;            // SGK_FLAG_* bits raised (all of them: errors | errPrev)
     int cellbuf;           // cell buffer holding the current lists (0/1)
     int rec;               // next record slot
     int rebuilds;          // rebuild counter
@@ -80,6 +82,8 @@ struct DevState {
     double cmVelX;         // metal centre-of-mass velocity x of the last step
     unsigned int shearCount;
     int nMolDeposited;     // metal atoms deposited so far (regime 1)
+    int errPrev;           // SGK_FLAG_* bits taken over from the other state (errors: raised since)
+    int pad;
 };
 
 // Grid of the complete-range RDF: cells at least rangeRdf/2 wide, so a pair within range lies within

@@ -86,28 +86,61 @@ __device__ __forceinline__ void reduce_chunk(const Partial<T> *part, int n, Part
     if (lane == 63) *out = q;
 }
 
-// Reduce nParts partials with the whole block (each thread a strided subset, then the block tree:
-// the order is fixed, so the result is bitwise reproducible), then evaluate the reference's host
-// arithmetic of SurfaceGrowth.cu:2307-2395 in thread 0.
-// mode 0: one step - advance the step counter, commit a rebuild, update dispHi / nebrNow / shear,
-//         append a record.  mode 1: evaluation only - write records[0], leave the state alone.
+// The next state's step, rebuild flag and displacement bound after a step with v^2 maximum vmax
+// (SurfaceGrowth.cu:2383-2395); the state itself is only read.  Every kernel that closes a step
+// calls it, so all round alike.
 template <class A>
-__device__ void finalize_body(const DevParams &p, const Partial<A> *part, int nParts, DevState *st,
-                              sgk_record *records, int recCap, int mode) {
+struct StepNext {
+    int step, nebrNow, cellbuf, rebuilds, displaced;
+    double dispHi;
+};
+__device__ __forceinline__ float fmaA(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ __forceinline__ double fmaA(double a, double b, double c) { return __builtin_fma(a, b, c); }
+template <class A>
+__device__ __forceinline__ StepNext<A> step_next(const DevParams &p, const DevState *st, A vmax) {
+    StepNext<A> n;
+    n.step = st->step + 1;
+    A dispHi = (A)st->dispHi;
+    n.cellbuf = st->cellbuf;
+    n.rebuilds = st->rebuilds;
+    if (st->nebrNow) {  // this step rebuilt: the new cell buffer becomes current (SurfaceGrowth.cu:2193-2195)
+        n.cellbuf ^= 1;
+        n.rebuilds += 1;
+        dispHi = A(0);
+    }
+    const A root = (A)sqrt(vmax), dt = (A)p.deltaT;
+    dispHi = fmaA(root, dt, dispHi);  // SurfaceGrowth.cu:2390-2391
+    // the reference's skin rule; a fixed cadence adds rebuilds but never removes one
+    n.nebrNow = dispHi > A(0.5f) * (A)p.rNebrShell;
+    if (p.rebuildEvery > 0 && n.step % p.rebuildEvery == 0) n.nebrNow = 1;
+    n.displaced = (double)fmaA(root, dt, dispHi) > (double)p.dispBound && !n.nebrNow;
+    n.dispHi = (double)dispHi;
+    return n;
+}
+
+// Total of nParts partials, in thread 0: each thread a strided subset, then the block tree (the order
+// is fixed, so the result is bitwise reproducible).
+template <class A>
+__device__ __forceinline__ Partial<A> reduce_parts(const Partial<A> *part, int nParts) {
     Partial<A> q;
     partial_identity(q);
     for (int k = threadIdx.x; k < nParts; k += blockDim.x) partial_combine(q, part[k]);
-    const Partial<A> P = block_reduce_partial(q);
-    if (threadIdx.x != 0) return;
+    return block_reduce_partial(q);
+}
+
+// The sums of a record, with the reference's host arithmetic (SurfaceGrowth.cu:2307-2395); returns the
+// metal's x velocity and the kinetic sum that the thermostat takes.
+template <class A>
+__device__ __forceinline__ void record_sums(const DevParams &p, const Partial<A> &P, sgk_record &rec, A &cmVelX,
+                                            A &vvSum) {
     const int nMe = p.nMolMe, nMol = p.nMol;
-    sgk_record rec;
     rec.shear = 0;
     rec.shearCount = 0;
     // cmVel.val = cmVel.x / nMolMe (SurfaceGrowth.cu:2308)
-    const A cmVelX = nMe ? P.cmv[0] / (A)nMe : A(0);
+    cmVelX = nMe ? P.cmv[0] / (A)nMe : A(0);
     // ComputeVvSumK subtracts cmVel.val from metal vx in regime 2 (SurfaceGrowth.cu:1230-1234):
     // sum m((vx-c)^2+vy^2+vz^2) = sum m|v|^2 - m c sum vx, since sum vx = nMe c.
-    A vvSum = P.vv;
+    vvSum = P.vv;
     if (p.iRegime == 2 && nMe) vvSum = vvSum - (A)p.massMe * cmVelX * P.cmv[0];
     // the metal bounding box includes the reference reduction's zero padding (SurfaceGrowth.cu:1671-1682)
     const bool pad = nMe != 1024 * 1024;
@@ -132,36 +165,42 @@ __device__ void finalize_body(const DevParams &p, const Partial<A> *part, int nP
     rec.uSum = (double)P.u;
     rec.virial = (double)P.vir;
     rec.frict = (p.iRegime != 0 && nMe) ? (double)P.fr : 0.0;
+    rec.pad = 0;
+}
+
+// Reduce nParts partials with the whole block, then evaluate the reference's host arithmetic of
+// SurfaceGrowth.cu:2307-2395 in thread 0.
+// mode 0: one step - advance the step counter, commit a rebuild, update dispHi / nebrNow / shear,
+//         append a record.  mode 1: evaluation only - write records[0], leave the state alone.
+template <class A>
+__device__ void finalize_body(const DevParams &p, const Partial<A> *part, int nParts, DevState *st,
+                              sgk_record *records, int recCap, int mode) {
+    const Partial<A> P = reduce_parts(part, nParts);
+    if (threadIdx.x != 0) return;
+    const int nMe = p.nMolMe;
+    sgk_record rec;
+    A cmVelX, vvSum;
+    record_sums(p, P, rec, cmVelX, vvSum);
     if (mode == 1) {
         rec.step = st->step;
         rec.rebuilt = 0;
         rec.nebrNow = st->nebrNow;
-        rec.errors = st->errors;
+        rec.errors = st->errors | st->errPrev;
         rec.dispHi = st->dispHi;
         rec.nMolDeposited = st->nMolDeposited;
-        rec.pad = 0;
         records[0] = rec;
         return;
     }
-    const int step = st->step + 1;
-    st->step = step;
+    const StepNext<A> n = step_next(p, st, P.vmax);
+    const int step = n.step;
     rec.step = step;
     rec.rebuilt = st->nebrNow;
-    A dispHi = (A)st->dispHi;
-    if (st->nebrNow) {  // this step rebuilt: the new cell buffer becomes current (SurfaceGrowth.cu:2193-2195)
-        const int old = st->cellbuf;
-        st->cellbuf = old ^ 1;
-        st->rebuilds += 1;
-        dispHi = A(0);
-    }
-    const A dstep = (A)sqrt(P.vmax) * (A)p.deltaT;
-    dispHi += dstep;  // SurfaceGrowth.cu:2390-2391
-    // the reference's skin rule; a fixed cadence adds rebuilds but never removes one
-    int nebrNow = dispHi > A(0.5f) * (A)p.rNebrShell;
-    if (p.rebuildEvery > 0 && step % p.rebuildEvery == 0) nebrNow = 1;
-    if ((double)(dispHi + dstep) > (double)p.dispBound && !nebrNow) st->errors |= SGK_FLAG_DISPLACEMENT;
-    st->nebrNow = nebrNow;
-    st->dispHi = (double)dispHi;
+    st->step = step;
+    st->cellbuf = n.cellbuf;
+    st->rebuilds = n.rebuilds;
+    if (n.displaced) st->errors |= SGK_FLAG_DISPLACEMENT;
+    st->nebrNow = n.nebrNow;
+    st->dispHi = n.dispHi;
     st->vvSum = (double)vvSum;
     st->cmVelX = (double)cmVelX;
     st->comX = nMe ? (double)(P.com[0] / (A)nMe) : 0.0;
@@ -174,13 +213,69 @@ __device__ void finalize_body(const DevParams &p, const Partial<A> *part, int nP
         (step - p.stepEquil) % p.stepDeposit == 0)
         st->nMolDeposited += p.nMolToDeposit;
     rec.nMolDeposited = st->nMolDeposited;
-    rec.pad = 0;
     rec.shear = st->shear;
-    rec.nebrNow = nebrNow;
-    rec.dispHi = st->dispHi;
-    rec.errors = st->errors;
+    rec.nebrNow = n.nebrNow;
+    rec.dispHi = n.dispHi;
+    rec.errors = st->errors | st->errPrev;
     if (st->rec < recCap) records[st->rec] = rec;
     st->rec += 1;
+}
+
+// ---- step closing folded into the next step --------------------------------------------------------
+// After a step that no thermostat, shear, deposition or sample follows, nothing needs the step's sums
+// before the next force pass, only its v^2 maximum (the skin rule).  Such a step has no closing
+// launches of its own: the next step's k_bin_next takes the maximum and advances the state into the
+// other DevState, and one workgroup of the next force launch reduces the sums and writes the record
+// while the others work (the force launch, not the density one: its registers cover the reduction, and it
+// is longer than the reduction's ~11 us at 1,000 partials).  The two closing launches cost a small
+// step ~6 us of latency.  Whole step, closed by launches / folded (us): 1,161 atoms 34.6 / 29.0,
+// 44,353 41.4 / 35.2, 137,940 (FP32) 50.3 / 45.3, 1.1 M 224.2 / 223.5.
+constexpr int kCloseLdsChunks = 16;                           // chunk totals kept in LDS
+// Partials closed without k_reduce1: beyond, every workgroup of k_bin_next would read more than 8 KB
+// of maxima and the closing workgroup's chunks would outlast the force launch.
+constexpr int kCloseDirectParts = kCloseLdsChunks * kPartChunk;
+
+template <class A>
+struct StepClose {
+    const Partial<A> *part;  // force-pass partials, or chunk totals (direct = 0)
+    int n, direct;           // their number; 1: reduce the chunks here
+    DevState *old, *st;      // the closed step's state, and the advanced one
+    sgk_record *records;
+    int recCap, on;
+};
+
+// The record of the closed step and the sums of the advanced state; called by one whole workgroup.
+// The sums are those of k_reduce1 and k_finalize, bit for bit.
+template <class A>
+__device__ __forceinline__ void close_body(const DevParams &p, const StepClose<A> &c) {
+    __shared__ Partial<A> tot[kCloseLdsChunks];
+    const Partial<A> *src = c.part;
+    int n = c.n;
+    if (c.direct) {  // as k_reduce1, one wave per chunk
+        n = (c.n + kPartChunk - 1) / kPartChunk;
+        for (int j = threadIdx.x >> 6; j < n; j += (int)blockDim.x >> 6)
+            reduce_chunk(c.part + j * kPartChunk, min(kPartChunk, c.n - j * kPartChunk), tot + j);
+        __syncthreads();
+        src = tot;
+    }
+    const Partial<A> P = reduce_parts(src, n);
+    if (threadIdx.x != 0) return;
+    sgk_record rec;
+    A cmVelX, vvSum;
+    record_sums(p, P, rec, cmVelX, vvSum);
+    rec.step = c.st->step;
+    rec.rebuilt = c.old->nebrNow;
+    rec.nebrNow = c.st->nebrNow;
+    rec.errors = c.st->errPrev;
+    rec.dispHi = c.st->dispHi;
+    rec.shear = c.old->shear;
+    rec.nMolDeposited = c.old->nMolDeposited;
+    const int slot = c.old->rec;
+    if (slot < c.recCap) c.records[slot] = rec;
+    c.st->vvSum = (double)vvSum;
+    c.st->cmVelX = (double)cmVelX;
+    c.st->comX = p.nMolMe ? (double)(P.com[0] / (A)p.nMolMe) : 0.0;
+    c.old->errors = 0;  // taken over into errPrev; this state is the next advance's target
 }
 
 }  // namespace sgk

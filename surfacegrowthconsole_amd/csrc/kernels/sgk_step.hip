@@ -32,7 +32,7 @@ __device__ __forceinline__ void lf1_body(const DevParams &p, int blk, typename P
     auto r = pos[n];
     if (drifted) {
         if (doBin && (rebuild < 0 ? st->nebrNow : rebuild))
-            bin_atom(p, n, make_float3((float)r.x, (float)r.y, (float)r.z), bufs, st);
+            bin_atom(p, n, make_float3((float)r.x, (float)r.y, (float)r.z), bufs, st->cellbuf ^ 1, &st->errors);
         return;
     }
     bool move = true;
@@ -56,7 +56,7 @@ __device__ __forceinline__ void lf1_body(const DevParams &p, int blk, typename P
     drift_wrap<R>(p, r, move, vx, vy, vz);
     pos[n] = r;
     if (doBin && (rebuild < 0 ? st->nebrNow : rebuild))
-        bin_atom(p, n, make_float3((float)r.x, (float)r.y, (float)r.z), bufs, st);
+        bin_atom(p, n, make_float3((float)r.x, (float)r.y, (float)r.z), bufs, st->cellbuf ^ 1, &st->errors);
 }
 
 template <bool M>
@@ -466,6 +466,22 @@ static void finalize_dispatch(sgk_ctx *c, int mode) {
     hipLaunchKernelGGL(k_reduce1<M>, dim3((nChunks + 3) / 4), dim3(256), 0, c->stream, part, nParts, part2);
     hipLaunchKernelGGL(k_finalize<M>, dim3(1), dim3(kFinalizeThreads), 0, c->stream, c->dp, part2, nChunks, c->state,
                        c->records, c->cfg.records_capacity, 0);
+}
+
+// The first reduction stage alone, for a step whose closing is folded into the next one: chunk totals
+// where the partials are too many for the workgroups that take it over.
+void launch_reduce_chunks(sgk_ctx *c) {
+    const int nParts = c->nbM + c->nbC, nChunks = (nParts + kPartChunk - 1) / kPartChunk;
+    if (nParts <= kCloseDirectParts) return;
+    profile_begin(c);
+    const dim3 g((nChunks + 3) / 4), t(256);
+    if (c->mixed)
+        hipLaunchKernelGGL(k_reduce1<true>, g, t, 0, c->stream, (const Partial<double> *)c->partials, nParts,
+                           (Partial<double> *)c->partials + c->part2Off);
+    else
+        hipLaunchKernelGGL(k_reduce1<false>, g, t, 0, c->stream, (const Partial<float> *)c->partials, nParts,
+                           (Partial<float> *)c->partials + c->part2Off);
+    profile_end(c, "reduce");
 }
 
 void launch_finalize(sgk_ctx *c, int mode) {
