@@ -308,6 +308,11 @@ int sgk_batch_create(int nrep, const SimParams *params, const sgk_config *cfgIn,
         cellOff += R.p.ncell;
     }
     nlTab.insert(nlTab.end(), nlTabC.begin(), nlTabC.end());
+    std::vector<int2> rdfTab;
+    const int rdfChunk = sgk::rdf_chunk(metalOff);
+    for (int r = 0; r < nrep; ++r)
+        for (int k = 0; k * rdfChunk < params[r].nMolMe; ++k) rdfTab.push_back(make_int2(r, k));
+    b->nRdfBlocks = (int)rdfTab.size();
     const std::vector<int2> forceTab = force_layout(b);
     size_t tabCap = 0, partCap = 0;
     worst_layout(b, tabCap, partCap);
@@ -329,6 +334,7 @@ int sgk_batch_create(int nrep, const SimParams *params, const sgk_config *cfgIn,
     BTRY(balloc(b, &b->atomTab, atomTab.size(), false));
     BTRY(balloc(b, &b->forceTab, tabCap, false));
     BTRY(balloc(b, &b->metalTab, metalTab.size(), false));
+    BTRY(balloc(b, &b->rdfTab, rdfTab.size(), false));
     if (cfg.nl_scheme == 3) {
         BTRY(balloc(b, &b->nlTab, nlTab.size(), false));
         BTRY(balloc(b, &b->order, (size_t)atomOff, false));
@@ -378,6 +384,9 @@ int sgk_batch_create(int nrep, const SimParams *params, const sgk_config *cfgIn,
                  ? SGK_OK : bfail(b, SGK_E_HIP, "copy of the block table"));
     if (!metalTab.empty())
         BTRY(hipMemcpyAsync(b->metalTab, metalTab.data(), sizeof(int2) * metalTab.size(), hipMemcpyHostToDevice, b->stream) == hipSuccess
+                 ? SGK_OK : bfail(b, SGK_E_HIP, "copy of the block table"));
+    if (!rdfTab.empty())
+        BTRY(hipMemcpyAsync(b->rdfTab, rdfTab.data(), sizeof(int2) * rdfTab.size(), hipMemcpyHostToDevice, b->stream) == hipSuccess
                  ? SGK_OK : bfail(b, SGK_E_HIP, "copy of the block table"));
     if (hipHostMalloc((void **)&b->hostState, sizeof(DevState) * nrep, 0) != hipSuccess) {
         g_batch_create_error = "hipHostMalloc failed";

@@ -105,6 +105,13 @@ constexpr int kNlMetalLanes = 4;
 // 1.1 M 224 / 248; batches of 373,577 atoms 112.9 / 113.0, of 448,542 125.0 / 127.4.
 constexpr int kNineAtoms = 4 * 7;
 constexpr int kNlNineAtoms = 1 << 18;
+// Reference-stencil RDF.
+constexpr int kRdfAtoms = 8;          // atoms a workgroup takes at once
+constexpr int kRdfBlocks = 512;       // workgroups per launch at most: each merges its bins into one histogram
+inline int rdf_chunk(long long nMe) {  // atoms per workgroup (at least one group)
+    const long long groups = (nMe + kRdfAtoms - 1) / kRdfAtoms;
+    return kRdfAtoms * (int)std::max<long long>(1, (groups + kRdfBlocks - 1) / kRdfBlocks);
+}
 }
 
 // Force-pass workgroups of nMe metal atoms at G lanes each.  With the density or force pass
@@ -129,8 +136,8 @@ struct sgk_batch {
     int grpOff[kLaneKinds] = {}, grpN[kLaneKinds] = {};
     std::vector<sgk::BatchRep> reps;  // host copy of the replica table
     sgk::BatchRep *dReps = nullptr;
-    int2 *atomTab = nullptr, *forceTab = nullptr, *metalTab = nullptr, *nlTab = nullptr;
-    int nAtomBlocks = 0, nForceBlocks = 0, nMetalBlocks = 0, nNlBlocks = 0;
+    int2 *atomTab = nullptr, *forceTab = nullptr, *metalTab = nullptr, *nlTab = nullptr, *rdfTab = nullptr;
+    int nAtomBlocks = 0, nForceBlocks = 0, nMetalBlocks = 0, nNlBlocks = 0, nRdfBlocks = 0;
     bool nlNine = false;  // nl_scheme 3 with nine lanes per atom (nlTab counts its workgroups)
     // cell-ordered list build (nl_scheme 3): the order of every replica from one counting sort
     int *order = nullptr, *ordCnt = nullptr, *ordKey = nullptr, *ordSlot = nullptr, *ordBlock = nullptr;
@@ -167,6 +174,7 @@ struct sgk_batch {
         a.forceTab = forceTab;
         a.metalTab = metalTab;
         a.nlTab = nlTab;
+        a.rdfTab = rdfTab;
         a.order = orderValid ? order : nullptr;
         a.pos = pos;
         a.posOut = nullptr;
