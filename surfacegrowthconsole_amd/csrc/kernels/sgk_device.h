@@ -230,6 +230,10 @@ __device__ __forceinline__ double dpp_all(double v) {
 enum : int {
     kQuadSwap1 = 0xB1,  // quad_perm [1,0,3,2]
     kQuadSwap2 = 0x4E,  // quad_perm [2,3,0,1]
+    kRowShr2 = 0x112,
+    kRowShr4 = 0x114,
+    kRowShr8 = 0x118,
+    kRowRor8 = 0x128,
     kRowMirror = 0x140,
     kRowHalfMirror = 0x141,
     kRowBcast15 = 0x142,
@@ -263,6 +267,20 @@ __device__ __forceinline__ T wave_reduce63(T v) {
     v = Op::f(v, dpp_all<kQuadSwap2>(v));
     v = Op::f(v, dpp_all<kRowHalfMirror>(v));
     v = Op::f(v, dpp_all<kRowMirror>(v));
+    v = Op::f(v, dpp<kRowBcast15, 0xA>(e, v));
+    v = Op::f(v, dpp<kRowBcast31, 0xC>(e, v));
+    return v;
+}
+
+// The same where only lanes G - 1, 2G - 1, ... hold something (the last lane of every group of G; the
+// others are not read): the tree of wave_reduce63 without its steps over lanes that hold nothing.
+template <class Op, int G, class T>
+__device__ __forceinline__ T wave_reduce63_of(T v) {
+    const T e = Op::template id<T>();
+    if (G < 2) v = Op::f(v, dpp_all<kQuadSwap1>(v));
+    if (G < 4) v = Op::f(v, G < 2 ? dpp_all<kQuadSwap2>(v) : dpp<kRowShr2, 0xF>(e, v));
+    if (G < 8) v = Op::f(v, dpp<kRowShr4, 0xF>(e, v));
+    if (G < 16) v = Op::f(v, dpp<kRowShr8, 0xF>(e, v));
     v = Op::f(v, dpp<kRowBcast15, 0xA>(e, v));
     v = Op::f(v, dpp<kRowBcast31, 0xC>(e, v));
     return v;

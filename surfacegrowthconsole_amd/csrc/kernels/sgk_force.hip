@@ -276,7 +276,7 @@ __device__ __forceinline__ Partial<typename Prec<M>::A> metal_body(
     w = group_sum<G>(w);
     Partial<A> q;
     partial_identity(q);
-    if (active && l == 0) {
+    if (active && l == G - 1) {  // the group's last lane holds its contribution (block_store_partial)
         const R ax = (R)(fx / (T)p.massMe), ay = (R)(fy / (T)p.massMe), az = (R)(fz / (T)p.massMe);
         if (integrate != 2) {  // after the next step's half-kick here, nothing reads it before it is rewritten
             acc[i] = ax;
@@ -608,19 +608,11 @@ __device__ __forceinline__ void force_block(const DevParams &p, int b, int nbM, 
     if (b < nbM) {
         const Partial<A> q = metal_body<M, T, G>(p, xm ? xcd_block(b, nbM) : b, pos, posOut, vel, acc, nlM, nnM, embF,
                                                  embDF, fric, integrate);
-        const Partial<A> r = block_reduce_partial<true>(q);
-        if (threadIdx.x == 0) {
-            part[b] = r;
-            if (vmax) vmax[b] = r.vmax;
-        }
+        block_store_partial<true, G>(q, part + b, vmax ? vmax + b : nullptr);
     } else {
         const Partial<A> q = carbon_body<M, T>(p, xm ? xcd_block(b - nbM, nb - nbM) : b - nbM, pos, posOut, vel, acc,
                                                lj, nlj, bondC, bondA, integrate);
-        const Partial<A> r = block_reduce_partial<false>(q);
-        if (threadIdx.x == 0) {
-            part[b] = r;
-            if (vmax) vmax[b] = r.vmax;
-        }
+        block_store_partial<false, 1>(q, part + b, vmax ? vmax + b : nullptr);
     }
 }
 

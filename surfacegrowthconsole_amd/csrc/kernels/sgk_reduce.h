@@ -35,34 +35,30 @@ __device__ __forceinline__ void partial_combine(Partial<T> &r, const Partial<T> 
     }
 }
 
-// Wave reduction of a Partial (result in lane 63).  METAL = false reduces only the fields a
-// carbon atom contributes (energy, virial, velocity sums, v^2 max); the others stay at their identity.
-template <bool METAL, class T>
+// Wave reduction of a Partial (result in lane 63).
+template <class T>
 __device__ __forceinline__ void partial_wave(Partial<T> &q) {
     q.u = wave_reduce63<OpSum>(q.u);
     q.vir = wave_reduce63<OpSum>(q.vir);
     q.vv = wave_reduce63<OpSum>(q.vv);
     q.vmax = wave_reduce63<OpMax>(q.vmax);
+    q.fr = wave_reduce63<OpSum>(q.fr);
 #pragma unroll
-    for (int d = 0; d < 3; ++d) q.vs[d] = wave_reduce63<OpSum>(q.vs[d]);
-    if (METAL) {
-        q.fr = wave_reduce63<OpSum>(q.fr);
-#pragma unroll
-        for (int d = 0; d < 3; ++d) {
-            q.com[d] = wave_reduce63<OpSum>(q.com[d]);
-            q.cmv[d] = wave_reduce63<OpSum>(q.cmv[d]);
-            q.bmin[d] = wave_reduce63<OpMin>(q.bmin[d]);
-            q.bmax[d] = wave_reduce63<OpMax>(q.bmax[d]);
-        }
+    for (int d = 0; d < 3; ++d) {
+        q.vs[d] = wave_reduce63<OpSum>(q.vs[d]);
+        q.com[d] = wave_reduce63<OpSum>(q.com[d]);
+        q.cmv[d] = wave_reduce63<OpSum>(q.cmv[d]);
+        q.bmin[d] = wave_reduce63<OpMin>(q.bmin[d]);
+        q.bmax[d] = wave_reduce63<OpMax>(q.bmax[d]);
     }
 }
 
 // Reduce one Partial per thread of the block; thread 0 returns the total (fixed order).  Every
 // thread of the block must call it.
-template <bool METAL = true, class T>
+template <class T>
 __device__ Partial<T> block_reduce_partial(Partial<T> q) {
     __shared__ Partial<T> sh[16];
-    partial_wave<METAL>(q);
+    partial_wave(q);
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = (blockDim.x + 63) >> 6;
     __syncthreads();
     if (lane == 63) sh[w] = q;
@@ -71,6 +67,91 @@ __device__ Partial<T> block_reduce_partial(Partial<T> q) {
     if (threadIdx.x == 0)
         for (int k = 1; k < nw; ++k) partial_combine(r, sh[k]);
     return r;
+}
+
+// The block's Partial into *out and its v^2 maximum into *vmax (if given), for the force pass: one atom
+// per G lanes, its contribution in the group's last lane (METAL), or one carbon per lane (G = 1).
+// The sums are those of block_reduce_partial, bit for bit, by fewer instructions (20 FP64 fields by 6
+// exchange steps each were 8 % of the force pass's VALU work and 2-3 us of a small launch's latency):
+//   metal   the exchange steps within a group are left out, its other lanes hold nothing;
+//   carbon  the six sums are exchanged in halves: after the steps over 2, 4 and 8 lanes a lane holds
+//           one sum over its 8 lanes instead of all six, and the rows of 16 meet in LDS;
+//   both    20 threads combine the waves, one field each, instead of one thread all of them.
+// Force launch at 1.1 M atoms 99.8 -> 96.4 us; whole step 26.0 -> 25.6 us at 1,161 atoms, 35.2 -> 34.2
+// at 44,353, 112.3 -> 110.0 for 64 replicas.
+constexpr int kPartVv = 11, kPartVmax = 12, kPartBmin = 13, kPartBmax = 16, kPartVir = 19, kPartFields = 20;
+
+// Half of a pair of sums: a lane with `hi` keeps b and gives a away, the others the reverse.
+template <int CTRL, class T>
+__device__ __forceinline__ T half_sum(bool hi, T a, T b) {
+    const T keep = hi ? b : a, give = hi ? a : b;
+    return keep + dpp_all<CTRL>(give);
+}
+
+template <bool METAL, int G, class T>
+__device__ __forceinline__ void block_store_partial(Partial<T> q, Partial<T> *out, T *vmax) {
+    static_assert(sizeof(Partial<T>) == kPartFields * sizeof(T), "fields of Partial in their order");
+    __shared__ Partial<T> sh[4];
+    __shared__ T row[4][4][8];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, f = threadIdx.x;
+    if (METAL) {
+        q.u = wave_reduce63_of<OpSum, G>(q.u);
+        q.vir = wave_reduce63_of<OpSum, G>(q.vir);
+        q.vv = wave_reduce63_of<OpSum, G>(q.vv);
+        q.vmax = wave_reduce63_of<OpMax, G>(q.vmax);
+        q.fr = wave_reduce63_of<OpSum, G>(q.fr);
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            q.vs[d] = wave_reduce63_of<OpSum, G>(q.vs[d]);
+            q.com[d] = wave_reduce63_of<OpSum, G>(q.com[d]);
+            q.cmv[d] = wave_reduce63_of<OpSum, G>(q.cmv[d]);
+            q.bmin[d] = wave_reduce63_of<OpMin, G>(q.bmin[d]);
+            q.bmax[d] = wave_reduce63_of<OpMax, G>(q.bmax[d]);
+        }
+        if (lane == 63) sh[w] = q;
+    } else {
+        // a lane's place among its 8 lanes, counted backwards in the upper four: lanes that the
+        // mirror of 8 pairs then hold the same sums
+        const int m = lane & 4 ? ~lane : lane;
+        const bool h1 = m & 1, h2 = m & 2, h4 = lane & 4;
+        const T a0 = half_sum<kQuadSwap1>(h1, q.u, q.vs[0]), a1 = half_sum<kQuadSwap1>(h1, q.vir, q.vs[1]),
+                a2 = half_sum<kQuadSwap1>(h1, q.vv, q.vs[2]);
+        const T b0 = half_sum<kQuadSwap2>(h2, a0, a2);
+        T b1 = a1 + dpp_all<kQuadSwap2>(a1);
+        T c = half_sum<kRowHalfMirror>(h4, b0, b1);
+        c = c + dpp_all<kRowRor8>(c);
+        q.vmax = wave_reduce63<OpMax>(q.vmax);
+        if ((lane & 15) < 8) row[w][lane >> 4][lane & 7] = c;
+        if (lane == 63) sh[w].vmax = q.vmax;
+    }
+    __syncthreads();
+    if (f >= kPartFields) return;
+    T r;
+    if (METAL || f == kPartVmax) {
+        const T *s = (const T *)sh;
+        r = s[f];
+        for (int k = 1; k < 4; ++k) {
+            const T x = s[k * kPartFields + f];
+            if (f >= kPartBmin && f < kPartBmax)
+                r = x < r ? x : r;
+            else if (f == kPartVmax || (f >= kPartBmax && f < kPartVir))
+                r = x > r ? x : r;
+            else
+                r += x;
+        }
+    } else {
+        // field -> the lane of the 8 that holds its sum (-1: a field carbons leave at its identity)
+        const int at = f == 0 ? 0 : f == 8 ? 1 : f == kPartVv ? 2 : f == 10 ? 3 : f == kPartVir ? 7 : f == 9 ? 6 : -1;
+        r = f >= kPartBmin && f < kPartBmax ? T(3.0e38f) : (f >= kPartBmax && f < kPartVir ? T(-3.0e38f) : T(0));
+        if (at >= 0) {
+            for (int k = 0; k < 4; ++k) {
+                const T x = (row[k][3][at] + row[k][2][at]) + (row[k][1][at] + row[k][0][at]);
+                r = k ? r + x : x;
+            }
+        }
+    }
+    ((T *)out)[f] = r;
+    if (vmax && f == kPartVmax) *vmax = r;
 }
 
 // First stage of the step reduction: one wave reduces a chunk of up to kPartChunk partials (lane k
@@ -82,7 +163,7 @@ __device__ __forceinline__ void reduce_chunk(const Partial<T> *part, int n, Part
     Partial<T> q;
     partial_identity(q);
     if (lane < n) q = part[lane];
-    partial_wave<true>(q);
+    partial_wave(q);
     if (lane == 63) *out = q;
 }
 
