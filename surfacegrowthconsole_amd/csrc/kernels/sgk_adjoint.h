@@ -69,7 +69,7 @@ struct Adjoint {
 void adjoint_free(Adjoint *a);
 
 // Kernels (sgk_adjoint.hip).  Mixed-precision contexts only.
-void launch_adh_obs(sgk_ctx *c, double *part, double *out, int recIndex);  // out[st.rec-1] if recIndex
+void launch_adh_obs(sgk_ctx *c, double *part, double *out);
 void launch_adj_rho(sgk_ctx *c, const AdjDev &d);
 void launch_adj_force(sgk_ctx *c, const AdjDev &d, double wE);
 void launch_adj_rho2(sgk_ctx *c, const AdjDev &d);

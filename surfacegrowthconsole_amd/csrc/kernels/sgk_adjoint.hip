@@ -206,17 +206,20 @@ __device__ __forceinline__ void ang_vjp(const DevParams &p, const double (&l)[3]
 }
 
 // ---- kernels ---------------------------------------------------------------------------------------
-// Adhesion energy: block partial sums of the metal-side LJ pair energies.
+// Adhesion energy: block partial sums of the metal-side LJ pair energies, G lanes per atom (the
+// forward's lanes).  One thread per atom took 35 us a step for 561 atoms on 3 workgroups, longer than
+// the step's force pass; now 6.
+template <int G>
 __global__ __launch_bounds__(kBs) void k_adh_part(DevParams p, const double4 *__restrict__ pos,
                                                   const int *__restrict__ nlM, const int *__restrict__ nnM,
                                                   double *__restrict__ part) {
-    const int i = blockIdx.x * kBs + threadIdx.x;
+    const int gt = blockIdx.x * kBs + threadIdx.x, i = gt / G, l = gt % G;
     double e = 0.0;
     if (i < p.nMolMe) {
         const double4 A = pos[i];
         const int *row = nlM + (size_t)i * p.nlCap;
         const int nn = nnM[i];
-        for (int j = 0; j < nn; ++j) {
+        for (int j = l; j < nn; j += G) {
             const int k = row[j];
             if (k < p.nMolMe) continue;
             double d[3];
@@ -228,14 +231,12 @@ __global__ __launch_bounds__(kBs) void k_adh_part(DevParams p, const double4 *__
     if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
 
-// Fixed-order total of the partials into out[st.rec - 1] (the record slot of the step just
-// finished) or out[0].
-__global__ void k_adh_fin(const double *__restrict__ part, int n, double *__restrict__ out, const DevState *st,
-                          int recIndex) {
-    if (threadIdx.x != 0) return;
+// Fixed-order total of the partials into *out.
+__global__ __launch_bounds__(kBs) void k_adh_fin(const double *__restrict__ part, int n, double *__restrict__ out) {
     double s = 0.0;
-    for (int k = 0; k < n; ++k) s += part[k];
-    out[recIndex ? st->rec - 1 : 0] = s;
+    for (int k = threadIdx.x; k < n; k += kBs) s += part[k];
+    s = block_sum(s);
+    if (threadIdx.x == 0) *out = s;
 }
 
 // FP64 density, F' and F'' of every metal atom (EamComputeRhoK, SurfaceGrowth.cu:716-773); G lanes
@@ -646,13 +647,6 @@ AdjArgs adj_args(sgk_ctx *c, const AdjDev &d) {
 }  // namespace
 
 // ---- launchers ---------------------------------------------------------------------------------------
-void launch_adh_obs(sgk_ctx *c, double *part, double *out, int recIndex) {
-    const unsigned g = blocks(std::max(c->dp.nMolMe, 1));
-    hipLaunchKernelGGL(k_adh_part, dim3(g), dim3(kBs), 0, c->stream, c->dp, (const double4 *)c->pos, c->nlM, c->nnM,
-                       part);
-    hipLaunchKernelGGL(k_adh_fin, dim3(1), dim3(64), 0, c->stream, part, (int)g, out, c->state, recIndex);
-}
-
 // Lanes per metal atom of the metal kernels: the context's forward choice (sgk_config.metal_lanes).
 #define SGK_ADJ_G(call)            \
     switch (c->metalLanes) {       \
@@ -662,6 +656,16 @@ void launch_adh_obs(sgk_ctx *c, double *part, double *out, int recIndex) {
         case 16: call(16); break;  \
         default: call(8); break;   \
     }
+
+void launch_adh_obs(sgk_ctx *c, double *part, double *out) {
+    const unsigned g = blocks(std::max<long long>((long long)c->dp.nMolMe * c->metalLanes, 1));
+#define K(G)                                                                                                      \
+    hipLaunchKernelGGL(k_adh_part<G>, dim3(g), dim3(kBs), 0, c->stream, c->dp, (const double4 *)c->pos, c->nlM, \
+                       c->nnM, part)
+    SGK_ADJ_G(K)
+#undef K
+    hipLaunchKernelGGL(k_adh_fin, dim3(1), dim3(kBs), 0, c->stream, part, (int)g, out);
+}
 
 void launch_adj_rho(sgk_ctx *c, const AdjDev &d) {
     if (c->dp.nMolMe == 0) return;

@@ -108,7 +108,8 @@ int alloc_vectors(sgk_ctx *c, Adjoint *a) {
     for (double **v : {&d.rhoBar, &d.rho, &d.dF, &d.ddF}) ADJ_TRY(aalloc(c, a, v, z.nMe));
     ADJ_TRY(aalloc(c, a, &d.pbar, 4));
     ADJ_TRY(aalloc(c, a, &d.therm, 8));
-    ADJ_TRY(aalloc(c, a, &d.part, 4 * ((z.N + 255) / 256) + 8));
+    // thermostat sums (4 per workgroup) or adhesion sums (up to 16 lanes per metal atom)
+    ADJ_TRY(aalloc(c, a, &d.part, std::max(4 * ((z.N + 255) / 256), (16 * z.nMe + 255) / 256) + 8));
     ADJ_TRY(aalloc(c, a, &d.mismatch, 1));
     ADJ_TRY(aalloc(c, a, &d.adh, (size_t)std::max(a->every, 1)));
     return SGK_OK;
@@ -458,7 +459,7 @@ int sgk_adhesion_energy(sgk_ctx *c, double *e) {
     if (!c->haveList) return sgk::set_error(c, SGK_E_STATE, "no neighbour list: call sgk_bin and sgk_build_nebr first");
     ADJ_HIP(c, hipStreamSynchronize(c->stream));
     ADJ_TRY(ensure(c, 0, 0));
-    sgk::launch_adh_obs(c, c->adj->d.part, c->adj->d.adh, 0);
+    sgk::launch_adh_obs(c, c->adj->d.part, c->adj->d.adh);
     ADJ_HIP(c, hipGetLastError());
     ADJ_HIP(c, hipMemcpyAsync(e, c->adj->d.adh, sizeof(double), hipMemcpyDeviceToHost, c->stream));
     ADJ_HIP(c, hipStreamSynchronize(c->stream));

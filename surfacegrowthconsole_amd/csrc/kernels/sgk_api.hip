@@ -933,7 +933,7 @@ static void enqueue_steps(sgk_ctx *c, const std::string &flags) {
         if (!pre[k] || !c->posAlt) continue;
         fuse[k] = !unfuse;
         unfuse = false;
-        fold[k] = fuse[k] && flags[k] == 'a' && c->stateAlt && c->partVmax;
+        fold[k] = fuse[k] && !((flags[k] - 'a') & ~8) && c->stateAlt && c->partVmax;  // 8 takes no sums
         nFold += fold[k];
     }
     for (size_t k = 0; (nFold & 1) && k < n; ++k)
@@ -964,7 +964,7 @@ static void enqueue_steps(sgk_ctx *c, const std::string &flags) {
         // the samples below read this step's positions, still in pos
         if (b & 4) sgk::launch_rdf(c);
         if (b & 16) sgk::launch_diffuse(c);
-        if (b & 8) sgk::launch_adh_obs(c, c->adj->d.part, c->adj->d.adh, 1);
+        if (b & 8) sgk::launch_adh_obs(c, c->adj->d.part, c->adj->d.adh + k);
         if (fuse[k]) std::swap(c->pos, c->posAlt);
         if (fold[k]) {
             std::swap(c->state, c->stateAlt);
