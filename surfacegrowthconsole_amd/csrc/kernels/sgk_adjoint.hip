@@ -343,87 +343,92 @@ __device__ void metal_pairs(const DevParams &p, int i, int gl, int stride, const
 
 // Carbon atom i: bonds, plane, angle terms and LJ with metal (SurfaceGrowth.cu:899-1062), the
 // structure of the force pass's carbon_body: bonds and near neighbours from bondC/bondA, the LJ
-// multiplicity of the reused loop counter.
-__device__ void carbon_vjp(const DevParams &p, int ic, const AdjArgs &a, double (&pb)[4]) {
+// multiplicity of the reused loop counter.  Four lanes per atom (q, a quad): lane q < 3 takes bond
+// q with its two neighbour angles and the central angle of bonds q and q + 1, every lane a quarter
+// of the LJ partners.  One lane per atom is a chain of nine FP64 angle derivatives: k_adj_force took
+// 38 us at 8,625 atoms, 61 at 44,353, 1,161 at 1.1 M; with four 18, 50 and 1,147 (there the atomics bound it).
+// The whole quad is here or not, so its exchanges find their lanes.
+__device__ void carbon_vjp(const DevParams &p, int ic, int q, const AdjArgs &a, double (&pb)[4]) {
+    constexpr int kNext = 0xC9, kPrev = 0xD2;  // quad_perm [1,2,0,3] and [2,0,1,3]: the next and last bond's lane
     const int N = p.nMol, i = p.nMolMe + ic;
     const double l[3] = {a.d.Lam[i], a.d.Lam[N + i], a.d.Lam[2 * N + i]};
     if (l[0] == 0.0 && l[1] == 0.0 && l[2] == 0.0) return;  // frozen, or no cotangent
     const double4 A = a.pos[i];
     const uint4 nbi = a.bondC[ic];
     const int counti = (int)nbi.w;
-    const unsigned be[3] = {nbi.x, nbi.y, nbi.z};
+    const unsigned be = q == 0 ? nbi.x : q == 1 ? nbi.y : nbi.z;
     const int j0 = counti == 3 ? (int)(nbi.z & 255u) : -1;
-    int kb[3];
-    double4 Bk[3];
-    double d[3][3], R[3], gk[3][3];
-    double gi[3] = {0.0, 0.0, 0.0};
-#pragma unroll
-    for (int b = 0; b < 3; ++b) {
-        kb[b] = b < counti ? (int)(be[b] >> 8) : i;
-        Bk[b] = a.pos[kb[b]];
-        R[b] = 1.0;
-        for (int x = 0; x < 3; ++x) gk[b][x] = d[b][x] = 0.0;
-        if (b < counti) R[b] = sqrt(dispd(A, Bk[b], p, d[b]));
-    }
+    const bool bond = q < 3 && q < counti;
+    double d[3] = {0.0, 0.0, 0.0}, R = 1.0, gk[3] = {0.0, 0.0, 0.0}, gi[3] = {0.0, 0.0, 0.0};
+    const int kb = bond ? (int)(be >> 8) : i;
     const double mup = (double)p.mu_p;
-    // neighbour-angle terms: k's first two near neighbours m != i (SurfaceGrowth.cu:940-978)
-#pragma unroll
-    for (int b = 0; b < 3; ++b) {
-        if (b >= counti) break;
-        const uint4 nbk = a.bondA[kb[b] - p.nMolMe];
+    if (bond) {
+        const double4 Bk = a.pos[kb];
+        R = sqrt(dispd(A, Bk, p, d));
+        // neighbour-angle terms: k's first two near neighbours m != i (SurfaceGrowth.cu:940-978)
+        const uint4 nbk = a.bondA[kb - p.nMolMe];
         const unsigned me[3] = {nbk.x, nbk.y, nbk.z};
         const int na = (int)nbk.w;
-        int countk = 0;
+        int ms[2] = {i, i}, nsel = 0;  // picked first: where i sits in k's list differs from lane to lane
 #pragma unroll
         for (int t = 0; t < 3; ++t) {
-            if (t >= na || countk >= 2 || (int)(me[t] >> 8) == i) continue;
             const int m = (int)(me[t] >> 8);
+            if (t < na && m != i) {
+                if (nsel == 0)
+                    ms[0] = m;
+                else if (nsel == 1)
+                    ms[1] = m;
+                ++nsel;
+            }
+        }
+        double4 Bm[2];
+#pragma unroll
+        for (int t = 0; t < 2; ++t) Bm[t] = a.pos[ms[t]];
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            if (t >= nsel) break;
             double e[3];
-            const double rr2 = dispd(Bk[b], a.pos[m], p, e);
+            const double rr2 = dispd(Bk, Bm[t], p, e);
             for (int x = 0; x < 3; ++x) e[x] = -e[x];  // r_m - r_k
             double gd[3], ge[3];
-            na_vjp(p, l, d[b], R[b], e, rr2, gd, ge);
+            na_vjp(p, l, d, R, e, rr2, gd, ge);
             for (int x = 0; x < 3; ++x) {
                 gi[x] += gd[x];
-                gk[b][x] -= gd[x] + ge[x];
+                gk[x] -= gd[x] + ge[x];
             }
             ge[2] += -mup * l[2] / 9.0;  // F_z += -mu_p (z_m - z_0)/9
-            scatter(a.d.G, N, m, 1.0, ge);
-            ++countk;
+            scatter(a.d.G, N, ms[t], 1.0, ge);
         }
     }
     if (counti == 3) {  // SurfaceGrowth.cu:985-1061
         const double mur = (double)p.mu_r, c23 = (double)0.666666667f;
-#pragma unroll
-        for (int b = 0; b < 3; ++b) {
+        const double dn[3] = {dpp_all<kNext>(d[0]), dpp_all<kNext>(d[1]), dpp_all<kNext>(d[2])};
+        const double Rn = dpp_all<kNext>(R);
+        double ga[3] = {0.0, 0.0, 0.0}, gb[3] = {0.0, 0.0, 0.0};
+        if (bond) {
             // F = -mu_r (R-1)/R d
-            const double g = -mur * (1.0 - 1.0 / R[b]), gp = -mur / (R[b] * R[b]);
-            const double P = dot3(l, d[b]);
+            const double g = -mur * (1.0 - 1.0 / R), gp = -mur / (R * R);
+            const double P = dot3(l, d);
             for (int x = 0; x < 3; ++x) {
-                const double v = g * l[x] + gp * P * d[b][x] / R[b];
+                const double v = g * l[x] + gp * P * d[x] / R;
                 gi[x] += v;
-                gk[b][x] -= v;
+                gk[x] -= v;
             }
             // F_z += -(2/3) mu_p (2 (z_i - z_0) - sum_b (z_kb - z_0))
-            gk[b][2] += c23 * mup * l[2];
-        }
-        gi[2] += -2.0 * c23 * mup * l[2];
-#pragma unroll
-        for (int q = 0; q < 3; ++q) {
-            const int ia = q, ib = q == 2 ? 0 : q + 1;
-            double ga[3], gb[3];
-            ang_vjp(p, l, d[ia], R[ia], d[ib], R[ib], ga, gb);
+            gk[2] += c23 * mup * l[2];
+            ang_vjp(p, l, d, R, dn, Rn, ga, gb);
             for (int x = 0; x < 3; ++x) {
                 gi[x] += ga[x] + gb[x];
-                gk[ia][x] -= ga[x];
-                gk[ib][x] -= gb[x];
+                gk[x] -= ga[x];
             }
         }
+        for (int x = 0; x < 3; ++x) gk[x] -= dpp_all<kPrev>(gb[x]);
+        if (q == 0) gi[2] += -2.0 * c23 * mup * l[2];
     }
     // LJ with metal: entries at list positions <= j0 count once, 4..j0 twice, and with j0 = 2
     // position 3 not at all (SurfaceGrowth.cu:989)
     const int nl = a.nlj[ic];
-    for (int qq = 0; qq < nl; ++qq) {
+    for (int qq = q; qq < nl; qq += 4) {
         const unsigned e = a.lj[(size_t)qq * p.nC + ic];
         const int k = (int)(e >> 8), pk = (int)(e & 255u);
         const int mult = j0 < 0 ? 1 : (int)(pk <= j0) + (int)(pk >= 4);
@@ -440,13 +445,12 @@ __device__ void carbon_vjp(const DevParams &p, int ic, const AdjArgs &a, double 
         pb[0] += mult * P * L.fc;
         pb[1] += mult * P * L.sfc;
     }
-    scatter(a.d.G, N, i, 1.0, gi);
-#pragma unroll
-    for (int b = 0; b < 3; ++b)
-        if (b < counti) scatter(a.d.G, N, kb[b], 1.0, gk[b]);
+    for (int x = 0; x < 3; ++x) gi[x] = group_sum<4>(gi[x]);
+    if (q == 0) scatter(a.d.G, N, i, 1.0, gi);
+    if (bond) scatter(a.d.G, N, kb, 1.0, gk);
 }
 
-// blocks [0, nbM): metal atoms, G lanes each; [nbM, nbM + nbC): carbon atoms, one thread each.
+// blocks [0, nbM): metal atoms, G lanes each; [nbM, nbM + nbC): carbon atoms, four lanes each.
 template <int G>
 __global__ __launch_bounds__(kBs) void k_adj_force(DevParams p, AdjArgs a, int nbM, double wE) {
     double pb[4] = {0.0, 0.0, 0.0, 0.0};
@@ -454,8 +458,8 @@ __global__ __launch_bounds__(kBs) void k_adj_force(DevParams p, AdjArgs a, int n
         const int gt = blockIdx.x * kBs + threadIdx.x, i = gt / G;
         metal_vjp<G>(p, i, gt % G, i < p.nMolMe, a, wE, pb);
     } else {
-        const int ic = (blockIdx.x - nbM) * kBs + threadIdx.x;
-        if (ic < p.nC) carbon_vjp(p, ic, a, pb);
+        const int t = (blockIdx.x - nbM) * kBs + threadIdx.x, ic = t / 4;
+        if (ic < p.nC) carbon_vjp(p, ic, t % 4, a, pb);
     }
     add_pbar(a.d.pbar, pb[0], pb[1], pb[2], pb[3]);
 }
@@ -678,7 +682,7 @@ void launch_adj_rho(sgk_ctx *c, const AdjDev &d) {
 }
 
 void launch_adj_force(sgk_ctx *c, const AdjDev &d, double wE) {
-    const int nbM = (int)blocks((long long)c->dp.nMolMe * c->metalLanes), nbC = (int)blocks(c->dp.nC);
+    const int nbM = (int)blocks((long long)c->dp.nMolMe * c->metalLanes), nbC = (int)blocks(4LL * c->dp.nC);
     if (nbM + nbC == 0) return;
 #define K(G) \
     hipLaunchKernelGGL(k_adj_force<G>, dim3(nbM + nbC), dim3(kBs), 0, c->stream, c->dp, adj_args(c, d), nbM, wE)

@@ -37,6 +37,36 @@ def test_adhesion_energy_by_lanes(gpu, ux, uy, metal, lanes):
     assert abs(e - want) <= 1e-12 * abs(want)
 
 
+@pytest.mark.parametrize("metal", [0, 31])
+def test_force_vjp_with_broken_bonds(gpu, metal):
+    """Carbons with 0 to 2 bonds left, beside whole ones: some are lifted out of the sheet.  (Pushed
+    within it they would bring the reference's neighbour-angle cosine, which divides by |e|^2, past 1,
+    where the force law has no value.)"""
+    s, r = _system(4, 3, metal)
+    rng = np.random.default_rng(8)
+    away = s.n_metal + rng.choice(s.n - s.n_metal, 25, replace=False)
+    r[away, 2] -= 1.3
+    o = oracle.Oracle(s.params, "f64")
+    err, nn, nbl = o.neighbour_list(r)
+    assert err == 0
+    abar = rng.standard_normal((s.n, 3))
+    with sg.Engine(s.params, precision="mixed") as eng:
+        eng.upload(r)
+        eng.bin()
+        eng.build_nebr()
+        rbar, pbar = eng.force_vjp(abar, 0.3)
+    dirs = rng.standard_normal((oracle.ND, s.n, 3))
+    _, dacc, _, dadh = o.tangent_forces(r, nn, nbl, rdir=dirs)
+    for k in range(oracle.ND):
+        want = np.sum(abar * dacc[k]) + 0.3 * dadh[k]
+        got = np.sum(rbar * dirs[k])
+        assert abs(got - want) <= 1e-9 * max(np.abs(abar * dacc[k]).sum(), np.abs(rbar * dirs[k]).sum())
+    if metal:
+        _, dacc, _, dadh = o.tangent_forces(r, nn, nbl, pdir=np.eye(4))
+        want = np.einsum("nx,knx->k", abar, dacc) + 0.3 * dadh
+        assert np.allclose(pbar, want, rtol=1e-9, atol=1e-12 * np.abs(want).max())
+
+
 def test_adhesion_record_of_folded_steps(gpu):
     """Segments of one step fold nothing; longer ones fold most steps: same observables, bit for bit."""
     s, r = _system(5, 6, 147)
