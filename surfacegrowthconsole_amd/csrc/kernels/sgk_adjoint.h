@@ -77,6 +77,7 @@ void launch_adj_therm(sgk_ctx *c, const AdjDev &d, const double *velPre, int ste
 void launch_adj_pre(sgk_ctx *c, const AdjDev &d, const double *velPre);
 void launch_adj_post(sgk_ctx *c, const AdjDev &d);
 void launch_adj_lam0(sgk_ctx *c, const AdjDev &d);
+void launch_adj_add(sgk_ctx *c, const AdjDev &d);  // G = Rb + G
 void launch_adj_seed(sgk_ctx *c, const AdjDev &d, double wHeight);
 void launch_adj_cmp(sgk_ctx *c, const AdjDev &d, const void *pos, const void *vel, const void *acc);
 

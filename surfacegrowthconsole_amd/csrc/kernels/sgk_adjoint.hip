@@ -601,6 +601,12 @@ __global__ __launch_bounds__(kBs) void k_adj_lam0(DevParams p, AdjDev d) {
     if (n < p.nMolMe) d.rhoBar[n] = 0.0;
 }
 
+// The gradient with respect to r_0: the sweep's position adjoint plus the initial acceleration's.
+__global__ __launch_bounds__(kBs) void k_adj_add(long long n3, AdjDev d) {
+    const long long t = (long long)blockIdx.x * kBs + threadIdx.x;
+    if (t < n3) d.G[t] = d.Rb[t] + d.G[t];
+}
+
 // Terminal adjoint: d (wH * height) / d r_W = wH / nMolMe on the metal z; zero elsewhere.
 __global__ __launch_bounds__(kBs) void k_adj_seed(DevParams p, AdjDev d, double wH) {
     const int N = p.nMol, n = blockIdx.x * kBs + threadIdx.x;
@@ -717,6 +723,11 @@ void launch_adj_post(sgk_ctx *c, const AdjDev &d) {
 
 void launch_adj_lam0(sgk_ctx *c, const AdjDev &d) {
     hipLaunchKernelGGL(k_adj_lam0, dim3(blocks(c->dp.nMol)), dim3(kBs), 0, c->stream, c->dp, d);
+}
+
+void launch_adj_add(sgk_ctx *c, const AdjDev &d) {
+    const long long n3 = 3LL * c->dp.nMol;
+    hipLaunchKernelGGL(k_adj_add, dim3(blocks(n3)), dim3(kBs), 0, c->stream, n3, d);
 }
 
 void launch_adj_seed(sgk_ctx *c, const AdjDev &d, double wHeight) {

@@ -223,19 +223,15 @@ int check_window(sgk_ctx *c, int nsteps, int every) {
     return SGK_OK;
 }
 
-// Host AoS <-> device SoA for 3-vectors.
+// Host x,y,z per atom <-> device blocks of x, y and z, through the context's stage.
 int upload_vec(sgk_ctx *c, double *dev, const double *host) {
-    const size_t N = (size_t)c->dp.nMol;
-    std::vector<double> t(3 * N);
-    for (size_t i = 0; i < N; ++i)
-        for (int x = 0; x < 3; ++x) t[x * N + i] = host[3 * i + x];
-    ADJ_HIP(c, hipMemcpy(dev, t.data(), 8 * 3 * N, hipMemcpyHostToDevice));
+    ADJ_HIP(c, sgk::state_to_device<double>(c->stage, c->device, c->stream, (size_t)c->dp.nMol, true, nullptr, host, nullptr,
+                                            nullptr, dev, nullptr));
     return SGK_OK;
 }
-int download_vec(sgk_ctx *c, std::vector<double> &t, const double *dev) {
-    const size_t N = (size_t)c->dp.nMol;
-    t.resize(3 * N);
-    ADJ_HIP(c, hipMemcpy(t.data(), dev, 8 * 3 * N, hipMemcpyDeviceToHost));
+int download_vec(sgk_ctx *c, const double *dev, double *host) {
+    ADJ_HIP(c, sgk::state_to_host<double>(c->stage, c->device, c->stream, (size_t)c->dp.nMol, true, nullptr, dev, nullptr,
+                                          nullptr, host, nullptr));
     return SGK_OK;
 }
 
@@ -383,19 +379,10 @@ int sgk_adjoint_backward(sgk_ctx *c, const double *w, double *grad, double *dr0,
     ADJ_HIP(c, hipMemcpyAsync(grad, d.pbar, 4 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
     ADJ_HIP(c, hipMemcpyAsync(&a->mismatches, d.mismatch, sizeof(int), hipMemcpyDeviceToHost, c->stream));
     ADJ_HIP(c, hipStreamSynchronize(c->stream));
-    if (dv0 || dr0) {
-        std::vector<double> V, R, G;
-        if (dv0) {
-            ADJ_TRY(download_vec(c, V, d.Vb));
-            for (size_t i = 0; i < N; ++i)
-                for (int x = 0; x < 3; ++x) dv0[3 * i + x] = V[x * N + i];
-        }
-        if (dr0) {
-            ADJ_TRY(download_vec(c, R, d.Rb));
-            ADJ_TRY(download_vec(c, G, d.G));
-            for (size_t i = 0; i < N; ++i)
-                for (int x = 0; x < 3; ++x) dr0[3 * i + x] = R[x * N + i] + G[x * N + i];
-        }
+    if (dv0) ADJ_TRY(download_vec(c, d.Vb, dv0));
+    if (dr0) {
+        sgk::launch_adj_add(c, d);  // G += Rb: the sweep is over, nothing reads G again
+        ADJ_TRY(download_vec(c, d.G, dr0));
     }
     ADJ_TRY(restore(c, a->ck.back()));  // leave the context where the forward ended
     ADJ_HIP(c, hipEventRecord(a->ev1, c->stream));
@@ -440,12 +427,7 @@ int sgk_force_vjp(sgk_ctx *c, const double *abar, double wAdh, double *rbar, dou
     enqueue_vjp(c, d, wAdh);
     ADJ_HIP(c, hipGetLastError());
     ADJ_HIP(c, hipStreamSynchronize(c->stream));
-    if (rbar) {
-        std::vector<double> G;
-        ADJ_TRY(download_vec(c, G, d.G));
-        for (size_t i = 0; i < N; ++i)
-            for (int x = 0; x < 3; ++x) rbar[3 * i + x] = G[x * N + i];
-    }
+    if (rbar) ADJ_TRY(download_vec(c, d.G, rbar));
     if (pbar) {
         ADJ_HIP(c, hipMemcpyAsync(pbar, d.pbar, 4 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
         ADJ_HIP(c, hipStreamSynchronize(c->stream));

@@ -432,6 +432,7 @@ int sgk_destroy(sgk_ctx *c) {
     for (void *q : ptrs)
         if (q) (void)hipFree(q);
     if (c->diffMem) (void)hipFree(c->diffMem);
+    sgk::stage_free(c->stage);
     if (c->hostState) (void)hipHostFree(c->hostState);
     if (c->ev0) (void)hipEventDestroy(c->ev0);
     if (c->ev1) (void)hipEventDestroy(c->ev1);
@@ -441,164 +442,41 @@ int sgk_destroy(sgk_ctx *c) {
 }
 
 // ---- state transfer --------------------------------------------------------------------------------
+static void positions_replaced(sgk_ctx *c) {
+    c->haveList = false;
+    c->haveCells = false;
+    c->orderValid = false;
+}
+
 int sgk_upload(sgk_ctx *c, const sg_float4 *r, const sg_float3 *v, const sg_float3 *a) {
     if (!c) return SGK_E_ARG;
     const size_t n = (size_t)c->dp.nMol;
-    if (r) {
-        if (c->mixed) {
-            std::vector<double> t(4 * n);
-            for (size_t i = 0; i < n; ++i) {
-                t[4 * i] = r[i].x;
-                t[4 * i + 1] = r[i].y;
-                t[4 * i + 2] = r[i].z;
-                t[4 * i + 3] = r[i].w;
-            }
-            SGK_HIP(c, hipMemcpy(c->pos, t.data(), 32 * n, hipMemcpyHostToDevice));
-        } else {
-            SGK_HIP(c, hipMemcpy(c->pos, r, 16 * n, hipMemcpyHostToDevice));
-        }
-        c->haveList = false;
-        c->haveCells = false;
-        c->orderValid = false;
-    }
-    if (v) {
-        if (c->mixed) {
-            std::vector<double> t(3 * n);
-            for (size_t i = 0; i < n; ++i) {
-                t[i] = v[i].x;
-                t[n + i] = v[i].y;
-                t[2 * n + i] = v[i].z;
-            }
-            SGK_HIP(c, hipMemcpy(c->vel, t.data(), 8 * 3 * n, hipMemcpyHostToDevice));
-        } else {
-            std::vector<float> t(3 * n);
-            for (size_t i = 0; i < n; ++i) {
-                t[i] = v[i].x;
-                t[n + i] = v[i].y;
-                t[2 * n + i] = v[i].z;
-            }
-            SGK_HIP(c, hipMemcpy(c->vel, t.data(), 4 * 3 * n, hipMemcpyHostToDevice));
-        }
-    }
-    if (a) {
-        if (c->mixed) {
-            std::vector<double> t(3 * n);
-            for (size_t i = 0; i < n; ++i) {
-                t[i] = a[i].x;
-                t[n + i] = a[i].y;
-                t[2 * n + i] = a[i].z;
-            }
-            SGK_HIP(c, hipMemcpy(c->acc, t.data(), 8 * 3 * n, hipMemcpyHostToDevice));
-        } else {
-            std::vector<float> t(3 * n);
-            for (size_t i = 0; i < n; ++i) {
-                t[i] = a[i].x;
-                t[n + i] = a[i].y;
-                t[2 * n + i] = a[i].z;
-            }
-            SGK_HIP(c, hipMemcpy(c->acc, t.data(), 4 * 3 * n, hipMemcpyHostToDevice));
-        }
-    }
+    const float *R = (const float *)r, *V = (const float *)v, *A = (const float *)a;
+    SGK_HIP(c, sgk::state_to_device(c->stage, c->device, c->stream, n, c->mixed, R, V, A, c->pos, c->vel, c->acc));
+    if (r) positions_replaced(c);
     return SGK_OK;
 }
 
 int sgk_upload_f64(sgk_ctx *c, const double *r, const double *v, const double *a) {
     if (!c) return SGK_E_ARG;
     const size_t n = (size_t)c->dp.nMol;
-    if (r) {
-        if (c->mixed) {
-            SGK_HIP(c, hipMemcpy(c->pos, r, 32 * n, hipMemcpyHostToDevice));
-        } else {
-            std::vector<float> t(4 * n);
-            for (size_t i = 0; i < 4 * n; ++i) t[i] = (float)r[i];
-            SGK_HIP(c, hipMemcpy(c->pos, t.data(), 16 * n, hipMemcpyHostToDevice));
-        }
-        c->haveList = false;
-        c->haveCells = false;
-        c->orderValid = false;
-    }
-    if (v) {
-        if (c->mixed) {
-            std::vector<double> t(3 * n);
-            for (size_t i = 0; i < n; ++i)
-                for (int d = 0; d < 3; ++d) t[d * n + i] = v[3 * i + d];
-            SGK_HIP(c, hipMemcpy(c->vel, t.data(), 8 * 3 * n, hipMemcpyHostToDevice));
-        } else {
-            std::vector<float> t(3 * n);
-            for (size_t i = 0; i < n; ++i)
-                for (int d = 0; d < 3; ++d) t[d * n + i] = (float)v[3 * i + d];
-            SGK_HIP(c, hipMemcpy(c->vel, t.data(), 4 * 3 * n, hipMemcpyHostToDevice));
-        }
-    }
-    if (a) {
-        if (c->mixed) {
-            std::vector<double> t(3 * n);
-            for (size_t i = 0; i < n; ++i)
-                for (int d = 0; d < 3; ++d) t[d * n + i] = a[3 * i + d];
-            SGK_HIP(c, hipMemcpy(c->acc, t.data(), 8 * 3 * n, hipMemcpyHostToDevice));
-        } else {
-            std::vector<float> t(3 * n);
-            for (size_t i = 0; i < n; ++i)
-                for (int d = 0; d < 3; ++d) t[d * n + i] = (float)a[3 * i + d];
-            SGK_HIP(c, hipMemcpy(c->acc, t.data(), 4 * 3 * n, hipMemcpyHostToDevice));
-        }
-    }
+    SGK_HIP(c, sgk::state_to_device(c->stage, c->device, c->stream, n, c->mixed, r, v, a, c->pos, c->vel, c->acc));
+    if (r) positions_replaced(c);
     return SGK_OK;
 }
 
 int sgk_download_f64(sgk_ctx *c, double *r, double *v, double *a) {
     if (!c) return SGK_E_ARG;
-    SGK_HIP(c, hipStreamSynchronize(c->stream));
     const size_t n = (size_t)c->dp.nMol;
-    if (r) {
-        if (c->mixed) {
-            SGK_HIP(c, hipMemcpy(r, c->pos, 32 * n, hipMemcpyDeviceToHost));
-        } else {
-            std::vector<float> t(4 * n);
-            SGK_HIP(c, hipMemcpy(t.data(), c->pos, 16 * n, hipMemcpyDeviceToHost));
-            for (size_t i = 0; i < 4 * n; ++i) r[i] = t[i];
-        }
-    }
-    if (v) {
-        if (c->mixed) {
-            std::vector<double> t(3 * n);
-            SGK_HIP(c, hipMemcpy(t.data(), c->vel, 8 * 3 * n, hipMemcpyDeviceToHost));
-            for (size_t i = 0; i < n; ++i)
-                for (int d = 0; d < 3; ++d) v[3 * i + d] = t[d * n + i];
-        } else {
-            std::vector<float> t(3 * n);
-            SGK_HIP(c, hipMemcpy(t.data(), c->vel, 4 * 3 * n, hipMemcpyDeviceToHost));
-            for (size_t i = 0; i < n; ++i)
-                for (int d = 0; d < 3; ++d) v[3 * i + d] = t[d * n + i];
-        }
-    }
-    if (a) {
-        if (c->mixed) {
-            std::vector<double> t(3 * n);
-            SGK_HIP(c, hipMemcpy(t.data(), c->acc, 8 * 3 * n, hipMemcpyDeviceToHost));
-            for (size_t i = 0; i < n; ++i)
-                for (int d = 0; d < 3; ++d) a[3 * i + d] = t[d * n + i];
-        } else {
-            std::vector<float> t(3 * n);
-            SGK_HIP(c, hipMemcpy(t.data(), c->acc, 4 * 3 * n, hipMemcpyDeviceToHost));
-            for (size_t i = 0; i < n; ++i)
-                for (int d = 0; d < 3; ++d) a[3 * i + d] = t[d * n + i];
-        }
-    }
+    SGK_HIP(c, sgk::state_to_host(c->stage, c->device, c->stream, n, c->mixed, c->pos, c->vel, c->acc, r, v, a));
     return SGK_OK;
 }
 
 int sgk_download(sgk_ctx *c, sg_float4 *r, sg_float3 *v, sg_float3 *a) {
     if (!c) return SGK_E_ARG;
     const size_t n = (size_t)c->dp.nMol;
-    std::vector<double> R(r ? 4 * n : 0), V(v ? 3 * n : 0), A(a ? 3 * n : 0);
-    int rc = sgk_download_f64(c, r ? R.data() : nullptr, v ? V.data() : nullptr, a ? A.data() : nullptr);
-    if (rc) return rc;
-    for (size_t i = 0; i < n; ++i) {
-        if (r) r[i] = {(float)R[4 * i], (float)R[4 * i + 1], (float)R[4 * i + 2], (float)R[4 * i + 3]};
-        if (v) v[i] = {(float)V[3 * i], (float)V[3 * i + 1], (float)V[3 * i + 2]};
-        if (a) a[i] = {(float)A[3 * i], (float)A[3 * i + 1], (float)A[3 * i + 2]};
-    }
+    float *R = (float *)r, *V = (float *)v, *A = (float *)a;
+    SGK_HIP(c, sgk::state_to_host(c->stage, c->device, c->stream, n, c->mixed, c->pos, c->vel, c->acc, R, V, A));
     return SGK_OK;
 }
 
@@ -735,31 +613,20 @@ int sgk_compute_forces(sgk_ctx *c) {
 
 int sgk_get_rho(sgk_ctx *c, double *rho) {
     if (!c || !rho) return SGK_E_ARG;
-    SGK_HIP(c, hipStreamSynchronize(c->stream));
-    std::vector<float> t(std::max(c->dp.nMolMe, 1));
-    SGK_HIP(c, hipMemcpy(t.data(), c->rho, 4 * (size_t)c->dp.nMolMe, hipMemcpyDeviceToHost));
-    for (int i = 0; i < c->dp.nMolMe; ++i) rho[i] = t[i];
+    const sgk::XferArray x = {rho, c->rho, (size_t)c->dp.nMolMe, sgk::XferLayout::plain, false};
+    SGK_HIP(c, sgk::xfer_to_host<double>(c->stage, c->device, c->stream, &x, 1));
     return SGK_OK;
 }
 
 int sgk_get_forces(sgk_ctx *c, double *acc, double *energy, double *fric) {
     if (!c) return SGK_E_ARG;
     const size_t n = (size_t)c->dp.nMol;
-    if (acc) {
-        int rc = sgk_download_f64(c, nullptr, nullptr, acc);
-        if (rc) return rc;
-    }
-    if (energy) {
-        std::vector<double> r(4 * n);
-        int rc = sgk_download_f64(c, r.data(), nullptr, nullptr);
-        if (rc) return rc;
-        for (size_t i = 0; i < n; ++i) energy[i] = r[4 * i + 3];
-    }
-    if (fric && c->dp.nMolMe) {
-        std::vector<float> t(c->dp.nMolMe);
-        SGK_HIP(c, hipMemcpy(t.data(), c->fric, 4 * (size_t)c->dp.nMolMe, hipMemcpyDeviceToHost));
-        for (int i = 0; i < c->dp.nMolMe; ++i) fric[i] = t[i];
-    }
+    sgk::XferArray x[3];
+    int k = 0;
+    if (acc) x[k++] = {acc, c->acc, 3 * n, sgk::XferLayout::blocks, c->mixed != 0};
+    if (energy) x[k++] = {energy, c->pos, n, sgk::XferLayout::energy, c->mixed != 0};
+    if (fric) x[k++] = {fric, c->fric, (size_t)c->dp.nMolMe, sgk::XferLayout::plain, false};
+    SGK_HIP(c, sgk::xfer_to_host<double>(c->stage, c->device, c->stream, x, k));
     return SGK_OK;
 }
 

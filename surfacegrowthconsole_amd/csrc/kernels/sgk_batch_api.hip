@@ -203,6 +203,7 @@ int sgk_batch_destroy(sgk_batch *b) {
     for (auto &g : b->graphs)
         if (g.second.exec) (void)hipGraphExecDestroy(g.second.exec);
     for (void *q : b->allocs) (void)hipFree(q);
+    sgk::stage_free(b->stage);
     if (b->hostState) (void)hipHostFree(b->hostState);
     if (b->ev0) (void)hipEventDestroy(b->ev0);
     if (b->ev1) (void)hipEventDestroy(b->ev1);
@@ -408,65 +409,18 @@ int sgk_batch_create(int nrep, const SimParams *params, const sgk_config *cfgIn,
 int sgk_batch_upload_f64(sgk_batch *b, int rep, const double *r, const double *v, const double *a) {
     if (!b || rep < 0 || rep >= b->nrep) return SGK_E_ARG;
     const BatchRep &R = b->reps[rep];
-    const size_t n = (size_t)R.p.nMol;
-    if (r) {
-        if (b->mixed) {
-            BHIP(b, hipMemcpy((double4 *)b->pos + R.atomOff, r, 32 * n, hipMemcpyHostToDevice));
-        } else {
-            std::vector<float> t(4 * n);
-            for (size_t i = 0; i < 4 * n; ++i) t[i] = (float)r[i];
-            BHIP(b, hipMemcpy((float4 *)b->pos + R.atomOff, t.data(), 16 * n, hipMemcpyHostToDevice));
-        }
-    }
-    const double *src[2] = {v, a};
-    void *dst[2] = {b->vel, b->acc};
-    for (int k = 0; k < 2; ++k) {
-        if (!src[k]) continue;
-        if (b->mixed) {
-            std::vector<double> t(3 * n);
-            for (size_t i = 0; i < n; ++i)
-                for (int d = 0; d < 3; ++d) t[d * n + i] = src[k][3 * i + d];
-            BHIP(b, hipMemcpy((double *)dst[k] + 3 * R.atomOff, t.data(), 8 * 3 * n, hipMemcpyHostToDevice));
-        } else {
-            std::vector<float> t(3 * n);
-            for (size_t i = 0; i < n; ++i)
-                for (int d = 0; d < 3; ++d) t[d * n + i] = (float)src[k][3 * i + d];
-            BHIP(b, hipMemcpy((float *)dst[k] + 3 * R.atomOff, t.data(), 4 * 3 * n, hipMemcpyHostToDevice));
-        }
-    }
+    const size_t w = b->mixed ? 8 : 4;
+    char *pos = (char *)b->pos + 4 * w * R.atomOff, *vel = (char *)b->vel + 3 * w * R.atomOff, *acc = (char *)b->acc + 3 * w * R.atomOff;
+    BHIP(b, sgk::state_to_device(b->stage, b->device, b->stream, (size_t)R.p.nMol, b->mixed, r, v, a, pos, vel, acc));
     return SGK_OK;
 }
 
 int sgk_batch_download_f64(sgk_batch *b, int rep, double *r, double *v, double *a) {
     if (!b || rep < 0 || rep >= b->nrep) return SGK_E_ARG;
-    BHIP(b, hipStreamSynchronize(b->stream));
     const BatchRep &R = b->reps[rep];
-    const size_t n = (size_t)R.p.nMol;
-    if (r) {
-        if (b->mixed) {
-            BHIP(b, hipMemcpy(r, (double4 *)b->pos + R.atomOff, 32 * n, hipMemcpyDeviceToHost));
-        } else {
-            std::vector<float> t(4 * n);
-            BHIP(b, hipMemcpy(t.data(), (float4 *)b->pos + R.atomOff, 16 * n, hipMemcpyDeviceToHost));
-            for (size_t i = 0; i < 4 * n; ++i) r[i] = t[i];
-        }
-    }
-    double *dstv[2] = {v, a};
-    void *srcv[2] = {b->vel, b->acc};
-    for (int k = 0; k < 2; ++k) {
-        if (!dstv[k]) continue;
-        if (b->mixed) {
-            std::vector<double> t(3 * n);
-            BHIP(b, hipMemcpy(t.data(), (double *)srcv[k] + 3 * R.atomOff, 8 * 3 * n, hipMemcpyDeviceToHost));
-            for (size_t i = 0; i < n; ++i)
-                for (int d = 0; d < 3; ++d) dstv[k][3 * i + d] = t[d * n + i];
-        } else {
-            std::vector<float> t(3 * n);
-            BHIP(b, hipMemcpy(t.data(), (float *)srcv[k] + 3 * R.atomOff, 4 * 3 * n, hipMemcpyDeviceToHost));
-            for (size_t i = 0; i < n; ++i)
-                for (int d = 0; d < 3; ++d) dstv[k][3 * i + d] = t[d * n + i];
-        }
-    }
+    const size_t w = b->mixed ? 8 : 4;
+    const char *pos = (char *)b->pos + 4 * w * R.atomOff, *vel = (char *)b->vel + 3 * w * R.atomOff, *acc = (char *)b->acc + 3 * w * R.atomOff;
+    BHIP(b, sgk::state_to_host(b->stage, b->device, b->stream, (size_t)R.p.nMol, b->mixed, pos, vel, acc, r, v, a));
     return SGK_OK;
 }
 

@@ -12,6 +12,7 @@
 #include "sgk_adjoint.h"
 #include "sgk_batch.h"
 #include "sgk_params.h"
+#include "sgk_xfer.h"
 
 namespace sgk {
 
@@ -71,6 +72,7 @@ struct sgk_ctx {
     sgk_record *records = nullptr;
     unsigned int *hist = nullptr;
     sgk::DevState *hostState = nullptr;                 // pinned mirror
+    sgk::HostStage stage;                               // state transfer, grown on demand
     // launch geometry
     int block = 256, metalLanes = 8, nbM = 0, nbC = 0, nbRho = 0, nbProps = 0;
     int part2Off = 0;                                   // chunk totals of the step reduction (in partials)
@@ -159,6 +161,7 @@ struct sgk_batch {
     sgk_record *records = nullptr;
     unsigned int *hist = nullptr;
     sgk::DevState *hostState = nullptr;  // pinned mirror, nrep entries
+    sgk::HostStage stage;                // state transfer, grown on demand
     long long bytes = 0;
     int hostStep = 0;
     double lastRunMs = 0;

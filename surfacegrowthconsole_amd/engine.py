@@ -154,9 +154,7 @@ class Engine:
             self._check(self.lib.sgk_upload(self.h, *[_ptr(x) for x in args]), "sgk_upload")
 
     def download(self):
-        r = np.zeros((self.n, 4))
-        v = np.zeros((self.n, 3))
-        a = np.zeros((self.n, 3))
+        r, v, a = np.empty((self.n, 4)), np.empty((self.n, 3)), np.empty((self.n, 3))
         self._check(self.lib.sgk_download_f64(self.h, _ptr(r), _ptr(v), _ptr(a)), "sgk_download_f64")
         return r, v, a
 
@@ -209,8 +207,7 @@ class Engine:
         return out[: self.n_metal]
 
     def forces(self):
-        acc = np.zeros((self.n, 3))
-        e = np.zeros(self.n)
+        acc, e = np.empty((self.n, 3)), np.empty(self.n)
         fr = np.zeros(max(self.n_metal, 1))
         self._check(self.lib.sgk_get_forces(self.h, _ptr(acc), _ptr(e), _ptr(fr)), "sgk_get_forces")
         return acc, e, fr[: self.n_metal]
@@ -253,7 +250,7 @@ class Engine:
     def run(self, nsteps, rdf_every=0, records=True):
         recs = (N.SgkRecord * nsteps)() if records else None
         self._check(self.lib.sgk_run(self.h, nsteps, rdf_every, recs), "sgk_run")
-        return [record_dict(r) for r in recs] if records else None
+        return record_dicts(recs) if records else None
 
     def prepare_run(self, nsteps, rdf_every=0):
         """Capture the graph of the next run(nsteps, rdf_every) now, so that run does not pay for it."""
@@ -293,7 +290,7 @@ class Engine:
                     "sgk_adjoint_forward")
         out = dict(zip(N.SGK_OBSERVABLES, obs.tolist()))
         if records:
-            out["records"] = [record_dict(r) for r in recs]
+            out["records"] = record_dicts(recs)
         return out
 
     def adjoint_backward(self, weights, initial_state=False):
@@ -403,16 +400,17 @@ class Batch:
 
     def upload(self, rep, r, v=None, a=None):
         n = self.params[rep].nMol
-        r4 = np.zeros((n, 4))
-        r = np.asarray(r, np.float64)
-        r4[:, : r.shape[1]] = r
+        r = r4 = np.asarray(r, np.float64)
+        if r.shape != (n, 4):
+            r4 = np.zeros((n, 4))
+            r4[:, : r.shape[1]] = r
         args = [np.ascontiguousarray(x, np.float64) if x is not None else None for x in (r4, v, a)]
         self._check(self.lib.sgk_batch_upload_f64(self.h, rep, *[_ptr(x) if x is not None else None for x in args]),
                     "sgk_batch_upload_f64")
 
     def download(self, rep):
         n = self.params[rep].nMol
-        r, v, a = np.zeros((n, 4)), np.zeros((n, 3)), np.zeros((n, 3))
+        r, v, a = np.empty((n, 4)), np.empty((n, 3)), np.empty((n, 3))
         self._check(self.lib.sgk_batch_download_f64(self.h, rep, _ptr(r), _ptr(v), _ptr(a)), "sgk_batch_download_f64")
         return r, v, a
 
@@ -426,7 +424,8 @@ class Batch:
             return None
         buf = (N.SgkRecord * (nsteps * self.nrep))()
         self._check(self.lib.sgk_batch_run(self.h, nsteps, rdf_every, buf), "sgk_batch_run")
-        return [[record_dict(buf[r * nsteps + k]) for k in range(nsteps)] for r in range(self.nrep)]
+        recs = record_dicts(buf)
+        return [recs[r * nsteps : (r + 1) * nsteps] for r in range(self.nrep)]
 
     def last_run_ms(self):
         return self.lib.sgk_batch_last_run_ms(self.h)
@@ -437,9 +436,15 @@ class Batch:
         return h
 
 
+_RECORD = np.dtype(N.SgkRecord)
+
+
+def record_dicts(recs):
+    """The records of a ctypes array as dicts of Python numbers and lists, column by column."""
+    a = np.frombuffer(recs, _RECORD)
+    cols = [a[name].tolist() for name in _RECORD.names]
+    return [dict(zip(_RECORD.names, row)) for row in zip(*cols)]
+
+
 def record_dict(r):
-    d = {}
-    for name, _ in N.SgkRecord._fields_:
-        val = getattr(r, name)
-        d[name] = list(val) if hasattr(val, "__len__") else val
-    return d
+    return record_dicts(r)[0]
