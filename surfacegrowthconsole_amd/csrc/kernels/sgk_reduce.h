@@ -199,14 +199,87 @@ __device__ __forceinline__ StepNext<A> step_next(const DevParams &p, const DevSt
     return n;
 }
 
-// Total of nParts partials, in thread 0: each thread a strided subset, then the block tree (the order
-// is fixed, so the result is bitwise reproducible).
+// Total of n partials by one workgroup of 256 threads, returned to every thread.  A thread takes one
+// field of 16 partials: their loads are all in flight at once and a field's tree is 15 operations in
+// registers, where a lane per partial moved 20 fields through 6 exchange steps each, twice, and a
+// launch of one workgroup has nothing to hide them behind.  The trees are reduce_chunk's (rows of 16,
+// then the rows of a chunk) and so are the sums, bit for bit.
+// totals: the n are chunk totals (any number): thread t of 256 first adds totals t, t + 256, ... in order.
+// Otherwise at most kSumParts partials: chunks of 64, then the chunk totals as the first 16 lanes of a wave.
+// One launch for up to 1,024 partials in place of k_reduce1 and k_finalize: a sheared step of 997 atoms
+// (FP32) 29.1 -> 26.8 us, a deposition step of 4,393 27.2 -> 25.3, kb_finalize of 64 replicas 8.0 -> 6.5.
+constexpr int kSumRows = 64, kSumParts = 16 * kSumRows, kSumGroups = 256 / kPartFields;
+
+// One field of a tree: all lanes run the same instructions, the field picks its result.
+enum class FieldOp : int { sum, max, min };
+__device__ __forceinline__ FieldOp field_op(int f) {
+    return f == kPartVmax || (f >= kPartBmax && f < kPartVir) ? FieldOp::max
+           : f >= kPartBmin && f < kPartBmax                  ? FieldOp::min
+                                                              : FieldOp::sum;
+}
 template <class A>
-__device__ __forceinline__ Partial<A> reduce_parts(const Partial<A> *part, int nParts) {
-    Partial<A> q;
-    partial_identity(q);
-    for (int k = threadIdx.x; k < nParts; k += blockDim.x) partial_combine(q, part[k]);
-    return block_reduce_partial(q);
+__device__ __forceinline__ A field_id(int f) {
+    return f >= kPartBmin && f < kPartBmax ? A(3.0e38f) : (f >= kPartBmax && f < kPartVir ? A(-3.0e38f) : A(0));
+}
+template <class A>
+__device__ __forceinline__ A field_join(FieldOp op, A x, A y) {
+    const A s = x + y, hi = y > x ? y : x, lo = y < x ? y : x;
+    return op == FieldOp::sum ? s : (op == FieldOp::max ? hi : lo);
+}
+template <class A>
+__device__ __forceinline__ A field_tree16(FieldOp op, A (&x)[16]) {
+#pragma unroll
+    for (int d = 1; d < 16; d *= 2)
+#pragma unroll
+        for (int j = 0; j < 16; j += 2 * d) x[j] = field_join(op, x[j], x[j + d]);
+    return x[0];
+}
+
+template <class A>
+__device__ __forceinline__ Partial<A> sum_parts(const Partial<A> *part, int n, bool totals) {
+    static_assert(sizeof(Partial<A>) == kPartFields * sizeof(A), "fields of Partial in their order");
+    __shared__ A rows[kSumRows][kPartFields], chunks[16][kPartFields];
+    __shared__ Partial<A> total;
+    const int f = threadIdx.x % kPartFields, g = threadIdx.x / kPartFields;
+    const bool mine = g < kSumGroups;
+    const FieldOp op = field_op(f);
+    const A id = field_id<A>(f);
+    const int lanes = totals ? min(n, 256) : n, nRows = (lanes + 15) / 16, nChunks = (nRows + 3) / 4;
+    const A *src = (const A *)part + f;
+    if (mine)
+        for (int r = g; r < nRows; r += kSumGroups) {
+            A x[16];
+#pragma unroll
+            for (int j = 0; j < 16; ++j) x[j] = 16 * r + j < lanes ? src[(16 * r + j) * kPartFields] : id;
+            if (totals)
+                for (int k = 256 + 16 * r; k < n; k += 256)
+#pragma unroll
+                    for (int j = 0; j < 16; ++j)
+                        if (k + j < n) x[j] = field_join(op, x[j], src[(size_t)(k + j) * kPartFields]);
+            rows[r][f] = field_tree16(op, x);
+        }
+    __syncthreads();
+    if (mine)
+        for (int c = g; c < nChunks; c += kSumGroups) {
+            auto row = [&](int r) { return r < nRows ? rows[r][f] : id; };
+            chunks[c][f] = field_join(op, field_join(op, row(4 * c + 3), row(4 * c + 2)),
+                                      field_join(op, row(4 * c + 1), row(4 * c)));
+        }
+    __syncthreads();
+    if (g == 0) {
+        A r = n > 0 ? chunks[0][f] : id;
+        if (totals) {
+            for (int c = 1; c < nChunks; ++c) r = field_join(op, r, chunks[c][f]);
+        } else if (nChunks > 1) {
+            A x[16];
+#pragma unroll
+            for (int c = 0; c < 16; ++c) x[c] = c < nChunks ? chunks[c][f] : id;
+            r = field_tree16(op, x);
+        }
+        ((A *)&total)[f] = r;
+    }
+    __syncthreads();
+    return total;
 }
 
 // The sums of a record, with the reference's host arithmetic (SurfaceGrowth.cu:2307-2395); returns the
@@ -249,57 +322,62 @@ __device__ __forceinline__ void record_sums(const DevParams &p, const Partial<A>
     rec.pad = 0;
 }
 
-// Reduce nParts partials with the whole block, then evaluate the reference's host arithmetic of
-// SurfaceGrowth.cu:2307-2395 in thread 0.
+// Reduce nParts partials (totals: chunk totals) with the whole workgroup of 256, then evaluate the
+// reference's host arithmetic of SurfaceGrowth.cu:2307-2395 in thread 0.
 // mode 0: one step - advance the step counter, commit a rebuild, update dispHi / nebrNow / shear,
 //         append a record.  mode 1: evaluation only - write records[0], leave the state alone.
 template <class A>
-__device__ void finalize_body(const DevParams &p, const Partial<A> *part, int nParts, DevState *st,
+__device__ void finalize_body(const DevParams &p, const Partial<A> *part, int nParts, bool totals, DevState *st,
                               sgk_record *records, int recCap, int mode) {
-    const Partial<A> P = reduce_parts(part, nParts);
+    const DevState s0 = *st;  // before the sums: its latency passes meanwhile
+    const Partial<A> P = sum_parts(part, nParts, totals);
     if (threadIdx.x != 0) return;
     const int nMe = p.nMolMe;
     sgk_record rec;
     A cmVelX, vvSum;
     record_sums(p, P, rec, cmVelX, vvSum);
     if (mode == 1) {
-        rec.step = st->step;
+        rec.step = s0.step;
         rec.rebuilt = 0;
-        rec.nebrNow = st->nebrNow;
-        rec.errors = st->errors | st->errPrev;
-        rec.dispHi = st->dispHi;
-        rec.nMolDeposited = st->nMolDeposited;
+        rec.nebrNow = s0.nebrNow;
+        rec.errors = s0.errors | s0.errPrev;
+        rec.dispHi = s0.dispHi;
+        rec.nMolDeposited = s0.nMolDeposited;
         records[0] = rec;
         return;
     }
-    const StepNext<A> n = step_next(p, st, P.vmax);
-    const int step = n.step;
-    rec.step = step;
-    rec.rebuilt = st->nebrNow;
+    const StepNext<A> n = step_next(p, &s0, P.vmax);
+    const int step = n.step, errors = s0.errors | (n.displaced ? SGK_FLAG_DISPLACEMENT : 0);
+    double shear = s0.shear;
+    int deposited = s0.nMolDeposited;
+    // shear increment (SurfaceGrowth.cu:2398-2404)
+    if (p.iRegime == 2 && nMe && step > p.stepEquil + p.stepCool) {
+        if ((float)cmVelX < 0.005f) shear = (double)((A)shear + (A)p.deltaF);
+    }
+    // deposition schedule (SurfaceGrowth.cu:2148-2168): the step's group counts from now on
+    if (p.iRegime == 1 && step > p.stepEquil && deposited < nMe && p.stepDeposit > 0 &&
+        (step - p.stepEquil) % p.stepDeposit == 0)
+        deposited += p.nMolToDeposit;
     st->step = step;
     st->cellbuf = n.cellbuf;
     st->rebuilds = n.rebuilds;
-    if (n.displaced) st->errors |= SGK_FLAG_DISPLACEMENT;
+    st->errors = errors;
     st->nebrNow = n.nebrNow;
     st->dispHi = n.dispHi;
     st->vvSum = (double)vvSum;
     st->cmVelX = (double)cmVelX;
     st->comX = nMe ? (double)(P.com[0] / (A)nMe) : 0.0;
-    // shear increment (SurfaceGrowth.cu:2398-2404)
-    if (p.iRegime == 2 && nMe && step > p.stepEquil + p.stepCool) {
-        if ((float)cmVelX < 0.005f) st->shear = (double)((A)st->shear + (A)p.deltaF);
-    }
-    // deposition schedule (SurfaceGrowth.cu:2148-2168): the step's group counts from now on
-    if (p.iRegime == 1 && step > p.stepEquil && st->nMolDeposited < nMe && p.stepDeposit > 0 &&
-        (step - p.stepEquil) % p.stepDeposit == 0)
-        st->nMolDeposited += p.nMolToDeposit;
-    rec.nMolDeposited = st->nMolDeposited;
-    rec.shear = st->shear;
+    st->shear = shear;
+    st->nMolDeposited = deposited;
+    st->rec = s0.rec + 1;
+    rec.step = step;
+    rec.rebuilt = s0.nebrNow;
+    rec.nMolDeposited = deposited;
+    rec.shear = shear;
     rec.nebrNow = n.nebrNow;
     rec.dispHi = n.dispHi;
-    rec.errors = st->errors | st->errPrev;
-    if (st->rec < recCap) records[st->rec] = rec;
-    st->rec += 1;
+    rec.errors = errors | s0.errPrev;
+    if (s0.rec < recCap) records[s0.rec] = rec;
 }
 
 // ---- step closing folded into the next step --------------------------------------------------------
@@ -311,10 +389,10 @@ __device__ void finalize_body(const DevParams &p, const Partial<A> *part, int nP
 // is longer than the reduction's ~11 us at 1,000 partials).  The two closing launches cost a small
 // step ~6 us of latency.  Whole step, closed by launches / folded (us): 1,161 atoms 34.6 / 29.0,
 // 44,353 41.4 / 35.2, 137,940 (FP32) 50.3 / 45.3, 1.1 M 224.2 / 223.5.
-constexpr int kCloseLdsChunks = 16;                           // chunk totals kept in LDS
+//
 // Partials closed without k_reduce1: beyond, every workgroup of k_bin_next would read more than 8 KB
-// of maxima and the closing workgroup's chunks would outlast the force launch.
-constexpr int kCloseDirectParts = kCloseLdsChunks * kPartChunk;
+// of maxima and the closing workgroup's rows would outlast the force launch.
+constexpr int kCloseDirectParts = kSumParts;
 
 template <class A>
 struct StepClose {
@@ -329,17 +407,7 @@ struct StepClose {
 // The sums are those of k_reduce1 and k_finalize, bit for bit.
 template <class A>
 __device__ __forceinline__ void close_body(const DevParams &p, const StepClose<A> &c) {
-    __shared__ Partial<A> tot[kCloseLdsChunks];
-    const Partial<A> *src = c.part;
-    int n = c.n;
-    if (c.direct) {  // as k_reduce1, one wave per chunk
-        n = (c.n + kPartChunk - 1) / kPartChunk;
-        for (int j = threadIdx.x >> 6; j < n; j += (int)blockDim.x >> 6)
-            reduce_chunk(c.part + j * kPartChunk, min(kPartChunk, c.n - j * kPartChunk), tot + j);
-        __syncthreads();
-        src = tot;
-    }
-    const Partial<A> P = reduce_parts(src, n);
+    const Partial<A> P = sum_parts(c.part, c.n, !c.direct);
     if (threadIdx.x != 0) return;
     sgk_record rec;
     A cmVelX, vvSum;

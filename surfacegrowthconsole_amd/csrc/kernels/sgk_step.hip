@@ -184,10 +184,10 @@ __global__ __launch_bounds__(256) void k_props(DevParams p, const typename Prec<
     if (threadIdx.x == 0) part[blockIdx.x] = r;
 }
 
-// The step reduction in two stages: k_reduce1 (one wave per chunk of kPartChunk force-pass
-// partials, many waves) and k_finalize (one workgroup over the chunk totals, then the step's
-// bookkeeping; mode 1 reduces k_props partials directly).  A single workgroup over all partials
-// took 26 us at 1.1 M atoms.
+// The step reduction: k_finalize (one workgroup: the sums, then the step's bookkeeping) takes up to
+// kSumParts force-pass partials directly.  More are first reduced to chunk totals by k_reduce1 (one
+// wave per chunk of kPartChunk): a single workgroup over all partials took 26 us at 1.1 M atoms.
+// mode 1 reduces k_props partials, which count as totals.
 constexpr int kFinalizeThreads = 256;
 template <bool M>
 __global__ __launch_bounds__(256) void k_reduce1(const Partial<typename Prec<M>::A> *__restrict__ part, int nParts,
@@ -200,27 +200,28 @@ __global__ __launch_bounds__(256) void k_reduce1(const Partial<typename Prec<M>:
 template <bool M>
 __global__ __launch_bounds__(kFinalizeThreads) void k_finalize(DevParams p,
                                                                const Partial<typename Prec<M>::A> *__restrict__ part,
-                                                               int nParts, DevState *st, sgk_record *records,
-                                                               int recCap, int mode) {
-    finalize_body<typename Prec<M>::A>(p, part, nParts, st, records, recCap, mode);
+                                                               int nParts, int totals, DevState *st,
+                                                               sgk_record *records, int recCap, int mode) {
+    finalize_body<typename Prec<M>::A>(p, part, nParts, totals, st, records, recCap, mode);
 }
 
-// Batched: both stages in one workgroup per replica - the waves reduce the chunks (the calls of
-// k_reduce1, in the same order), then the workgroup finalizes - so a replica's reduction order is
-// that of the replica run alone.  Up to kFinalizeLdsChunks chunk totals stay in LDS.
-constexpr int kFinalizeLdsChunks = 16;
+// Batched: one workgroup per replica, which also reduces the chunks where the partials are too many to
+// take directly - so a replica's reduction order is that of the replica run alone.
 template <bool M>
 __global__ __launch_bounds__(kFinalizeThreads) void kb_finalize(BatchArgs a) {
     using A = typename Prec<M>::A;
-    __shared__ Partial<A> tot[kFinalizeLdsChunks];
     const BatchRep &B = a.reps[blockIdx.x];
     const Partial<A> *part = (const Partial<A> *)a.partials + B.partOff;
-    Partial<A> *part2 = B.nChunks <= kFinalizeLdsChunks ? tot : (Partial<A> *)a.partials + B.part2Off;
-    for (int j = threadIdx.x >> 6; j < B.nChunks; j += kFinalizeThreads / 64)
-        reduce_chunk(part + j * kPartChunk, min(kPartChunk, B.nbForce - j * kPartChunk), part2 + j);
-    __syncthreads();
-    finalize_body<A>(B.p, part2, B.nChunks, a.state + blockIdx.x, a.records + (size_t)blockIdx.x * a.recCap,
-                     a.recCap, 0);
+    const bool totals = B.nbForce > kSumParts;
+    if (totals) {
+        Partial<A> *part2 = (Partial<A> *)a.partials + B.part2Off;
+        for (int j = threadIdx.x >> 6; j < B.nChunks; j += kFinalizeThreads / 64)
+            reduce_chunk(part + j * kPartChunk, min(kPartChunk, B.nbForce - j * kPartChunk), part2 + j);
+        __syncthreads();
+        part = part2;
+    }
+    finalize_body<A>(B.p, part, totals ? B.nChunks : B.nbForce, totals, a.state + blockIdx.x,
+                     a.records + (size_t)blockIdx.x * a.recCap, a.recCap, 0);
 }
 
 // ApplyBerendsenThermostat (SurfaceGrowth.cu:455-485), kinetic energy of all atoms.
@@ -456,16 +457,16 @@ template <bool M>
 static void finalize_dispatch(sgk_ctx *c, int mode) {
     using A = typename Prec<M>::A;
     Partial<A> *part = (Partial<A> *)c->partials;
-    if (mode == 1) {
-        hipLaunchKernelGGL(k_finalize<M>, dim3(1), dim3(kFinalizeThreads), 0, c->stream, c->dp, part, c->nbProps,
-                           c->state, c->records, 1, 1);
-        return;
+    int n = mode == 1 ? c->nbProps : c->nbM + c->nbC;
+    const bool totals = mode == 1 || n > kSumParts;
+    if (mode != 1 && totals) {
+        const int nChunks = (n + kPartChunk - 1) / kPartChunk;
+        hipLaunchKernelGGL(k_reduce1<M>, dim3((nChunks + 3) / 4), dim3(256), 0, c->stream, part, n, part + c->part2Off);
+        part += c->part2Off;
+        n = nChunks;
     }
-    const int nParts = c->nbM + c->nbC, nChunks = (nParts + kPartChunk - 1) / kPartChunk;
-    Partial<A> *part2 = part + c->part2Off;
-    hipLaunchKernelGGL(k_reduce1<M>, dim3((nChunks + 3) / 4), dim3(256), 0, c->stream, part, nParts, part2);
-    hipLaunchKernelGGL(k_finalize<M>, dim3(1), dim3(kFinalizeThreads), 0, c->stream, c->dp, part2, nChunks, c->state,
-                       c->records, c->cfg.records_capacity, 0);
+    hipLaunchKernelGGL(k_finalize<M>, dim3(1), dim3(kFinalizeThreads), 0, c->stream, c->dp, part, n, (int)totals, c->state,
+                       c->records, mode == 1 ? 1 : c->cfg.records_capacity, mode);
 }
 
 // The first reduction stage alone, for a step whose closing is folded into the next one: chunk totals
