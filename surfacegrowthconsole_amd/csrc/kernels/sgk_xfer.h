@@ -8,8 +8,9 @@
 // fresh array are shared then too).  No device memory is needed.  Download of everything as doubles:
 // 68 -> 20 us at 1,161 atoms, 328 -> 135 at 44,353, 15.4 -> 2.8 ms at 1.1 M; upload 65 -> 19 us,
 // 216 -> 139, 5.3 -> 2.8 ms.  A device stage with copy-engine transfers took 39, 188 and 3,093 us and its
-// allocation made a context's first download 1 ms longer.  Slots of 256 KiB, 512 KiB and 1 MiB
-// measure alike (138, 135, 135 us; 2.79-2.82 ms).
+// allocation made a context's first download 1 ms longer.  Slots of
+// 256 KiB, 512 KiB and 1 MiB: 177, 136 and 145 us at 44,353 atoms, 3.8, 2.9 and 2.4 ms at 1.1 M; a
+// context's first transfers (pages pinned and touched) 0.3, 0.5 and 1.7 ms.
 #pragma once
 
 #include <hip/hip_runtime.h>
