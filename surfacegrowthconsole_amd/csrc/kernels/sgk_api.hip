@@ -255,7 +255,8 @@ int sgk::prepare_ctx(const SimParams *sp, const sgk_config *cfgIn, sgk_ctx *c, s
     c->metalLanes = G;
     c->block = 256;
     c->nbM = metal_blocks(p.nMolMe, G, p.xcdMap);
-    c->nbC = (p.nC + 255) / 256;
+    c->carbonLanes = sgk::carbon_lanes(p.nC);
+    c->nbC = sgk::carbon_blocks(p.nC, c->carbonLanes);
     c->nbRho = c->nbM;
     c->nbProps = (p.nMol + 255) / 256;
     // partials for the largest force grid any launch shape gives (16 lanes per metal atom), then one

@@ -21,6 +21,7 @@ struct BatchRep {
     int partOff;         // first force-pass partial
     int nbForce;         // force-pass workgroups: nbM metal then carbon
     int nbM;             // metal workgroups of the density and force passes
+    int carbonLanes;     // lanes per carbon there, 1 or 4
     int part2Off;        // first chunk total of the two-stage step reduction
     int nChunks;         // chunks of kPartChunk force-pass partials
     int nbNlM;           // workgroups of the metal part of the cell-ordered list build (4 lanes per atom)

@@ -142,9 +142,9 @@ std::vector<int2> force_layout(sgk_batch *b) {
         BatchRep &R = b->reps[r];
         const int G = b->repLanes[r];
         R.nbM = metal_blocks(R.p.nMolMe, G, 0);  // the batch remaps nothing
-        R.nbForce = R.nbM + (R.p.nC + 255) / 256;
+        R.nbForce = R.nbM + sgk::carbon_blocks(R.p.nC, R.carbonLanes);
         R.partOff = partOff;
-        R.nChunks = (R.nbForce + 63) / 64;  // sgk::kPartChunk partials per chunk
+        R.nChunks = (sgk::PartMap{R.nbM, R.nbForce, R.carbonLanes == 4}.count() + 63) / 64;  // kPartChunk partials per chunk
         partOff += R.nbForce;
         auto &g = groups[sgk::batch_lane_index(G)];
         for (int k = 0; k < R.nbForce; ++k) g.push_back(make_int2(r, k));
@@ -172,7 +172,8 @@ std::vector<int2> force_layout(sgk_batch *b) {
 void worst_layout(const sgk_batch *b, size_t &tab, size_t &parts) {
     tab = parts = 0;
     for (const BatchRep &R : b->reps) {
-        const size_t nb = (size_t)((((long long)R.p.nMolMe * 16 + 255) / 256 + 7) / 8 * 8) + (R.p.nC + 255) / 256;
+        const size_t nb = (size_t)((((long long)R.p.nMolMe * 16 + 255) / 256 + 7) / 8 * 8) +
+                          (size_t)sgk::carbon_blocks(R.p.nC, R.carbonLanes);
         tab += nb;
         parts += nb + (nb + 63) / 64;
     }
@@ -232,7 +233,7 @@ int sgk_batch_create(int nrep, const SimParams *params, const sgk_config *cfgIn,
     if (cfg.cell_capacity > 64 || cfg.cell_capacity % 8)
         return bfail(nullptr, SGK_E_UNSUPPORTED, "cell capacity must be a multiple of 8 up to 64");
     if (cfg.close_capacity % 8) return bfail(nullptr, SGK_E_UNSUPPORTED, "close capacity must be a multiple of 8");
-    long long sumAtoms = 0;
+    long long sumAtoms = 0, sumCarbons = 0;
     for (int r = 0; r < nrep; ++r) {
         const SimParams &s = params[r];
         if (s.nMol <= 0 || s.nMolMe < 0 || s.nMolMe > s.nMol || s.nMol >= (1 << 24))
@@ -245,6 +246,7 @@ int sgk_batch_create(int nrep, const SimParams *params, const sgk_config *cfgIn,
         if (const char *m = mismatch(s0, s))
             return bfail(nullptr, SGK_E_ARG, "replica " + std::to_string(r) + " differs from replica 0 in " + m);
         sumAtoms += s.nMol;
+        sumCarbons += s.nMol - s.nMolMe;
     }
     int ndev = 0;
     if (hipGetDeviceCount(&ndev) != hipSuccess || ndev == 0) return bfail(nullptr, SGK_E_HIP, "no HIP device");
@@ -283,6 +285,7 @@ int sgk_batch_create(int nrep, const SimParams *params, const sgk_config *cfgIn,
         sgk::make_dev_params(s, cfg, R.p);
         R.p.xcdMap = 0;
         R.p.keepFull = 0;  // the reference-layout list is a single-system test aid
+        R.carbonLanes = sgk::carbon_lanes(sumCarbons);  // the launch's carbons
         R.atomOff = atomOff;
         R.metalOff = metalOff;
         R.carbonOff = carbonOff;

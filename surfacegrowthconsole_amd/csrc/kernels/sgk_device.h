@@ -230,6 +230,7 @@ __device__ __forceinline__ double dpp_all(double v) {
 enum : int {
     kQuadSwap1 = 0xB1,  // quad_perm [1,0,3,2]
     kQuadSwap2 = 0x4E,  // quad_perm [2,3,0,1]
+    kQuadNext3 = 0xC9,  // quad_perm [1,2,0,3]
     kRowShr2 = 0x112,
     kRowShr4 = 0x114,
     kRowShr8 = 0x118,
@@ -258,6 +259,11 @@ struct OpMin {
     template <class T>
     __device__ static __forceinline__ T f(T a, T b) { return b < a ? b : a; }
 };
+
+template <int CTRL>
+__device__ __forceinline__ unsigned quad_word(unsigned v) {
+    return (unsigned)__builtin_amdgcn_mov_dpp((int)v, CTRL, 0xF, 0xF, false);
+}
 
 // Reduction over the wave; the result is valid in lane 63 (fixed order, so reproducible).
 template <class Op, class T>

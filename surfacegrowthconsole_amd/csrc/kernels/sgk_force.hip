@@ -5,13 +5,14 @@
 // (SurfaceGrowth.cu:716-773).  Here:
 //   k_rho    blocks [0, nbRho): G lanes per metal atom split its neighbour list; rho, F(rho),
 //            F'(rho) stored, so the force pass reads F'(rho_k) instead of recomputing it per pair.
-//            blocks [nbRho, nbRho + nbC): one thread per carbon scans its close list once and stores
+//            blocks [nbRho, nbRho + nbC): one thread per carbon (four in small systems, carbon_lanes)
+//            scans its close list once and stores
 //            the first three carbons within rCutC (its bonds) and the first three atoms of any kind
 //            within rCutC (what a bonded neighbour's angle terms need), so the force pass reads
 //            four near lists instead of scanning four close lists.
 //   k_force  one launch: blocks [0, nbM) are the metal pass (G lanes per atom: EAM pairs + LJ with
-//            carbon), blocks [nbM, nbM + nbC) the carbon pass (one thread per atom: bond, plane and
-//            angle terms from the close list + LJ with metal).  The epilogue writes acceleration,
+//            carbon), blocks [nbM, nbM + nbC) the carbon pass (one thread per atom, or four: bond, plane
+//            and angle terms from the close list + LJ with metal).  The epilogue writes acceleration,
 //            energy, friction, applies leapfrog part 2 and leaves one Partial per block; k_finalize
 //            (sgk_step.hip), the next launch, reduces them and runs the step bookkeeping.  (A
 //            last-block reduction inside k_force needs a device-scope release fence per block, which
@@ -160,9 +161,81 @@ __device__ __forceinline__ void bonds_body(const DevParams &p, int blk, const ty
     bondA[ic] = make_uint4(ab[0], ab[1], ab[2], (unsigned)na);
 }
 
+// The same near lists by four lanes per carbon, for launches that leave the chip idle: lane l takes
+// entries l, l + 4, l + 8 and l + 12 of a round of 16, so a close list of a dozen is one round of
+// loads where bonds_body makes three.  A hit's place is its rank among the round's hits (a mask over
+// the quad); the lane that holds one of the first three stores it.  Density launch 6.0 -> 4.5 us at 1,161
+// atoms, 8.5 -> 7.0 at 44,353.
+template <bool M>
+__device__ __forceinline__ void bonds4_body(const DevParams &p, int blk, const typename Prec<M>::P4 *__restrict__ pos,
+                                            const unsigned *__restrict__ cl, const int *__restrict__ ncl,
+                                            uint4 *__restrict__ bondC, uint4 *__restrict__ bondA) {
+    using R = typename Prec<M>::R;
+    using P4 = typename Prec<M>::P4;
+    const int gt = blk * blockDim.x + threadIdx.x, ic = gt / 4, l = gt & 3;
+    if (ic >= p.nC) return;  // whole quads
+    const int i = p.nMolMe + ic;
+    const P4 Ai = pos[i];
+    unsigned *const outC = (unsigned *)(bondC + ic), *const outA = (unsigned *)(bondA + ic);
+    int nc = 0, na = 0;  // the quad's counts so far, at most 3 of each matter
+    const int nclose = ncl[ic];
+    const unsigned *row = cl + (size_t)ic * p.clCap;
+    for (int base = 0; base < nclose && (nc < 3 || na < 3); base += 16) {
+        unsigned ent[4];
+        P4 B[4];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            const int j = base + 4 * t + l;
+            ent[t] = j < nclose ? row[j] : (unsigned)i << 8;
+        }
+#pragma unroll
+        for (int t = 0; t < 4; ++t) B[t] = pos[ent[t] >> 8];
+        unsigned hitA = 0u, hitC = 0u;  // bit 4t + l
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            R dx, dy, dz;
+            const R rr = disp<R>(Ai, B[t], p, dx, dy, dz);
+            if (base + 4 * t + l >= nclose || !(rr < (R)p.rrCutC)) continue;
+            hitA |= 1u << (4 * t + l);
+            if ((int)(ent[t] >> 8) >= p.nMolMe) hitC |= 1u << (4 * t + l);
+        }
+        unsigned all = hitA | hitC << 16;
+        all |= quad_word<kQuadSwap1>(all);
+        all |= quad_word<kQuadSwap2>(all);
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            const unsigned bit = 1u << (4 * t + l);
+            const int ra = na + __popc(all & 0xFFFFu & (bit - 1u)), rc = nc + __popc((all >> 16) & (bit - 1u));
+            if ((hitA & bit) && ra < 3) outA[ra] = ent[t];
+            if ((hitC & bit) && rc < 3) outC[rc] = ent[t];
+        }
+        na += __popc(all & 0xFFFFu);
+        nc += __popc(all >> 16);
+    }
+    na = min(na, 3);
+    nc = min(nc, 3);
+    // lane 3 stores the counts, lanes 0..2 the places no hit took
+    if (l == 3 || l >= na) outA[l] = l == 3 ? (unsigned)na : 0u;
+    if (l == 3 || l >= nc) outC[l] = l == 3 ? (unsigned)nc : 0u;
+}
+
+// Carbon workgroup b of a launch with four lanes per carbon: its 64 carbons and the place of its partial.
+// Four of them are the workgroup w that a lane per carbon gives, parts r = 0..3.  With XCD ranges (xm) the
+// four run on the XCD of w: b % 8 is w % 8, and the launch is padded to whole 32s (quad_grid).
+struct QuadBlock {
+    int blk, slot;  // slot < 0: padding
+};
+__device__ __forceinline__ QuadBlock quad_block(int b, int nC, bool xm) {
+    if (!xm) return {b, b};
+    const int n = (nC + 255) / 256, r = b / kXcds % 4, w = b / (4 * kXcds) * kXcds + b % kXcds;
+    if (w >= n) return {-1, -1};
+    return {4 * xcd_block(w, n) + r, 4 * w + r};
+}
+static inline int quad_grid(int nbC, bool xm) { return xm ? (nbC / 4 + kXcds - 1) / kXcds * kXcds * 4 : nbC; }
+
 // One workgroup of the density launch: blocks [0, nbRho) metal density, the rest carbon near lists.
 template <bool M, class T, int G>
-__device__ __forceinline__ void rho_block(const DevParams &p, int b, int nbRho, int nb, bool xm,
+__device__ __forceinline__ void rho_block(bool quad, const DevParams &p, int b, int nbRho, int nb, bool xm,
                                           const typename Prec<M>::P4 *__restrict__ pos, const int *__restrict__ nlM,
                                           const int *__restrict__ nnM, float *__restrict__ rho,
                                           float *__restrict__ embF, float *__restrict__ embDF,
@@ -170,11 +243,14 @@ __device__ __forceinline__ void rho_block(const DevParams &p, int b, int nbRho, 
                                           uint4 *__restrict__ bondC, uint4 *__restrict__ bondA) {
     if (b < nbRho)
         rho_body<M, T, G>(p, xm ? xcd_block(b, nbRho) : b, pos, nlM, nnM, rho, embF, embDF);
-    else
+    else if (quad) {
+        const QuadBlock q = quad_block(b - nbRho, p.nC, xm);
+        if (q.slot >= 0) bonds4_body<M>(p, q.blk, pos, cl, ncl, bondC, bondA);
+    } else
         bonds_body<M>(p, xm ? xcd_block(b - nbRho, nb - nbRho) : b - nbRho, pos, cl, ncl, bondC, bondA);
 }
 
-template <bool M, class T, int G>
+template <bool M, class T, int G, int CL>
 __global__ __launch_bounds__(256) void k_rho(DevParams p, int nbRho, const typename Prec<M>::P4 *__restrict__ pos,
                                              const int *__restrict__ nlM, const int *__restrict__ nnM,
                                              float *__restrict__ rho, float *__restrict__ embF,
@@ -182,7 +258,7 @@ __global__ __launch_bounds__(256) void k_rho(DevParams p, int nbRho, const typen
                                              const int *__restrict__ ncl, uint4 *__restrict__ bondC,
                                              uint4 *__restrict__ bondA) {
     // nbRho is a multiple of 8: both ranges keep the XCD of each block
-    rho_block<M, T, G>(p, blockIdx.x, nbRho, gridDim.x, p.xcdMap & 2, pos, nlM, nnM, rho, embF, embDF, cl, ncl,
+    rho_block<M, T, G>(CL == 4, p, blockIdx.x, nbRho, gridDim.x, p.xcdMap & 2, pos, nlM, nnM, rho, embF, embDF, cl, ncl,
                        bondC, bondA);
 }
 
@@ -191,7 +267,7 @@ __global__ __launch_bounds__(256) void kb_rho(BatchArgs a) {
     const int2 e = a.forceTab[blockIdx.x];
     const BatchRep &B = a.reps[e.x];
     const DevParams &p = B.p;
-    rho_block<M, T, G>(p, e.y, B.nbM, B.nbForce, false, (const typename Prec<M>::P4 *)a.pos + B.atomOff,
+    rho_block<M, T, G>(B.carbonLanes == 4, p, e.y, B.nbM, B.nbForce, false, (const typename Prec<M>::P4 *)a.pos + B.atomOff,
                        a.nlM + B.metalOff * p.nlCap, a.nnM + B.metalOff, a.rho + B.metalOff, a.embF + B.metalOff,
                        a.embDF + B.metalOff, a.cl + B.carbonOff * p.clCap, a.ncl + B.carbonOff,
                        a.bondC + B.carbonOff, a.bondA + B.carbonOff);
@@ -380,26 +456,93 @@ __device__ __forceinline__ double sqrtR(double x) { return sqrt64(x); }
 __device__ __forceinline__ void gacc(float &a, float t) { a += t; }
 __device__ __forceinline__ void gacc(double &a, float t) { a += (double)t; }
 
-// Neighbour-angle terms of bond (i,k) with k's bonded neighbour m (SurfaceGrowth.cu:953-978).
+// The factors of a neighbour angle's terms (SurfaceGrowth.cu:953-978), fe along e and fr along rik.
 // rik: r_i - r_k, aik = |rik|; e: r_m - r_k, rr2 = |e|^2 (the reference divides by rr2 where |e|
 // is meant; kept).
 template <class R>
-__device__ __forceinline__ void neighbour_angle(const DevParams &p, const V3<R> &rik, R aik, const V3<R> &e, R rr2,
-                                                float mz_rel, R &fx, R &fy, R &fz) {
+__device__ __forceinline__ void angle_factors(const DevParams &p, const V3<R> &rik, R aik, const V3<R> &e, R rr2,
+                                              float &fe, float &fr) {
     const R c = (rik.x * e.x + rik.y * e.y + rik.z * e.z) * rcpR(aik * rr2);
     float s;
     const float dth = AngleDev<R>::eval(c, p, s);
     const float tmp = p.mu_theta * dth * rcpf(s);
     const float fa = (float)aik, frr = (float)rr2;
-    float fc = tmp * rcpf(fa * frr);
+    fe = tmp * rcpf(fa * frr);
+    fr = -tmp * (float)c * rcpf(fa * fa);
+}
+
+// Neighbour-angle terms of bond (i,k) with k's bonded neighbour m.
+template <class R>
+__device__ __forceinline__ void neighbour_angle(const DevParams &p, const V3<R> &rik, R aik, const V3<R> &e, R rr2,
+                                                float mz_rel, R &fx, R &fy, R &fz) {
+    float fc, fr;
+    angle_factors<R>(p, rik, aik, e, rr2, fc, fr);
     gacc(fx, fc * (float)e.x);
     gacc(fy, fc * (float)e.y);
     gacc(fz, fc * (float)e.z);
-    fc = -tmp * (float)c * rcpf(fa * fa);
+    fc = fr;
     gacc(fx, fc * (float)rik.x);
     gacc(fy, fc * (float)rik.y);
     gacc(fz, fc * (float)rik.z);
     gacc(fz, -p.mu_p * mz_rel * (1.f / 9.f));
+}
+
+// Acceleration, energy and leapfrog part 2 of a carbon from its sums; `store`: this lane writes them.
+template <bool M, class T>
+__device__ __forceinline__ Partial<typename Prec<M>::A> carbon_finish(
+    const DevParams &p, int i, const typename Prec<M>::P4 &Ai, T gx, T gy, T gz, T gu, T gw, bool store,
+    typename Prec<M>::P4 *__restrict__ pos, typename Prec<M>::P4 *__restrict__ posOut,
+    typename Prec<M>::R *__restrict__ vel, typename Prec<M>::R *__restrict__ acc, int integrate) {
+    using R = typename Prec<M>::R;
+    using A = typename Prec<M>::A;
+    using P4 = typename Prec<M>::P4;
+    Partial<A> q;
+    partial_identity(q);
+    const R ax = (R)gx, ay = (R)gy, az = (R)gz;  // carbon mass is the unit
+    if (store && integrate != 2) {  // after the next step's half-kick here, nothing reads it before it is rewritten
+        acc[i] = ax;
+        acc[p.nMol + i] = ay;
+        acc[2 * p.nMol + i] = az;
+    }
+    const float e = (float)(T(0.5f) * gu);
+    R vx = vel[i], vy = vel[p.nMol + i], vz = vel[2 * p.nMol + i];
+    R nx = vx, ny = vy, nz = vz;
+    const bool move = Ai.x != (R)p.xLeft && Ai.x < (R)p.xRight && Ai.y != (R)p.yTop && Ai.y != (R)p.yBottom;
+    if (integrate && move) {
+#pragma clang fp contract(off)
+        const R hdt = (R)(0.5f * p.deltaT);
+        vx = vx + hdt * ax;
+        vy = vy + hdt * ay;
+        vz = vz + hdt * az;
+        nx = integrate == 2 ? vx + hdt * ax : vx;  // 2: with the next step's first half-kick
+        ny = integrate == 2 ? vy + hdt * ay : vy;
+        nz = integrate == 2 ? vz + hdt * az : vz;
+        if (store) {
+            vel[i] = nx;
+            vel[p.nMol + i] = ny;
+            vel[2 * p.nMol + i] = nz;
+        }
+    }
+    if (store) {
+        if (posOut) {  // integrate 2 with the next step's drift (k_lf1's move test: Ai is its position)
+            P4 rn = Ai;
+            rn.w = (R)e;
+            drift_wrap<R>(p, rn, move, nx, ny, nz);
+            posOut[i] = rn;
+        } else {
+            pos[i].w = (R)e;
+        }
+    }
+    q.u = (A)e;
+    q.vir = (A)(T(0.5f) * gw);
+    q.vs[0] = (A)vx;
+    q.vs[1] = (A)vy;
+    q.vs[2] = (A)vz;
+    // written out: which product a contraction rounds would depend on the code around it
+    const A v2 = fmaA((A)vz, (A)vz, fmaA((A)vx, (A)vx, (A)vy * (A)vy));
+    q.vv = v2;
+    q.vmax = v2;
+    return q;
 }
 
 // ComputeForcesK carbon branch (SurfaceGrowth.cu:899-1062, 1083-1088), one thread per carbon.
@@ -412,9 +555,11 @@ __device__ __forceinline__ Partial<typename Prec<M>::A> carbon_body(
     using A = typename Prec<M>::A;
     using P4 = typename Prec<M>::P4;
     const int ic = blk * blockDim.x + threadIdx.x;
-    Partial<A> q;
-    partial_identity(q);
-    if (ic >= p.nC) return q;
+    if (ic >= p.nC) {
+        Partial<A> q;
+        partial_identity(q);
+        return q;
+    }
     const int i = p.nMolMe + ic;
     const P4 Ai = pos[i];
     const R z0 = (R)p.z_0;
@@ -547,52 +692,214 @@ __device__ __forceinline__ Partial<typename Prec<M>::A> carbon_body(
             }
         }
     }
-    const R ax = (R)gx, ay = (R)gy, az = (R)gz;  // carbon mass is the unit
-    if (integrate != 2) {  // after the next step's half-kick here, nothing reads it before it is rewritten
-        acc[i] = ax;
-        acc[p.nMol + i] = ay;
-        acc[2 * p.nMol + i] = az;
+    return carbon_finish<M, T>(p, i, Ai, gx, gy, gz, gu, gw, true, pos, posOut, vel, acc, integrate);
+}
+
+// The same by four lanes per carbon, for launches that leave the chip idle: one lane's chain - three
+// bonds with six neighbour angles, three angles of its own, then up to 40 LJ entries four at a time -
+// lasts longer than the metal part.  Lane b < 3 evaluates bond b: its two neighbour angles, its stretch
+// and the angle between bonds b and b + 1, whose vector comes from the next lane; of 16 LJ entries
+// each lane evaluates four.  Every lane then adds all the terms, in the order of carbon_body and by the
+// same operations, so the two give the same bits: a trajectory does not depend on the lanes.
+// A term that carbon_body leaves out is added as 0.  Bound by latency: dependent gathers (bonds, their
+// neighbours, LJ entries), then a wave's own instructions.  Force launch 11.5 -> 7.4 us at 1,161 atoms,
+// 9.6 -> 6.0 at 1,175 (FP32), 14.3 -> 12.5 at 44,353; sums per lane, joined over the quad at the end, took
+// 6.5 us but round differently, and a plain-precision run shows that after 100 steps.
+template <int B>
+__device__ __forceinline__ float from_lane(float v) { return dpp_all<B * 0x55>(v); }  // quad_perm [B,B,B,B]
+template <int B>
+__device__ __forceinline__ double from_lane(double v) { return dpp_all<B * 0x55>(v); }
+
+// What one neighbour angle adds (neighbour_angle): fe along e, fr along rik, and mz.
+struct AngleTerm {
+    float fe = 0.f, fr = 0.f, mz = 0.f, ex = 0.f, ey = 0.f, ez = 0.f;
+};
+template <int B, class R>
+__device__ __forceinline__ void add_angle(const DevParams &p, const AngleTerm &a, float rx, float ry, float rz, R &fx,
+                                          R &fy, R &fz) {
+    float fc = from_lane<B>(a.fe);
+    gacc(fx, fc * from_lane<B>(a.ex));
+    gacc(fy, fc * from_lane<B>(a.ey));
+    gacc(fz, fc * from_lane<B>(a.ez));
+    fc = from_lane<B>(a.fr);
+    gacc(fx, fc * rx);
+    gacc(fy, fc * ry);
+    gacc(fz, fc * rz);
+    gacc(fz, -p.mu_p * from_lane<B>(a.mz) * (1.f / 9.f));
+}
+// What a bond adds when there are three: fs along it and dr of the stretch, the angle's two factors with
+// their vectors' sum left to the adder, and dth.
+struct BondTerm {
+    float fs = 0.f, dr = 0.f, fcb = 0.f, fca = 0.f, dth = 0.f;
+};
+template <class T>
+struct LjTerm {
+    T fc, dx, dy, dz, ul, rr;
+    int mult;
+};
+template <int B, class T>
+__device__ __forceinline__ void add_lj(const LjTerm<T> &t, T &gx, T &gy, T &gz, T &gu, T &gw) {
+    const T fc = from_lane<B>(t.fc), dx = from_lane<B>(t.dx), dy = from_lane<B>(t.dy), dz = from_lane<B>(t.dz),
+            ul = from_lane<B>(t.ul), rr = from_lane<B>(t.rr);
+    const int mult = (int)quad_word<B * 0x55>((unsigned)t.mult);
+    for (int m = 0; m < mult; ++m) {
+        gx += fc * dx;
+        gy += fc * dy;
+        gz += fc * dz;
+        gu += ul;
+        gw += fc * rr;
     }
-    const float e = (float)(T(0.5f) * gu);
-    R vx = vel[i], vy = vel[p.nMol + i], vz = vel[2 * p.nMol + i];
-    R nx = vx, ny = vy, nz = vz;
-    const bool move = Ai.x != (R)p.xLeft && Ai.x < (R)p.xRight && Ai.y != (R)p.yTop && Ai.y != (R)p.yBottom;
-    if (integrate && move) {
-#pragma clang fp contract(off)
-        const R hdt = (R)(0.5f * p.deltaT);
-        vx = vx + hdt * ax;
-        vy = vy + hdt * ay;
-        vz = vz + hdt * az;
-        nx = integrate == 2 ? vx + hdt * ax : vx;  // 2: with the next step's first half-kick
-        ny = integrate == 2 ? vy + hdt * ay : vy;
-        nz = integrate == 2 ? vz + hdt * az : vz;
-        vel[i] = nx;
-        vel[p.nMol + i] = ny;
-        vel[2 * p.nMol + i] = nz;
+}
+template <bool M, class T>
+__device__ __forceinline__ Partial<typename Prec<M>::A> carbon4_body(
+    const DevParams &p, int blk, typename Prec<M>::P4 *__restrict__ pos, typename Prec<M>::P4 *__restrict__ posOut,
+    typename Prec<M>::R *__restrict__ vel, typename Prec<M>::R *__restrict__ acc, const unsigned *__restrict__ lj,
+    const int *__restrict__ nlj, const uint4 *__restrict__ bondC, const uint4 *__restrict__ bondA, int integrate) {
+    using R = typename Prec<M>::R;
+    using P4 = typename Prec<M>::P4;
+    const int gt = blk * blockDim.x + threadIdx.x, ic = gt / 4, l = gt & 3;
+    if (ic >= p.nC) {  // whole quads
+        Partial<typename Prec<M>::A> q;
+        partial_identity(q);
+        return q;
     }
-    if (posOut) {  // integrate 2 with the next step's drift (k_lf1's move test: Ai is its position)
-        P4 rn = Ai;
-        rn.w = (R)e;
-        drift_wrap<R>(p, rn, move, nx, ny, nz);
-        posOut[i] = rn;
-    } else {
-        pos[i].w = (R)e;
+    const int i = p.nMolMe + ic;
+    const P4 Ai = pos[i];
+    const R z0 = (R)p.z_0;
+    R fx = R(0), fy = R(0), fz = R(0), u = R(0);
+    const uint4 nbi = bondC[ic];
+    const int counti = (int)nbi.w;  // at most 3: lane 3 has no bond
+    const int j0 = counti == 3 ? (int)(nbi.z & 255u) : -1;
+    const bool mine = l < counti;
+    const int kb = mine ? (int)((l == 0 ? nbi.x : l == 1 ? nbi.y : nbi.z) >> 8) : i;
+    const P4 Bk = pos[kb];
+    const uint4 nbk = bondA[mine ? kb - p.nMolMe : ic];
+    V3<R> rnn = {R(0), R(0), R(0)};
+    R absR = R(1);
+    AngleTerm at[2];
+    if (mine) {
+        const R rrr = disp<R>(Ai, Bk, p, rnn.x, rnn.y, rnn.z);
+        absR = sqrtR(rrr);
+        const unsigned me[3] = {nbk.x, nbk.y, nbk.z};
+        const int na = (int)nbk.w;
+        int ms[2] = {i, i}, nsel = 0;
+#pragma unroll
+        for (int t = 0; t < 3; ++t) {
+            const int m = (int)(me[t] >> 8);
+            if (t < na && m != i) {
+                if (nsel == 0)
+                    ms[0] = m;
+                else if (nsel == 1)
+                    ms[1] = m;
+                ++nsel;
+            }
+        }
+        P4 Bm[2];
+#pragma unroll
+        for (int t = 0; t < 2; ++t) Bm[t] = pos[ms[t]];
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            if (t >= nsel) break;
+            V3<R> e;
+            const R rr2 = disp<R>(Bk, Bm[t], p, e.x, e.y, e.z);
+            const V3<R> em = {-e.x, -e.y, -e.z};
+            angle_factors<R>(p, rnn, absR, em, rr2, at[t].fe, at[t].fr);
+            at[t].ex = (float)em.x;
+            at[t].ey = (float)em.y;
+            at[t].ez = (float)em.z;
+            at[t].mz = (float)(Bm[t].z - z0);
+        }
     }
-    q.u = (A)e;
-    q.vir = (A)(T(0.5f) * gw);
-    q.vs[0] = (A)vx;
-    q.vs[1] = (A)vy;
-    q.vs[2] = (A)vz;
-    const A v2 = (A)vx * (A)vx + (A)vy * (A)vy + (A)vz * (A)vz;
-    q.vv = v2;
-    q.vmax = v2;
-    return q;
+    const float rx = (float)rnn.x, ry = (float)rnn.y, rz = (float)rnn.z;
+    const float rx0 = from_lane<0>(rx), ry0 = from_lane<0>(ry), rz0 = from_lane<0>(rz);
+    const float rx1 = from_lane<1>(rx), ry1 = from_lane<1>(ry), rz1 = from_lane<1>(rz);
+    const float rx2 = from_lane<2>(rx), ry2 = from_lane<2>(ry), rz2 = from_lane<2>(rz);
+    add_angle<0>(p, at[0], rx0, ry0, rz0, fx, fy, fz);
+    add_angle<0>(p, at[1], rx0, ry0, rz0, fx, fy, fz);
+    add_angle<1>(p, at[0], rx1, ry1, rz1, fx, fy, fz);
+    add_angle<1>(p, at[1], rx1, ry1, rz1, fx, fy, fz);
+    add_angle<2>(p, at[0], rx2, ry2, rz2, fx, fy, fz);
+    add_angle<2>(p, at[1], rx2, ry2, rz2, fx, fy, fz);
+    if (counti == 3) {  // the same for the whole quad, as every lane that an exchange reads must be active
+        const V3<R> rn = {dpp_all<kQuadNext3>(rnn.x), dpp_all<kQuadNext3>(rnn.y), dpp_all<kQuadNext3>(rnn.z)};
+        const R absN = dpp_all<kQuadNext3>(absR);
+        const float dZ = (float)(Bk.z - z0);
+        BondTerm bt;
+        if (l < 3) {
+            bt.dr = (float)(absR - R(1));
+            bt.fs = -p.mu_r * bt.dr * rcpf((float)absR);
+            const R c = (rnn.x * rn.x + rnn.y * rn.y + rnn.z * rn.z) * rcpR(absR * absN);
+            float s;
+            bt.dth = AngleDev<R>::eval(c, p, s);
+            const float tmp = p.mu_theta * bt.dth * rcpf(s);
+            const float ra = (float)absR, rb = (float)absN, fcos = (float)c;
+            const float ira = rcpf(ra), irb = rcpf(rb);
+            const float inv = ira * irb;
+            bt.fcb = tmp * (1.f - ra * fcos * irb) * inv;
+            bt.fca = tmp * (1.f - rb * fcos * ira) * inv;
+        }
+        auto stretch = [&](float fc, float dr, float x, float y, float z) {
+            gacc(fx, fc * x);
+            gacc(fy, fc * y);
+            gacc(fz, fc * z);
+            gacc(u, p.mu_r * dr * dr);
+        };
+        stretch(from_lane<0>(bt.fs), from_lane<0>(bt.dr), rx0, ry0, rz0);
+        stretch(from_lane<1>(bt.fs), from_lane<1>(bt.dr), rx1, ry1, rz1);
+        stretch(from_lane<2>(bt.fs), from_lane<2>(bt.dr), rx2, ry2, rz2);
+        const float zi = (float)(Ai.z - z0), dZs = from_lane<0>(dZ) + from_lane<1>(dZ) + from_lane<2>(dZ);
+        float dz = 2.f * zi - dZs;
+        gacc(fz, -0.666666667f * p.mu_p * dz);
+        dz = zi - 0.33333333f * dZs;
+        gacc(u, p.mu_p * dz * dz);
+        auto angle = [&](float fcb, float fca, float dth, float bx, float by, float bz, float ax, float ay, float az) {
+            gacc(fx, fcb * bx + fca * ax);
+            gacc(fy, fcb * by + fca * ay);
+            gacc(fz, fcb * bz + fca * az);
+            gacc(u, p.mu_theta * dth * dth);
+        };
+        angle(from_lane<0>(bt.fcb), from_lane<0>(bt.fca), from_lane<0>(bt.dth), rx1, ry1, rz1, rx0, ry0, rz0);
+        angle(from_lane<1>(bt.fcb), from_lane<1>(bt.fca), from_lane<1>(bt.dth), rx2, ry2, rz2, rx1, ry1, rz1);
+        angle(from_lane<2>(bt.fcb), from_lane<2>(bt.fca), from_lane<2>(bt.dth), rx0, ry0, rz0, rx2, ry2, rz2);
+    }
+    T gx = (T)fx, gy = (T)fy, gz = (T)fz, gu = (T)u, gw = T(0);
+    const int nl = nlj[ic];
+    for (int base = 0; base < nl; base += 16) {
+        unsigned e[4];
+        P4 B[4];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) e[t] = lj[(size_t)min(base + 4 * t + l, nl - 1) * p.nC + ic];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) B[t] = pos[e[t] >> 8];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            if (base + 4 * t >= nl) break;  // the same for the whole quad
+            LjTerm<T> g = {};
+            const int pk = (int)(e[t] & 255u);
+            const int mult = j0 < 0 ? 1 : (int)(pk <= j0) + (int)(pk >= 4);
+            R dxr, dyr, dzr;
+            const R rrr = disp<R>(Ai, B[t], p, dxr, dyr, dzr);
+            if (base + 4 * t + l < nl && mult != 0 && rrr < (R)p.rrCutLJ) {
+                g.fc = lj_pair<T>(p, (T)rrr, g.ul);
+                g.dx = (T)dxr;
+                g.dy = (T)dyr;
+                g.dz = (T)dzr;
+                g.rr = (T)rrr;
+                g.mult = mult;
+            }
+            add_lj<0>(g, gx, gy, gz, gu, gw);
+            add_lj<1>(g, gx, gy, gz, gu, gw);
+            add_lj<2>(g, gx, gy, gz, gu, gw);
+            add_lj<3>(g, gx, gy, gz, gu, gw);
+        }
+    }
+    return carbon_finish<M, T>(p, i, Ai, gx, gy, gz, gu, gw, l == 0, pos, posOut, vel, acc, integrate);
 }
 
 // One workgroup of the force launch (blocks [0, nbM) metal, [nbM, nb) carbon): forces, energies,
 // leapfrog part 2 and the block's Partial in part[b].
 template <bool M, class T, int G>
-__device__ __forceinline__ void force_block(const DevParams &p, int b, int nbM, int nb, bool xm,
+__device__ __forceinline__ void force_block(bool quad, const DevParams &p, int b, int nbM, int nb, bool xm,
                                             typename Prec<M>::P4 *__restrict__ pos,
                                             typename Prec<M>::P4 *__restrict__ posOut,
                                             typename Prec<M>::R *__restrict__ vel, typename Prec<M>::R *__restrict__ acc,
@@ -608,15 +915,22 @@ __device__ __forceinline__ void force_block(const DevParams &p, int b, int nbM, 
     if (b < nbM) {
         const Partial<A> q = metal_body<M, T, G>(p, xm ? xcd_block(b, nbM) : b, pos, posOut, vel, acc, nlM, nnM, embF,
                                                  embDF, fric, integrate);
-        block_store_partial<true, G>(q, part + b, vmax ? vmax + b : nullptr);
+        if (integrate) block_store_partial<true, G>(q, part + b, vmax ? vmax + b : nullptr);
     } else {
-        const Partial<A> q = carbon_body<M, T>(p, xm ? xcd_block(b - nbM, nb - nbM) : b - nbM, pos, posOut, vel, acc,
-                                               lj, nlj, bondC, bondA, integrate);
-        block_store_partial<false, 1>(q, part + b, vmax ? vmax + b : nullptr);
+        if (quad) {
+            const QuadBlock at = quad_block(b - nbM, p.nC, xm);
+            if (at.slot < 0) return;
+            const Partial<A> q = carbon4_body<M, T>(p, at.blk, pos, posOut, vel, acc, lj, nlj, bondC, bondA, integrate);
+            if (integrate) block_store_quad(q, part + nbM + at.slot, vmax ? vmax + nbM + at.slot : nullptr);
+        } else {
+            const Partial<A> q = carbon_body<M, T>(p, xm ? xcd_block(b - nbM, nb - nbM) : b - nbM, pos, posOut, vel, acc,
+                                                   lj, nlj, bondC, bondA, integrate);
+            if (integrate) block_store_partial<false, 1>(q, part + b, vmax ? vmax + b : nullptr);
+        }
     }
 }
 
-template <bool M, class T, int G>
+template <bool M, class T, int G, int CL>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_force(DevParams p, int nbM, typename Prec<M>::P4 *__restrict__ pos,
                                                typename Prec<M>::P4 *__restrict__ posOut,
                                                typename Prec<M>::R *__restrict__ vel, typename Prec<M>::R *__restrict__ acc,
@@ -635,7 +949,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
         return;
     }
     // nbM is a multiple of 8: both ranges keep the XCD of each block
-    force_block<M, T, G>(p, blockIdx.x - first, nbM, gridDim.x - first, p.xcdMap & 4, pos, posOut, vel, acc, nlM, nnM, embF, embDF,
+    force_block<M, T, G>(CL == 4, p, blockIdx.x - first, nbM, gridDim.x - first, p.xcdMap & 4, pos, posOut, vel, acc, nlM, nnM, embF, embDF,
                          fric, lj, nlj, bondC, bondA, part, vmax, integrate);
 }
 
@@ -647,7 +961,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     const int2 e = a.forceTab[blockIdx.x];
     const BatchRep &B = a.reps[e.x];
     const DevParams &p = B.p;
-    force_block<M, T, G>(p, e.y, B.nbM, B.nbForce, false, (typename Prec<M>::P4 *)a.pos + B.atomOff,
+    force_block<M, T, G>(B.carbonLanes == 4, p, e.y, B.nbM, B.nbForce, false, (typename Prec<M>::P4 *)a.pos + B.atomOff,
                          a.posOut ? (typename Prec<M>::P4 *)a.posOut + B.atomOff : nullptr,
                          (R *)a.vel + 3 * B.atomOff, (R *)a.acc + 3 * B.atomOff, a.nlM + B.metalOff * p.nlCap,
                          a.nnM + B.metalOff, a.embF + B.metalOff, a.embDF + B.metalOff, a.fric + B.metalOff,
@@ -661,11 +975,13 @@ template <bool M, class T>
 static void rho_dispatch(sgk_ctx *c) {
     using P4 = typename Prec<M>::P4;
     const int G = c->metalLanes;
-    const unsigned g = (unsigned)(c->nbRho + c->nbC);
+    const bool quad = c->carbonLanes == 4;
+    const unsigned g = (unsigned)(c->nbRho + (quad ? quad_grid(c->nbC, c->dp.xcdMap & 2) : c->nbC));
     const P4 *pos = (const P4 *)c->pos;
-#define SGK_RHO(GG)                                                                                              \
-    hipLaunchKernelGGL((k_rho<M, T, GG>), dim3(g), dim3(256), 0, c->stream, c->dp, c->nbRho, pos, c->nlM, c->nnM, \
-                       c->rho, c->embF, c->embDF, c->cl, c->ncl, c->bondC, c->bondA)
+#define SGK_RHO(GG)                                                                                                \
+    hipLaunchKernelGGL((quad ? k_rho<M, T, GG, 4> : k_rho<M, T, GG, 1>), dim3(g), dim3(256), 0,      \
+                       c->stream, c->dp, c->nbRho, pos, c->nlM, c->nnM, c->rho, c->embF, c->embDF, c->cl, c->ncl, \
+                       c->bondC, c->bondA)
     switch (G) {
         case 1: SGK_RHO(1); break;
         case 2: SGK_RHO(2); break;
@@ -682,13 +998,14 @@ static void force_dispatch(sgk_ctx *c, int integrate, void *posOut, bool closePr
     using R = typename Prec<M>::R;
     using A = typename Prec<M>::A;
     const int G = c->metalLanes;
-    const int nParts = c->nbM + c->nbC;
-    const unsigned g = (unsigned)nParts + (closePrev ? 1u : 0u);
+    const bool quad = c->carbonLanes == 4;
+    const unsigned g = (unsigned)(c->nbM + (quad ? quad_grid(c->nbC, c->dp.xcdMap & 4) : c->nbC)) + (closePrev ? 1u : 0u);
     StepClose<A> close = {};
     if (closePrev) {
-        const bool direct = nParts <= kCloseDirectParts;
+        const PartMap map = part_map(c);
+        const bool direct = map.count() <= kCloseDirectParts;
         close.part = (const Partial<A> *)c->partialsAlt + (direct ? 0 : c->part2Off);
-        close.n = direct ? nParts : (nParts + kPartChunk - 1) / kPartChunk;
+        close.map = direct ? map : plain_map((map.count() + kPartChunk - 1) / kPartChunk);
         close.direct = direct;
         close.old = c->stateAlt;
         close.st = c->state;
@@ -700,8 +1017,8 @@ static void force_dispatch(sgk_ctx *c, int integrate, void *posOut, bool closePr
     R *vel = (R *)c->vel;
     Partial<A> *part = (Partial<A> *)c->partials;
 #define SGK_F(GG)                                                                                                \
-    hipLaunchKernelGGL((k_force<M, T, GG>), dim3(g), dim3(256), 0, c->stream, c->dp, c->nbM, pos, (P4 *)posOut,  \
-                       vel, (R *)c->acc,                                                                        \
+    hipLaunchKernelGGL((quad ? k_force<M, T, GG, 4> : k_force<M, T, GG, 1>), dim3(g), dim3(256),  \
+                       0, c->stream, c->dp, c->nbM, pos, (P4 *)posOut, vel, (R *)c->acc,                                                                        \
                        c->nlM, c->nnM, c->embF, c->embDF, c->fric, c->lj, c->nlj, c->bondC, c->bondA, part,     \
                        (A *)c->partVmax, integrate, close)
     switch (G) {

@@ -74,7 +74,7 @@ struct sgk_ctx {
     sgk::DevState *hostState = nullptr;                 // pinned mirror
     sgk::HostStage stage;                               // state transfer, grown on demand
     // launch geometry
-    int block = 256, metalLanes = 8, nbM = 0, nbC = 0, nbRho = 0, nbProps = 0;
+    int block = 256, metalLanes = 8, carbonLanes = 1, nbM = 0, nbC = 0, nbRho = 0, nbProps = 0;
     int part2Off = 0;                                   // chunk totals of the step reduction (in partials)
     long long bytes = 0;
     bool haveList = false;
@@ -107,6 +107,15 @@ constexpr int kNlMetalLanes = 4;
 // 1.1 M 224 / 248; batches of 373,577 atoms 112.9 / 113.0, of 448,542 125.0 / 127.4.
 constexpr int kNineAtoms = 4 * 7;
 constexpr int kNlNineAtoms = 1 << 18;
+// A system, or a batch in all, of up to so many carbons takes four lanes per carbon in the density and
+// force passes: there one lane's chain, not the chip's throughput, sets the time.  The results are the
+// same bits either way.  Whole step with one lane / four (us), FP64 pairs unless said: 1,161 atoms
+// 27.3 / 21.1, 18,896 29.5 / 25.4, 50,208 34.6 / 33.9, 60,448 34.9 / 36.0; FP32 17,196 24.9 / 21.1, 33,768
+// 27.3 / 23.5; 14 replicas of 31,901 together 38.1 / 35.2, 64 of 413,000 107 / 126.
+constexpr int kQuadCarbons = 49152;
+inline int carbon_lanes(long long nC) { return nC <= kQuadCarbons ? 4 : 1; }
+// Carbon workgroups that store a partial: one per 256 carbons, in four parts with four lanes.
+inline int carbon_blocks(long long nC, int lanes) { return (int)((nC + 255) / 256) * lanes; }
 // Reference-stencil RDF.
 constexpr int kRdfAtoms = 8;          // atoms a workgroup takes at once
 constexpr int kRdfBlocks = 512;       // workgroups per launch at most: each merges its bins into one histogram
@@ -123,6 +132,9 @@ inline int metal_blocks(long long nMe, int G, int xcdMap) {
     const long long nb = (nMe * G + 255) / 256;
     return (int)((xcdMap & 6) ? (nb + 7) / 8 * 8 : nb);
 }
+
+// The force pass's partials of a step.
+inline sgk::PartMap part_map(const sgk_ctx *c) { return {c->nbM, c->nbM + c->nbC, c->carbonLanes == 4}; }
 
 struct sgk_batch {
     int nrep = 0;

@@ -1624,8 +1624,9 @@ void launch_bin_next(sgk_ctx *c) {
     if (c->dp.nMol == 0) return;
     profile_begin(c);
     const unsigned g = blocks_for(c->dp.nMol, 256);
-    const int nParts = c->nbM + c->nbC, nChunks = (nParts + kPartChunk - 1) / kPartChunk;
-    const bool direct = nParts <= kCloseDirectParts;
+    const PartMap map = part_map(c);
+    const int nParts = map.stored, nChunks = (map.count() + kPartChunk - 1) / kPartChunk;
+    const bool direct = map.count() <= kCloseDirectParts;
 #define SGK_BN(MM, P4, A)                                                                                              \
     hipLaunchKernelGGL(k_bin_next<MM>, dim3(g), dim3(256), 0, c->stream, c->dp, (const P4 *)c->pos, cell_bufs(c),     \
                        direct ? (const A *)c->partVmaxAlt                                                               \

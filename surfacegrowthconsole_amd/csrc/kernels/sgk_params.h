@@ -65,6 +65,18 @@ struct Partial {
     T vir;  // pair virial 1/2 sum f_ik |d_ik|^2 of the EAM and LJ terms (force pass only)
 };
 
+// The partials of a step: nbM of the metal workgroups, then the carbon ones.  With four lanes per carbon
+// (quad) a workgroup holds 64 carbons, and four workgroups are the parts of the one of 256 that a lane per
+// carbon gives: their partials are joined in order, as the waves of that workgroup are, so the sums of a
+// step do not depend on the lanes.
+struct PartMap {
+    int nbM, stored, quad;
+    __host__ __device__ int count() const { return quad ? nbM + (stored - nbM) / 4 : stored; }
+    __device__ int first(int k) const { return quad && k >= nbM ? nbM + 4 * (k - nbM) : k; }
+    __device__ int parts(int k) const { return quad && k >= nbM ? 4 : 1; }
+};
+inline __host__ __device__ PartMap plain_map(int n) { return {n, n, 0}; }
+
 // Device-resident run state.  A context has two: a step whose closing is folded into the next step
 // leaves its state as it is, and the next step's first kernel writes the advanced state into the
 // other one (k_bin_next), because all of its workgroups still read the old one.

@@ -154,15 +154,65 @@ __device__ __forceinline__ void block_store_partial(Partial<T> q, Partial<T> *ou
     if (vmax && f == kPartVmax) *vmax = r;
 }
 
+// The same sums for a workgroup with four lanes per carbon (64 carbons), each of which holds its carbon's
+// contribution: lane l of a quad takes two fields, the quads of a row of 16 lanes are summed in it and the
+// rows in LDS.  The tree is that of one wave of block_store_partial with a carbon per lane.
+template <class T>
+__device__ __forceinline__ void block_store_quad(Partial<T> q, Partial<T> *out, T *vmax) {
+    __shared__ T rows[16][8];
+    const int l = threadIdx.x & 3, f = threadIdx.x;
+    T a = q.vmax, b = q.vs[2];
+    if (l == 2) a = q.vv;
+    if (l == 1) {
+        a = q.vir;
+        b = q.vs[1];
+    }
+    if (l == 0) {
+        a = q.u;
+        b = q.vs[0];
+    }
+    const T a4 = dpp<kRowShr4, 0xF>(T(0), a);
+    a = l == 3 ? OpMax::f(a, a4) : a + a4;
+    b += dpp<kRowShr4, 0xF>(T(0), b);
+    const T a8 = dpp<kRowShr8, 0xF>(T(0), a);
+    a = l == 3 ? OpMax::f(a, a8) : a + a8;
+    b += dpp<kRowShr8, 0xF>(T(0), b);
+    if ((threadIdx.x & 15) >= 12) {
+        rows[threadIdx.x >> 4][2 * l] = a;
+        rows[threadIdx.x >> 4][2 * l + 1] = b;
+    }
+    __syncthreads();
+    if (f >= kPartFields) return;
+    const int at = f == 0 ? 0 : f == 8 ? 1 : f == kPartVir ? 2 : f == 9 ? 3 : f == kPartVv ? 4 : f == 10 ? 5 : f == kPartVmax ? 6 : -1;
+    T r = f >= kPartBmin && f < kPartBmax ? T(3.0e38f) : (f >= kPartBmax && f < kPartVir ? T(-3.0e38f) : T(0));
+    if (at >= 0) {
+        T x[16];
+#pragma unroll
+        for (int k = 0; k < 16; ++k) x[k] = rows[k][at];
+#pragma unroll
+        for (int d = 1; d < 16; d *= 2)
+#pragma unroll
+            for (int k = 0; k < 16; k += 2 * d) x[k] = f == kPartVmax ? OpMax::f(x[k], x[k + d]) : x[k] + x[k + d];
+        r = x[0];
+    }
+    ((T *)out)[f] = r;
+    if (vmax && f == kPartVmax) *vmax = r;
+}
+
 // First stage of the step reduction: one wave reduces a chunk of up to kPartChunk partials (lane k
 // takes partial k; fixed order), the result goes to *out.  The chunk count is wave-uniform.
+// Chunk j of the map's partials.
 constexpr int kPartChunk = 64;
 template <class T>
-__device__ __forceinline__ void reduce_chunk(const Partial<T> *part, int n, Partial<T> *out) {
-    const int lane = threadIdx.x & 63;
+__device__ __forceinline__ void reduce_chunk(const Partial<T> *part, const PartMap &map, int j, Partial<T> *out) {
+    const int lane = threadIdx.x & 63, k = j * kPartChunk + lane;
     Partial<T> q;
     partial_identity(q);
-    if (lane < n) q = part[lane];
+    if (k < map.count()) {
+        const Partial<T> *at = part + map.first(k);
+        q = at[0];
+        for (int s = 1; s < map.parts(k); ++s) partial_combine(q, at[s]);
+    }
     partial_wave(q);
     if (lane == 63) *out = q;
 }
@@ -199,84 +249,135 @@ __device__ __forceinline__ StepNext<A> step_next(const DevParams &p, const DevSt
     return n;
 }
 
-// Total of n partials by one workgroup of 256 threads, returned to every thread.  A thread takes one
-// field of 16 partials: their loads are all in flight at once and a field's tree is 15 operations in
-// registers, where a lane per partial moved 20 fields through 6 exchange steps each, twice, and a
-// launch of one workgroup has nothing to hide them behind.  The trees are reduce_chunk's (rows of 16,
-// then the rows of a chunk) and so are the sums, bit for bit.
+// Total of the map's n partials by one workgroup of 256 threads, returned to every thread.  A thread takes
+// one field of four partials: their loads are all in flight at once and a field's tree is a few
+// operations in registers, where a lane per partial moved 20 fields through 6 exchange steps each,
+// twice, and a launch of one workgroup has nothing to hide them behind.  The trees are reduce_chunk's
+// (fours, rows of 16, then the rows of a chunk) and so are the sums, bit for bit.
 // totals: the n are chunk totals (any number): thread t of 256 first adds totals t, t + 256, ... in order.
 // Otherwise at most kSumParts partials: chunks of 64, then the chunk totals as the first 16 lanes of a wave.
 // One launch for up to 1,024 partials in place of k_reduce1 and k_finalize: a sheared step of 997 atoms
 // (FP32) 29.1 -> 26.8 us, a deposition step of 4,393 27.2 -> 25.3, kb_finalize of 64 replicas 8.0 -> 6.5.
-constexpr int kSumRows = 64, kSumParts = 16 * kSumRows, kSumGroups = 256 / kPartFields;
+constexpr int kSumFours = 64, kSumParts = 1024, kSumGroups = 256 / kPartFields;
 
-// One field of a tree: all lanes run the same instructions, the field picks its result.
-enum class FieldOp : int { sum, max, min };
-__device__ __forceinline__ FieldOp field_op(int f) {
-    return f == kPartVmax || (f >= kPartBmax && f < kPartVir) ? FieldOp::max
-           : f >= kPartBmin && f < kPartBmax                  ? FieldOp::min
-                                                              : FieldOp::sum;
-}
+// One field of a tree: sums add, the others keep the larger value, minima with their sign turned.
 template <class A>
-__device__ __forceinline__ A field_id(int f) {
-    return f >= kPartBmin && f < kPartBmax ? A(3.0e38f) : (f >= kPartBmax && f < kPartVir ? A(-3.0e38f) : A(0));
-}
+struct Field {
+    bool sum, turn;
+    A id;
+    __device__ explicit Field(int f)
+        : sum(f < kPartVmax || f >= kPartVir), turn(f >= kPartBmin && f < kPartBmax),
+          id(f >= kPartBmin && f < kPartVir ? A(-3.0e38f) : A(0)) {}
+    __device__ __forceinline__ A in(A x) const { return turn ? -x : x; }  // its own inverse
+    __device__ __forceinline__ A join(A x, A y) const {
+        const A s = x + y, m = y > x ? y : x;
+        return sum ? s : m;
+    }
+    __device__ __forceinline__ A four(A a, A b, A c, A d) const { return join(join(a, b), join(c, d)); }
+};
+
+// Partials 4q .. 4q + 3 of the map's first `lanes`, one field, joined as the tree takes them.
 template <class A>
-__device__ __forceinline__ A field_join(FieldOp op, A x, A y) {
-    const A s = x + y, hi = y > x ? y : x, lo = y < x ? y : x;
-    return op == FieldOp::sum ? s : (op == FieldOp::max ? hi : lo);
-}
-template <class A>
-__device__ __forceinline__ A field_tree16(FieldOp op, A (&x)[16]) {
+__device__ __forceinline__ A field_four(const Field<A> &fl, const A *src, const PartMap &map, int q, int lanes) {
+    const int k0 = 4 * q;
+    if (map.quad && k0 >= map.nbM && k0 + 4 <= lanes) {  // sixteen in a row
+        const A *s = src + (size_t)map.first(k0) * kPartFields;
+        A v[16];
 #pragma unroll
-    for (int d = 1; d < 16; d *= 2)
+        for (int t = 0; t < 16; ++t) v[t] = fl.in(s[t * kPartFields]);
 #pragma unroll
-        for (int j = 0; j < 16; j += 2 * d) x[j] = field_join(op, x[j], x[j + d]);
-    return x[0];
+        for (int t = 0; t < 16; t += 4) v[t] = fl.join(fl.join(fl.join(v[t], v[t + 1]), v[t + 2]), v[t + 3]);
+        return fl.four(v[0], v[4], v[8], v[12]);
+    }
+    A x[4];
+    if (!map.quad || k0 + 4 <= map.nbM) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) x[j] = src[(size_t)min(k0 + j, map.stored - 1) * kPartFields];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) x[j] = k0 + j < lanes ? fl.in(x[j]) : fl.id;
+    } else {  // metal and carbon, or the last: all loads in flight, those past an end discarded
+        A v[4][4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int s = 0; s < 4; ++s) v[j][s] = src[(size_t)min(map.first(k0 + j) + s, map.stored - 1) * kPartFields];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int have = k0 + j < lanes ? map.parts(k0 + j) : 0;
+            x[j] = have > 0 ? fl.in(v[j][0]) : fl.id;
+#pragma unroll
+            for (int s = 1; s < 4; ++s) x[j] = have > s ? fl.join(x[j], fl.in(v[j][s])) : x[j];
+        }
+    }
+    return fl.four(x[0], x[1], x[2], x[3]);
 }
 
 template <class A>
-__device__ __forceinline__ Partial<A> sum_parts(const Partial<A> *part, int n, bool totals) {
+__device__ __forceinline__ Partial<A> sum_parts(const Partial<A> *part, const PartMap &map, bool totals) {
     static_assert(sizeof(Partial<A>) == kPartFields * sizeof(A), "fields of Partial in their order");
-    __shared__ A rows[kSumRows][kPartFields], chunks[16][kPartFields];
+    __shared__ A fours[kSumFours][kPartFields], chunks[16][kPartFields];
     __shared__ Partial<A> total;
     const int f = threadIdx.x % kPartFields, g = threadIdx.x / kPartFields;
     const bool mine = g < kSumGroups;
-    const FieldOp op = field_op(f);
-    const A id = field_id<A>(f);
-    const int lanes = totals ? min(n, 256) : n, nRows = (lanes + 15) / 16, nChunks = (nRows + 3) / 4;
+    const Field<A> fl(f);
+    const int n = map.count(), lanes = totals ? min(n, 256) : n, nFours = (lanes + 3) / 4, nChunks = (lanes + 63) / 64;
     const A *src = (const A *)part + f;
-    if (mine)
-        for (int r = g; r < nRows; r += kSumGroups) {
-            A x[16];
+    // four fours in a row per thread where one would leave it with 4 loads in flight and many rounds
+    const bool rows = !map.quad && nFours > 2 * kSumGroups;
+    for (int pass = 0; pass * kSumFours < nFours; ++pass) {
+        const int q0 = pass * kSumFours, here = min(kSumFours, nFours - q0);
+        if (pass) __syncthreads();
+        if (mine && totals && n > 256) {
+            for (int q = g; q < here; q += kSumGroups) {
+                A x[4];
 #pragma unroll
-            for (int j = 0; j < 16; ++j) x[j] = 16 * r + j < lanes ? src[(16 * r + j) * kPartFields] : id;
-            if (totals)
-                for (int k = 256 + 16 * r; k < n; k += 256)
+                for (int j = 0; j < 4; ++j) {
+                    x[j] = fl.in(src[(size_t)(4 * q + j) * kPartFields]);
+                    for (int k = 4 * q + j + 256; k < n; k += 256) x[j] = fl.join(x[j], fl.in(src[(size_t)k * kPartFields]));
+                }
+                fours[q][f] = fl.four(x[0], x[1], x[2], x[3]);
+            }
+        } else if (mine && rows) {
+            for (int q = 4 * g; q < here; q += 4 * kSumGroups) {
+                const int k0 = 4 * (q0 + q);
+                A v[16];
 #pragma unroll
-                    for (int j = 0; j < 16; ++j)
-                        if (k + j < n) x[j] = field_join(op, x[j], src[(size_t)(k + j) * kPartFields]);
-            rows[r][f] = field_tree16(op, x);
+                for (int t = 0; t < 16; ++t) v[t] = src[(size_t)min(k0 + t, n - 1) * kPartFields];
+#pragma unroll
+                for (int t = 0; t < 16; ++t) v[t] = k0 + t < lanes ? fl.in(v[t]) : fl.id;
+#pragma unroll
+                for (int t = 0; t < 16; t += 4) fours[q + t / 4][f] = fl.four(v[t], v[t + 1], v[t + 2], v[t + 3]);
+            }
+        } else if (mine) {
+            for (int q = g; q < here; q += kSumGroups) fours[q][f] = field_four(fl, src, map, q0 + q, lanes);
         }
-    __syncthreads();
-    if (mine)
-        for (int c = g; c < nChunks; c += kSumGroups) {
-            auto row = [&](int r) { return r < nRows ? rows[r][f] : id; };
-            chunks[c][f] = field_join(op, field_join(op, row(4 * c + 3), row(4 * c + 2)),
-                                      field_join(op, row(4 * c + 1), row(4 * c)));
+        __syncthreads();
+        if (g < 4 && 16 * g < here) {
+            A r[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                auto four = [&](int j) { return 16 * g + 4 * k + j < here ? fours[16 * g + 4 * k + j][f] : fl.id; };
+                r[k] = fl.four(four(0), four(1), four(2), four(3));
+            }
+            chunks[4 * pass + g][f] = fl.four(r[3], r[2], r[1], r[0]);
         }
+    }
     __syncthreads();
     if (g == 0) {
-        A r = n > 0 ? chunks[0][f] : id;
+        A r = n > 0 ? chunks[0][f] : fl.id;
         if (totals) {
-            for (int c = 1; c < nChunks; ++c) r = field_join(op, r, chunks[c][f]);
+            for (int c = 1; c < nChunks; ++c) r = fl.join(r, chunks[c][f]);
         } else if (nChunks > 1) {
             A x[16];
 #pragma unroll
-            for (int c = 0; c < 16; ++c) x[c] = c < nChunks ? chunks[c][f] : id;
-            r = field_tree16(op, x);
+            for (int c = 0; c < 16; ++c) x[c] = c < nChunks ? chunks[c][f] : fl.id;
+#pragma unroll
+            for (int d = 1; d < 16; d *= 2)
+#pragma unroll
+                for (int j = 0; j < 16; j += 2 * d) x[j] = fl.join(x[j], x[j + d]);
+            r = x[0];
         }
-        ((A *)&total)[f] = r;
+        ((A *)&total)[f] = fl.in(r);
     }
     __syncthreads();
     return total;
@@ -322,15 +423,15 @@ __device__ __forceinline__ void record_sums(const DevParams &p, const Partial<A>
     rec.pad = 0;
 }
 
-// Reduce nParts partials (totals: chunk totals) with the whole workgroup of 256, then evaluate the
+// Reduce the map's partials (totals: chunk totals) with the whole workgroup of 256, then evaluate the
 // reference's host arithmetic of SurfaceGrowth.cu:2307-2395 in thread 0.
 // mode 0: one step - advance the step counter, commit a rebuild, update dispHi / nebrNow / shear,
 //         append a record.  mode 1: evaluation only - write records[0], leave the state alone.
 template <class A>
-__device__ void finalize_body(const DevParams &p, const Partial<A> *part, int nParts, bool totals, DevState *st,
+__device__ void finalize_body(const DevParams &p, const Partial<A> *part, const PartMap &map, bool totals, DevState *st,
                               sgk_record *records, int recCap, int mode) {
     const DevState s0 = *st;  // before the sums: its latency passes meanwhile
-    const Partial<A> P = sum_parts(part, nParts, totals);
+    const Partial<A> P = sum_parts(part, map, totals);
     if (threadIdx.x != 0) return;
     const int nMe = p.nMolMe;
     sgk_record rec;
@@ -397,7 +498,8 @@ constexpr int kCloseDirectParts = kSumParts;
 template <class A>
 struct StepClose {
     const Partial<A> *part;  // force-pass partials, or chunk totals (direct = 0)
-    int n, direct;           // their number; 1: reduce the chunks here
+    PartMap map;
+    int direct;              // 1: reduce the chunks here
     DevState *old, *st;      // the closed step's state, and the advanced one
     sgk_record *records;
     int recCap, on;
@@ -407,7 +509,7 @@ struct StepClose {
 // The sums are those of k_reduce1 and k_finalize, bit for bit.
 template <class A>
 __device__ __forceinline__ void close_body(const DevParams &p, const StepClose<A> &c) {
-    const Partial<A> P = sum_parts(c.part, c.n, !c.direct);
+    const Partial<A> P = sum_parts(c.part, c.map, !c.direct);
     if (threadIdx.x != 0) return;
     sgk_record rec;
     A cmVelX, vvSum;

@@ -190,19 +190,18 @@ __global__ __launch_bounds__(256) void k_props(DevParams p, const typename Prec<
 // mode 1 reduces k_props partials, which count as totals.
 constexpr int kFinalizeThreads = 256;
 template <bool M>
-__global__ __launch_bounds__(256) void k_reduce1(const Partial<typename Prec<M>::A> *__restrict__ part, int nParts,
+__global__ __launch_bounds__(256) void k_reduce1(const Partial<typename Prec<M>::A> *__restrict__ part, PartMap map,
                                                  Partial<typename Prec<M>::A> *__restrict__ part2) {
     const int j = blockIdx.x * 4 + (threadIdx.x >> 6);
-    const int nChunks = (nParts + kPartChunk - 1) / kPartChunk;
-    if (j < nChunks) reduce_chunk(part + j * kPartChunk, min(kPartChunk, nParts - j * kPartChunk), part2 + j);
+    if (j * kPartChunk < map.count()) reduce_chunk(part, map, j, part2 + j);
 }
 
 template <bool M>
 __global__ __launch_bounds__(kFinalizeThreads) void k_finalize(DevParams p,
                                                                const Partial<typename Prec<M>::A> *__restrict__ part,
-                                                               int nParts, int totals, DevState *st,
+                                                               PartMap map, int totals, DevState *st,
                                                                sgk_record *records, int recCap, int mode) {
-    finalize_body<typename Prec<M>::A>(p, part, nParts, totals, st, records, recCap, mode);
+    finalize_body<typename Prec<M>::A>(p, part, map, totals, st, records, recCap, mode);
 }
 
 // Batched: one workgroup per replica, which also reduces the chunks where the partials are too many to
@@ -212,15 +211,17 @@ __global__ __launch_bounds__(kFinalizeThreads) void kb_finalize(BatchArgs a) {
     using A = typename Prec<M>::A;
     const BatchRep &B = a.reps[blockIdx.x];
     const Partial<A> *part = (const Partial<A> *)a.partials + B.partOff;
-    const bool totals = B.nbForce > kSumParts;
+    PartMap map = {B.nbM, B.nbForce, B.carbonLanes == 4};
+    const bool totals = map.count() > kSumParts;
     if (totals) {
         Partial<A> *part2 = (Partial<A> *)a.partials + B.part2Off;
         for (int j = threadIdx.x >> 6; j < B.nChunks; j += kFinalizeThreads / 64)
-            reduce_chunk(part + j * kPartChunk, min(kPartChunk, B.nbForce - j * kPartChunk), part2 + j);
+            reduce_chunk(part, map, j, part2 + j);
         __syncthreads();
         part = part2;
+        map = plain_map(B.nChunks);
     }
-    finalize_body<A>(B.p, part, totals ? B.nChunks : B.nbForce, totals, a.state + blockIdx.x,
+    finalize_body<A>(B.p, part, map, totals, a.state + blockIdx.x,
                      a.records + (size_t)blockIdx.x * a.recCap, a.recCap, 0);
 }
 
@@ -457,30 +458,31 @@ template <bool M>
 static void finalize_dispatch(sgk_ctx *c, int mode) {
     using A = typename Prec<M>::A;
     Partial<A> *part = (Partial<A> *)c->partials;
-    int n = mode == 1 ? c->nbProps : c->nbM + c->nbC;
-    const bool totals = mode == 1 || n > kSumParts;
+    PartMap map = mode == 1 ? plain_map(c->nbProps) : part_map(c);
+    const bool totals = mode == 1 || map.count() > kSumParts;
     if (mode != 1 && totals) {
-        const int nChunks = (n + kPartChunk - 1) / kPartChunk;
-        hipLaunchKernelGGL(k_reduce1<M>, dim3((nChunks + 3) / 4), dim3(256), 0, c->stream, part, n, part + c->part2Off);
+        const int nChunks = (map.count() + kPartChunk - 1) / kPartChunk;
+        hipLaunchKernelGGL(k_reduce1<M>, dim3((nChunks + 3) / 4), dim3(256), 0, c->stream, part, map, part + c->part2Off);
         part += c->part2Off;
-        n = nChunks;
+        map = plain_map(nChunks);
     }
-    hipLaunchKernelGGL(k_finalize<M>, dim3(1), dim3(kFinalizeThreads), 0, c->stream, c->dp, part, n, (int)totals, c->state,
-                       c->records, mode == 1 ? 1 : c->cfg.records_capacity, mode);
+    hipLaunchKernelGGL(k_finalize<M>, dim3(1), dim3(kFinalizeThreads), 0, c->stream, c->dp, part, map, (int)totals,
+                       c->state, c->records, mode == 1 ? 1 : c->cfg.records_capacity, mode);
 }
 
 // The first reduction stage alone, for a step whose closing is folded into the next one: chunk totals
 // where the partials are too many for the workgroups that take it over.
 void launch_reduce_chunks(sgk_ctx *c) {
-    const int nParts = c->nbM + c->nbC, nChunks = (nParts + kPartChunk - 1) / kPartChunk;
-    if (nParts <= kCloseDirectParts) return;
+    const PartMap map = part_map(c);
+    const int nChunks = (map.count() + kPartChunk - 1) / kPartChunk;
+    if (map.count() <= kCloseDirectParts) return;
     profile_begin(c);
     const dim3 g((nChunks + 3) / 4), t(256);
     if (c->mixed)
-        hipLaunchKernelGGL(k_reduce1<true>, g, t, 0, c->stream, (const Partial<double> *)c->partials, nParts,
+        hipLaunchKernelGGL(k_reduce1<true>, g, t, 0, c->stream, (const Partial<double> *)c->partials, map,
                            (Partial<double> *)c->partials + c->part2Off);
     else
-        hipLaunchKernelGGL(k_reduce1<false>, g, t, 0, c->stream, (const Partial<float> *)c->partials, nParts,
+        hipLaunchKernelGGL(k_reduce1<false>, g, t, 0, c->stream, (const Partial<float> *)c->partials, map,
                            (Partial<float> *)c->partials + c->part2Off);
     profile_end(c, "reduce");
 }
