@@ -804,16 +804,27 @@ static void enqueue_steps(sgk_ctx *c, const std::string &flags) {
         fold[k] = fuse[k] && !((flags[k] - 'a') & ~8) && c->stateAlt && c->partVmax;  // 8 takes no sums
         nFold += fold[k];
     }
+    // A step that only a shear or the next insertion follows is closed by the next k_lf1 (k_lf1_next).
+    std::vector<char> lf1(n, 0);
+    for (size_t k = 0; k + 1 < n; ++k) {
+        const int b = flags[k] - 'a';
+        if (fold[k] || !c->stateAlt || !c->partVmax || c->dp.nMolMe == 0 || part_map(c).count() > kCloseLf1Parts) continue;
+        lf1[k] = c->dp.iRegime == 1 ? b == 0 : b == 2;
+        fold[k] = lf1[k];
+        nFold += fold[k];
+    }
     for (size_t k = 0; (nFold & 1) && k < n; ++k)
         if (fold[k]) {
-            fold[k] = 0;
+            fold[k] = lf1[k] = 0;
             break;
         }
-    bool kicked = false, drifted = false, folded = false;
+    bool kicked = false, drifted = false, folded = false, next = false;
     for (size_t k = 0; k < n; ++k) {
         const int b = flags[k] - 'a';
-        sgk::launch_insert(c);  // regime 1 only
-        if (folded)
+        if (!next) sgk::launch_insert(c);  // regime 1 only
+        if (next)
+            sgk::launch_lf1_next(c, c->dp.iRegime == 2);
+        else if (folded)
             sgk::launch_bin_next(c);
         else if (drifted)
             sgk::launch_bin(c, false);
@@ -827,8 +838,9 @@ static void enqueue_steps(sgk_ctx *c, const std::string &flags) {
         kicked = pre[k];
         drifted = fuse[k];
         folded = fold[k];
+        next = lf1[k];
         if (b & 1) sgk::launch_thermostat(c, 0, 0.0, 0);
-        if (b & 2) sgk::launch_shear(c);
+        if ((b & 2) && !next) sgk::launch_shear(c);
         // the samples below read this step's positions, still in pos
         if (b & 4) sgk::launch_rdf(c);
         if (b & 16) sgk::launch_diffuse(c);

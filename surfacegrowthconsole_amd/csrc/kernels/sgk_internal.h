@@ -133,6 +133,11 @@ inline int metal_blocks(long long nMe, int G, int xcdMap) {
     return (int)((xcdMap & 6) ? (nb + 7) / 8 * 8 : nb);
 }
 
+// Most partials of a step that k_lf1_next closes (kSumParts: it takes no chunk totals).  Each of its
+// workgroups reads them all, and that still costs less than the launches it replaces: whole step
+// without / with it (us), sheared FP32 9,417 atoms 24.8 / 21.5, 47,776 36.0 / 32.6, 119,200 43.7 / 42.0,
+// mixed 119,200 53.8 / 53.2; deposition 17,196 24.1 / 19.0, 205,100 67.9 / 53.0.
+constexpr int kCloseLf1Parts = 1024;
 // The force pass's partials of a step.
 inline sgk::PartMap part_map(const sgk_ctx *c) { return {c->nbM, c->nbM + c->nbC, c->carbonLanes == 4}; }
 
@@ -262,6 +267,7 @@ void launch_force(sgk_ctx *c, bool integrate, bool finalize, bool prekick = fals
 // sgk_step.hip
 void launch_lf1(sgk_ctx *c, bool bin, bool kicked = false);
 void launch_insert(sgk_ctx *c);
+void launch_lf1_next(sgk_ctx *c, bool shear);  // with the closing of a folded step (regime 1: and the insertion)
 // drifted: the previous force pass drifted the positions (posOut), so only the binning is left.
 void launch_batch_lf1(sgk_batch *b, bool kicked = false, bool drifted = false);
 void launch_batch_finalize(sgk_batch *b);

@@ -102,26 +102,8 @@ __global__ __launch_bounds__(256) void k_bin_next(DevParams p, const typename Pr
                                                   CellBufs bufs, const typename Prec<M>::A *__restrict__ vmax, int n,
                                                   int stride, const DevState *old, DevState *st) {
     using A = typename Prec<M>::A;
-    __shared__ A sh[4];
-    A v = A(0);
-    for (int k = threadIdx.x; k < n; k += 256) v = OpMax::f(v, vmax[(size_t)k * stride]);
-    v = wave_reduce63<OpMax>(v);
-    if ((threadIdx.x & 63) == 63) sh[threadIdx.x >> 6] = v;
-    __syncthreads();
-    v = OpMax::f(OpMax::f(sh[0], sh[1]), OpMax::f(sh[2], sh[3]));
-    const StepNext<A> s = step_next(p, old, v);
-    if (blockIdx.x == 0 && threadIdx.x == 0) {  // all but errors, which this launch's binning may raise
-        st->step = s.step;
-        st->nebrNow = s.nebrNow;
-        st->cellbuf = s.cellbuf;
-        st->rec = old->rec + 1;
-        st->rebuilds = s.rebuilds;
-        st->dispHi = s.dispHi;
-        st->shear = old->shear;
-        st->shearCount = old->shearCount;
-        st->nMolDeposited = old->nMolDeposited;
-        st->errPrev = old->errPrev | old->errors | (s.displaced ? SGK_FLAG_DISPLACEMENT : 0);
-    }
+    const StepNext<A> s = step_next(p, old, block_max(vmax, n, stride));
+    if (blockIdx.x == 0 && threadIdx.x == 0) advance_state(st, old, s, old->shear, old->nMolDeposited);
     if (!s.nebrNow) return;
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= p.nMol) return;

@@ -423,6 +423,21 @@ __device__ __forceinline__ void record_sums(const DevParams &p, const Partial<A>
     rec.pad = 0;
 }
 
+// The shear increment after step `step` (SurfaceGrowth.cu:2398-2404) and the atoms deposited by then (the
+// step's group counts from now on, SurfaceGrowth.cu:2148-2168).
+template <class A>
+__device__ __forceinline__ double shear_next(const DevParams &p, int step, double shear, A cmVelX) {
+    if (p.iRegime == 2 && p.nMolMe && step > p.stepEquil + p.stepCool && (float)cmVelX < 0.005f)
+        shear = (double)((A)shear + (A)p.deltaF);
+    return shear;
+}
+__device__ __forceinline__ int deposited_next(const DevParams &p, int step, int deposited) {
+    if (p.iRegime == 1 && step > p.stepEquil && deposited < p.nMolMe && p.stepDeposit > 0 &&
+        (step - p.stepEquil) % p.stepDeposit == 0)
+        deposited += p.nMolToDeposit;
+    return deposited;
+}
+
 // Reduce the map's partials (totals: chunk totals) with the whole workgroup of 256, then evaluate the
 // reference's host arithmetic of SurfaceGrowth.cu:2307-2395 in thread 0.
 // mode 0: one step - advance the step counter, commit a rebuild, update dispHi / nebrNow / shear,
@@ -449,16 +464,8 @@ __device__ void finalize_body(const DevParams &p, const Partial<A> *part, const 
     }
     const StepNext<A> n = step_next(p, &s0, P.vmax);
     const int step = n.step, errors = s0.errors | (n.displaced ? SGK_FLAG_DISPLACEMENT : 0);
-    double shear = s0.shear;
-    int deposited = s0.nMolDeposited;
-    // shear increment (SurfaceGrowth.cu:2398-2404)
-    if (p.iRegime == 2 && nMe && step > p.stepEquil + p.stepCool) {
-        if ((float)cmVelX < 0.005f) shear = (double)((A)shear + (A)p.deltaF);
-    }
-    // deposition schedule (SurfaceGrowth.cu:2148-2168): the step's group counts from now on
-    if (p.iRegime == 1 && step > p.stepEquil && deposited < nMe && p.stepDeposit > 0 &&
-        (step - p.stepEquil) % p.stepDeposit == 0)
-        deposited += p.nMolToDeposit;
+    const double shear = shear_next(p, step, s0.shear, cmVelX);
+    const int deposited = deposited_next(p, step, s0.nMolDeposited);
     st->step = step;
     st->cellbuf = n.cellbuf;
     st->rebuilds = n.rebuilds;
@@ -495,6 +502,36 @@ __device__ void finalize_body(const DevParams &p, const Partial<A> *part, const 
 // of maxima and the closing workgroup's rows would outlast the force launch.
 constexpr int kCloseDirectParts = kSumParts;
 
+// A step that only a shear or a deposition follows closes the same way: k_lf1_next (sgk_step.hip) takes the
+// place of k_bin_next, up to kCloseLf1Parts partials.
+
+// The advanced state, all but errors, which the launch's binning may raise.
+template <class A>
+__device__ __forceinline__ void advance_state(DevState *st, const DevState *old, const StepNext<A> &s, double shear,
+                                              int deposited) {
+    st->step = s.step;
+    st->nebrNow = s.nebrNow;
+    st->cellbuf = s.cellbuf;
+    st->rec = old->rec + 1;
+    st->rebuilds = s.rebuilds;
+    st->dispHi = s.dispHi;
+    st->shear = shear;
+    st->nMolDeposited = deposited;
+    st->errPrev = old->errPrev | old->errors | (s.displaced ? SGK_FLAG_DISPLACEMENT : 0);
+}
+
+// Maximum of n values v[0], v[stride], ... by one workgroup of 256 threads, returned to every thread.
+template <class A>
+__device__ __forceinline__ A block_max(const A *__restrict__ v, int n, int stride) {
+    __shared__ A sh[4];
+    A m = A(0);
+    for (int k = threadIdx.x; k < n; k += 256) m = OpMax::f(m, v[(size_t)k * stride]);
+    m = wave_reduce63<OpMax>(m);
+    if ((threadIdx.x & 63) == 63) sh[threadIdx.x >> 6] = m;
+    __syncthreads();
+    return OpMax::f(OpMax::f(sh[0], sh[1]), OpMax::f(sh[2], sh[3]));
+}
+
 template <class A>
 struct StepClose {
     const Partial<A> *part;  // force-pass partials, or chunk totals (direct = 0)
@@ -519,14 +556,16 @@ __device__ __forceinline__ void close_body(const DevParams &p, const StepClose<A
     rec.nebrNow = c.st->nebrNow;
     rec.errors = c.st->errPrev;
     rec.dispHi = c.st->dispHi;
-    rec.shear = c.old->shear;
-    rec.nMolDeposited = c.old->nMolDeposited;
+    rec.shear = c.st->shear;
+    rec.shearCount = (double)c.old->shearCount;
+    rec.nMolDeposited = c.st->nMolDeposited;
     const int slot = c.old->rec;
     if (slot < c.recCap) c.records[slot] = rec;
     c.st->vvSum = (double)vvSum;
     c.st->cmVelX = (double)cmVelX;
     c.st->comX = p.nMolMe ? (double)(P.com[0] / (A)p.nMolMe) : 0.0;
     c.old->errors = 0;  // taken over into errPrev; this state is the next advance's target
+    c.old->shearCount = 0u;
 }
 
 }  // namespace sgk

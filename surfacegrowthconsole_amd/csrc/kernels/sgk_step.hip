@@ -99,20 +99,17 @@ __global__ __launch_bounds__(256) void kb_lf1(BatchArgs a, int kicked, int syncN
                 rep_cells(a, B), st, 1, kicked, rebuild, drifted);
 }
 
-// InsertAtomsK (SurfaceGrowth.cu:488-514) with the schedule of .cu:2148-2168, for the step about to
-// run (st->step + 1): metal atoms of this step's group are placed at z = 0.49 Lz moving down at
-// velMagDepos; atoms not yet due are parked above the box at rest (outside every cell).
+// InsertAtomsK (SurfaceGrowth.cu:488-514) with the schedule of .cu:2148-2168, for the step `next` about
+// to run with dep atoms deposited: metal atoms of this step's group are placed at z = 0.49 Lz moving
+// down at velMagDepos; atoms not yet due are parked above the box at rest (outside every cell).
 template <bool M>
-__global__ __launch_bounds__(256) void k_insert(DevParams p, typename Prec<M>::P4 *__restrict__ pos,
-                                                typename Prec<M>::R *__restrict__ vel, const DevState *st) {
+__device__ __forceinline__ void insert_atom(const DevParams &p, int n, int next, int dep,
+                                            typename Prec<M>::P4 *pos, typename Prec<M>::R *vel) {
     using R = typename Prec<M>::R;
-    const int n = blockIdx.x * blockDim.x + threadIdx.x;
-    if (n >= p.nMolMe) return;
-    const int step = st->step + 1, dep = st->nMolDeposited;
     int toDeposit = 0;
-    if (step > p.stepEquil) {
+    if (next > p.stepEquil) {
         if (dep >= p.nMolMe) return;
-        if (p.stepDeposit > 0 && (step - p.stepEquil) % p.stepDeposit == 0) toDeposit = p.nMolToDeposit;
+        if (p.stepDeposit > 0 && (next - p.stepEquil) % p.stepDeposit == 0) toDeposit = p.nMolToDeposit;
     }
     const int interval = dep + toDeposit;
     if (n >= dep && n < interval) {
@@ -124,6 +121,76 @@ __global__ __launch_bounds__(256) void k_insert(DevParams p, typename Prec<M>::P
         vel[n] = R(0);
         vel[p.nMol + n] = R(0);
         vel[2 * p.nMol + n] = R(0);
+    }
+}
+
+template <bool M>
+__global__ __launch_bounds__(256) void k_insert(DevParams p, typename Prec<M>::P4 *__restrict__ pos,
+                                                typename Prec<M>::R *__restrict__ vel, const DevState *st) {
+    const int n = blockIdx.x * blockDim.x + threadIdx.x;
+    if (n < p.nMolMe) insert_atom<M>(p, n, st->step + 1, st->nMolDeposited, pos, vel);
+}
+
+// k_lf1 of a step whose predecessor has no closing launches of its own although a shear or a deposition
+// stands between them (StepClose, sgk_reduce.h): every workgroup takes what these need of the closed
+// step - its v^2 maximum, and for the shear its sums - advances the state (the first workgroup stores it),
+// shears or inserts its atoms, then kicks, drifts and bins them.  One launch in place of k_finalize,
+// k_shear or k_insert, and k_lf1, each of which waited for the one before: a sheared step of 1,175 atoms
+// (FP32) 22.9 -> 20.1 us, a deposition step of 4,883 21.7 -> 17.2.
+template <bool M>
+__global__ __launch_bounds__(256) void k_lf1_next(DevParams p, typename Prec<M>::P4 *__restrict__ pos,
+                                                  typename Prec<M>::R *__restrict__ vel,
+                                                  const typename Prec<M>::R *__restrict__ acc, CellBufs bufs,
+                                                  const Partial<typename Prec<M>::A> *__restrict__ part, PartMap map,
+                                                  const typename Prec<M>::A *__restrict__ vmax, DevState *old,
+                                                  DevState *st, int shear) {
+#pragma clang fp contract(off)
+    using R = typename Prec<M>::R;
+    using A = typename Prec<M>::A;
+    const int n = blockIdx.x * blockDim.x + threadIdx.x;
+    A vm, comX = A(0);
+    double inc = old->shear;
+    if (shear) {
+        const Partial<A> P = sum_parts(part, map, false);
+        vm = P.vmax;
+        comX = P.com[0] / (A)p.nMolMe;
+        const A cmVelX = P.cmv[0] / (A)p.nMolMe;
+        inc = shear_next(p, old->step + 1, inc, cmVelX);
+    } else {
+        vm = block_max(vmax, map.stored, 1);
+    }
+    const StepNext<A> s = step_next(p, old, vm);
+    const int deposited = deposited_next(p, s.step, old->nMolDeposited);
+    if (n == 0) advance_state(st, old, s, inc, deposited);
+    const bool metal = n < p.nMolMe;
+    int hit = 0;
+    if (n < p.nMol) {
+        if (p.iRegime == 1 && metal) insert_atom<M>(p, n, s.step + 1, deposited, pos, vel);
+        auto r = pos[n];
+        bool move = true;
+        if (!metal) move = r.x != (R)p.xLeft && r.x < (R)p.xRight && r.y != (R)p.yTop && r.y != (R)p.yBottom;
+        R vx = R(0), vy = R(0), vz = R(0);
+        R ax = acc[n];
+        if (shear && metal && (float)(double)comX - (float)r.x > 0.f) {  // shear_body
+            ax += (R)inc;
+            hit = 1;
+        }
+        if (move) {
+            const R hdt = (R)(0.5f * p.deltaT);
+            vx = vel[n] + hdt * ax;
+            vy = vel[p.nMol + n] + hdt * acc[p.nMol + n];
+            vz = vel[2 * p.nMol + n] + hdt * acc[2 * p.nMol + n];
+            vel[n] = vx;
+            vel[p.nMol + n] = vy;
+            vel[2 * p.nMol + n] = vz;
+        }
+        drift_wrap<R>(p, r, move, vx, vy, vz);
+        pos[n] = r;
+        if (s.nebrNow) bin_atom(p, n, make_float3((float)r.x, (float)r.y, (float)r.z), bufs, s.cellbuf ^ 1, &st->errors);
+    }
+    if (shear) {
+        const int cnt = __syncthreads_count(hit);
+        if (threadIdx.x == 0 && cnt) atomicAdd(&old->shearCount, (unsigned)cnt);
     }
 }
 
@@ -413,6 +480,22 @@ void launch_lf1(sgk_ctx *c, bool bin, bool kicked) {
     else
         hipLaunchKernelGGL(k_lf1<false>, dim3(g), dim3(256), 0, c->stream, c->dp, (float4 *)c->pos, (float *)c->vel,
                            (const float *)c->acc, cell_bufs(c), c->state, (int)bin, (int)kicked);
+    profile_end(c, "lf1");
+}
+
+void launch_lf1_next(sgk_ctx *c, bool shear) {
+    static_assert(kCloseLf1Parts <= kSumParts, "sum_parts takes the partials directly");
+    profile_begin(c);
+    const unsigned g = blocks_for(c->dp.nMol, 256);
+    const PartMap map = part_map(c);
+    if (c->mixed)
+        hipLaunchKernelGGL(k_lf1_next<true>, dim3(g), dim3(256), 0, c->stream, c->dp, (double4 *)c->pos, (double *)c->vel,
+                           (const double *)c->acc, cell_bufs(c), (const Partial<double> *)c->partialsAlt, map,
+                           (const double *)c->partVmaxAlt, c->stateAlt, c->state, (int)shear);
+    else
+        hipLaunchKernelGGL(k_lf1_next<false>, dim3(g), dim3(256), 0, c->stream, c->dp, (float4 *)c->pos, (float *)c->vel,
+                           (const float *)c->acc, cell_bufs(c), (const Partial<float> *)c->partialsAlt, map,
+                           (const float *)c->partVmaxAlt, c->stateAlt, c->state, (int)shear);
     profile_end(c, "lf1");
 }
 
