@@ -45,8 +45,9 @@ struct BatchArgs {
     int *nlM, *nnM, *nlj, *ncl;
     unsigned *lj, *cl;
     uint4 *bondC, *bondA;
-    void *partials;
-    DevState *state;
+    void *partials, *partialsOld;           // Old: of the step that this one closes (a folded step)
+    DevState *state, *stateOld;
+    unsigned long long *vmax, *vmaxOld;     // per replica, the step's v^2 maximum (bits of a double >= 0)
     sgk_record *records;
     int recCap;
     unsigned *hist;

@@ -105,27 +105,43 @@ void enqueue_batch(sgk_batch *b, const std::string &flags) {
         pre[s] = !((flags[s] - 'a') & 3) && s + 1 < n;
         nPre += pre[s];
     }
+    // and a fused step with no sample behind it is closed by the next step's kernels, an even number again
     bool unfuseFirst = (nPre & 1) != 0;
-    bool kicked = false, drifted = false;
+    std::vector<char> fuse(n, 0), fold(n, 0);
+    int nFold = 0;
+    for (size_t s = 0; s < n; ++s) {
+        if (!pre[s] || !b->posAlt) continue;
+        fuse[s] = !unfuseFirst;
+        unfuseFirst = false;
+        fold[s] = fuse[s] && flags[s] == 'a' && b->canFold;
+        nFold += fold[s];
+    }
+    for (size_t s = 0; (nFold & 1) && s < n; ++s)
+        if (fold[s]) {
+            fold[s] = 0;
+            break;
+        }
+    bool kicked = false, drifted = false, folded = false;
     for (size_t s = 0; s < n; ++s) {
         const int k = flags[s] - 'a';
-        bool fuse = false;
-        if (pre[s] && b->posAlt) {
-            fuse = !unfuseFirst;
-            unfuseFirst = false;
-        }
-        sgk::launch_batch_lf1(b, kicked, drifted);
+        sgk::launch_batch_lf1(b, kicked, drifted, folded);
         sgk::launch_batch_sortcells(b);
         sgk::launch_batch_nl(b);
         sgk::launch_batch_rho(b);
-        sgk::launch_batch_force(b, pre[s], fuse ? b->posAlt : nullptr);
-        sgk::launch_batch_finalize(b);
+        sgk::launch_batch_force(b, pre[s], fuse[s] ? b->posAlt : nullptr, folded);
+        if (!fold[s]) sgk::launch_batch_finalize(b);
         kicked = pre[s];
-        drifted = fuse;
+        drifted = fuse[s];
+        folded = fold[s];
         if (k & 1) sgk::launch_batch_thermostat(b);
         if (k & 2) sgk::launch_batch_shear(b);
         if (k & 4) sgk::launch_batch_rdf(b);  // this step's positions, still in pos
-        if (fuse) std::swap(b->pos, b->posAlt);
+        if (fuse[s]) std::swap(b->pos, b->posAlt);
+        if (fold[s]) {
+            std::swap(b->state, b->stateAlt);
+            std::swap(b->partials, b->partialsAlt);
+            std::swap(b->vmax, b->vmaxAlt);
+        }
     }
 }
 
@@ -138,12 +154,14 @@ int default_lanes(int nMe) { return nMe >= 65536 ? 4 : nMe >= 2048 ? 8 : 16; }
 std::vector<int2> force_layout(sgk_batch *b) {
     std::vector<std::vector<int2>> groups(sgk_batch::kLaneKinds);
     int partOff = 0;
+    b->canFold = true;
     for (int r = 0; r < b->nrep; ++r) {
         BatchRep &R = b->reps[r];
         const int G = b->repLanes[r];
         R.nbM = metal_blocks(R.p.nMolMe, G, 0);  // the batch remaps nothing
         R.nbForce = R.nbM + sgk::carbon_blocks(R.p.nC, R.carbonLanes);
         R.partOff = partOff;
+        b->canFold &= (sgk::PartMap{R.nbM, R.nbForce, R.carbonLanes == 4}.count() <= sgk::kFoldParts);
         R.nChunks = (sgk::PartMap{R.nbM, R.nbForce, R.carbonLanes == 4}.count() + 63) / 64;  // kPartChunk partials per chunk
         partOff += R.nbForce;
         auto &g = groups[sgk::batch_lane_index(G)];
@@ -374,7 +392,11 @@ int sgk_batch_create(int nrep, const SimParams *params, const sgk_config *cfgIn,
     BTRY(balloc(b, &b->bondC, (size_t)carbonOff, true));
     BTRY(balloc(b, &b->bondA, (size_t)carbonOff, true));
     BTRY(balloc(b, (char **)&b->partials, partCap * sgk::partial_bytes_for(b->mixed), true));
+    BTRY(balloc(b, (char **)&b->partialsAlt, partCap * sgk::partial_bytes_for(b->mixed), true));
+    BTRY(balloc(b, &b->vmax, (size_t)nrep, true));
+    BTRY(balloc(b, &b->vmaxAlt, (size_t)nrep, true));
     BTRY(balloc(b, &b->state, (size_t)nrep, true));
+    BTRY(balloc(b, &b->stateAlt, (size_t)nrep, true));
     BTRY(balloc(b, &b->records, (size_t)nrep * cfg.records_capacity, true));
     BTRY(balloc(b, &b->hist, (size_t)nrep * s0.sizeHistRdf, true));
     BTRY(hipMemcpyAsync(b->dReps, b->reps.data(), sizeof(BatchRep) * nrep, hipMemcpyHostToDevice, b->stream) == hipSuccess

@@ -908,24 +908,25 @@ __device__ __forceinline__ void force_block(bool quad, const DevParams &p, int b
                                             float *__restrict__ fric, const unsigned *__restrict__ lj,
                                             const int *__restrict__ nlj, const uint4 *__restrict__ bondC,
                                             const uint4 *__restrict__ bondA, Partial<typename Prec<M>::A> *part,
-                                            typename Prec<M>::A *vmax, int integrate) {
+                                            typename Prec<M>::A *vmax, unsigned long long *vmaxAll, int integrate) {
     using A = typename Prec<M>::A;
     // Each branch reduces and stores on its own: a Partial merged across the two branches keeps
     // both bodies' registers live at once (154 VGPRs in the FP64 form against 120 apart).
     if (b < nbM) {
         const Partial<A> q = metal_body<M, T, G>(p, xm ? xcd_block(b, nbM) : b, pos, posOut, vel, acc, nlM, nnM, embF,
                                                  embDF, fric, integrate);
-        if (integrate) block_store_partial<true, G>(q, part + b, vmax ? vmax + b : nullptr);
+        if (integrate) block_store_partial<true, G>(q, part + b, vmax ? vmax + b : nullptr, vmaxAll);
     } else {
         if (quad) {
             const QuadBlock at = quad_block(b - nbM, p.nC, xm);
             if (at.slot < 0) return;
             const Partial<A> q = carbon4_body<M, T>(p, at.blk, pos, posOut, vel, acc, lj, nlj, bondC, bondA, integrate);
-            if (integrate) block_store_quad(q, part + nbM + at.slot, vmax ? vmax + nbM + at.slot : nullptr);
+            if (integrate)
+                block_store_quad(q, part + nbM + at.slot, vmax ? vmax + nbM + at.slot : nullptr, vmaxAll);
         } else {
             const Partial<A> q = carbon_body<M, T>(p, xm ? xcd_block(b - nbM, nb - nbM) : b - nbM, pos, posOut, vel, acc,
                                                    lj, nlj, bondC, bondA, integrate);
-            if (integrate) block_store_partial<false, 1>(q, part + b, vmax ? vmax + b : nullptr);
+            if (integrate) block_store_partial<false, 1>(q, part + b, vmax ? vmax + b : nullptr, vmaxAll);
         }
     }
 }
@@ -950,15 +951,32 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     }
     // nbM is a multiple of 8: both ranges keep the XCD of each block
     force_block<M, T, G>(CL == 4, p, blockIdx.x - first, nbM, gridDim.x - first, p.xcdMap & 4, pos, posOut, vel, acc, nlM, nnM, embF, embDF,
-                         fric, lj, nlj, bondC, bondA, part, vmax, integrate);
+                         fric, lj, nlj, bondC, bondA, part, vmax, nullptr, integrate);
 }
 
-// Batched: each replica's workgroups write into its own range of partials (kb_finalize reduces).
+// Batched: each replica's workgroups write into its own range of partials.  With a step to close, the first
+// nClose workgroups close one replica's each.
 template <bool M, class T, int G>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void kb_force(BatchArgs a, int integrate) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void kb_force(BatchArgs a, int nClose, int integrate) {
     using R = typename Prec<M>::R;
     using A = typename Prec<M>::A;
-    const int2 e = a.forceTab[blockIdx.x];
+    if ((int)blockIdx.x < nClose) {
+        const int r = blockIdx.x;
+        const BatchRep &B = a.reps[r];
+        StepClose<A> c;
+        c.part = (const Partial<A> *)a.partialsOld + B.partOff;
+        c.map = {B.nbM, B.nbForce, B.carbonLanes == 4};
+        c.direct = 1;
+        c.old = a.stateOld + r;
+        c.st = a.state + r;
+        c.records = a.records + (size_t)r * a.recCap;
+        c.recCap = a.recCap;
+        c.on = 1;
+        close_body(B.p, c);
+        if (threadIdx.x == 0) a.vmaxOld[r] = 0ull;
+        return;
+    }
+    const int2 e = a.forceTab[blockIdx.x - nClose];
     const BatchRep &B = a.reps[e.x];
     const DevParams &p = B.p;
     force_block<M, T, G>(B.carbonLanes == 4, p, e.y, B.nbM, B.nbForce, false, (typename Prec<M>::P4 *)a.pos + B.atomOff,
@@ -966,7 +984,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
                          (R *)a.vel + 3 * B.atomOff, (R *)a.acc + 3 * B.atomOff, a.nlM + B.metalOff * p.nlCap,
                          a.nnM + B.metalOff, a.embF + B.metalOff, a.embDF + B.metalOff, a.fric + B.metalOff,
                          a.lj + B.carbonOff * p.ljCap, a.nlj + B.carbonOff, a.bondC + B.carbonOff,
-                         a.bondA + B.carbonOff, (Partial<A> *)a.partials + B.partOff, nullptr, integrate);
+                         a.bondA + B.carbonOff, (Partial<A> *)a.partials + B.partOff, nullptr, a.vmax + e.x, integrate);
 }
 
 // ---- launchers ---------------------------------------------------------------------------------
@@ -1048,18 +1066,19 @@ int batch_lane_index(int G) { return G == 1 ? 0 : G == 2 ? 1 : G == 4 ? 2 : G ==
 // One launch per lane count present: the replicas with G lanes per metal atom, through their own
 // block table (the kernel body is templated on G).
 template <bool M, class T>
-static void batch_dispatch(sgk_batch *b, bool force, int integrate, void *posOut) {
+static void batch_dispatch(sgk_batch *b, bool force, int integrate, void *posOut, bool closePrev) {
+    int nClose = closePrev ? b->nrep : 0;  // in the first launch
     static const int kinds[sgk_batch::kLaneKinds] = {1, 2, 4, 8, 16};
     for (int q = 0; q < sgk_batch::kLaneKinds; ++q) {
         if (b->grpN[q] == 0) continue;
         BatchArgs a = b->args();
         a.posOut = posOut;
         a.forceTab = b->forceTab + b->grpOff[q];
-        const dim3 g(b->grpN[q]), t(256);
+        const dim3 g((force ? nClose : 0) + b->grpN[q]), t(256);
 #define SGK_B(GG)                                                                            \
     do {                                                                                     \
         if (force)                                                                           \
-            hipLaunchKernelGGL((kb_force<M, T, GG>), g, t, 0, b->stream, a, integrate);     \
+            hipLaunchKernelGGL((kb_force<M, T, GG>), g, t, 0, b->stream, a, nClose, integrate); \
         else                                                                                 \
             hipLaunchKernelGGL((kb_rho<M, T, GG>), g, t, 0, b->stream, a);                  \
     } while (0)
@@ -1071,22 +1090,25 @@ static void batch_dispatch(sgk_batch *b, bool force, int integrate, void *posOut
             default: SGK_B(8); break;
         }
 #undef SGK_B
+        nClose = 0;
     }
 }
 
-static void batch_launch(sgk_batch *b, bool force, int integrate, void *posOut = nullptr) {
+static void batch_launch(sgk_batch *b, bool force, int integrate, void *posOut = nullptr, bool closePrev = false) {
     if (b->nForceBlocks == 0) return;
     if (integrate != 2) posOut = nullptr;  // the drift follows the next step's half-kick only
     if (!b->mixed)
-        batch_dispatch<false, float>(b, force, integrate, posOut);
+        batch_dispatch<false, float>(b, force, integrate, posOut, closePrev);
     else if (b->cfg.pair_fp64)
-        batch_dispatch<true, double>(b, force, integrate, posOut);
+        batch_dispatch<true, double>(b, force, integrate, posOut, closePrev);
     else
-        batch_dispatch<true, float>(b, force, integrate, posOut);
+        batch_dispatch<true, float>(b, force, integrate, posOut, closePrev);
 }
 
 void launch_batch_rho(sgk_batch *b) { batch_launch(b, false, 0); }
-void launch_batch_force(sgk_batch *b, bool prekick, void *posOut) { batch_launch(b, true, prekick ? 2 : 1, posOut); }
+void launch_batch_force(sgk_batch *b, bool prekick, void *posOut, bool closePrev) {
+    batch_launch(b, true, prekick ? 2 : 1, posOut, closePrev);
+}
 void launch_batch_force_eval(sgk_batch *b) { batch_launch(b, true, 0); }
 
 void launch_force(sgk_ctx *c, bool integrate, bool finalize, bool prekick, void *posOut, bool closePrev) {

@@ -133,11 +133,11 @@ inline int metal_blocks(long long nMe, int G, int xcdMap) {
     return (int)((xcdMap & 6) ? (nb + 7) / 8 * 8 : nb);
 }
 
-// Most partials of a step that k_lf1_next closes (kSumParts: it takes no chunk totals).  Each of its
+// Most partials of a step that k_lf1_next closes (it takes no chunk totals).  Each of its
 // workgroups reads them all, and that still costs less than the launches it replaces: whole step
 // without / with it (us), sheared FP32 9,417 atoms 24.8 / 21.5, 47,776 36.0 / 32.6, 119,200 43.7 / 42.0,
 // mixed 119,200 53.8 / 53.2; deposition 17,196 24.1 / 19.0, 205,100 67.9 / 53.0.
-constexpr int kCloseLf1Parts = 1024;
+constexpr int kCloseLf1Parts = sgk::kFoldParts;
 // The force pass's partials of a step.
 inline sgk::PartMap part_map(const sgk_ctx *c) { return {c->nbM, c->nbM + c->nbC, c->carbonLanes == 4}; }
 
@@ -173,8 +173,10 @@ struct sgk_batch {
     int *nlM = nullptr, *nnM = nullptr, *nlj = nullptr, *ncl = nullptr;
     unsigned int *lj = nullptr, *cl = nullptr;
     uint4 *bondC = nullptr, *bondA = nullptr;
-    void *partials = nullptr;
-    sgk::DevState *state = nullptr;
+    void *partials = nullptr, *partialsAlt = nullptr;  // the Alt ones swapped inside a chunk of steps, as in sgk_ctx
+    sgk::DevState *state = nullptr, *stateAlt = nullptr;
+    unsigned long long *vmax = nullptr, *vmaxAlt = nullptr;
+    bool canFold = false;                // every replica's partials can be closed by the next step's kernels
     sgk_record *records = nullptr;
     unsigned int *hist = nullptr;
     sgk::DevState *hostState = nullptr;  // pinned mirror, nrep entries
@@ -220,7 +222,11 @@ struct sgk_batch {
         a.bondC = bondC;
         a.bondA = bondA;
         a.partials = partials;
+        a.partialsOld = partialsAlt;
         a.state = state;
+        a.stateOld = stateAlt;
+        a.vmax = vmax;
+        a.vmaxOld = vmaxAlt;
         a.records = records;
         a.recCap = cfg.records_capacity;
         a.hist = hist;
@@ -256,8 +262,8 @@ RdfGrid rdf_grid(const DevParams &p, int S);  // complete-range RDF grid, cells 
 void launch_rho(sgk_ctx *c);
 void launch_batch_rho(sgk_batch *b);
 int batch_lane_index(int G);  // position of G in the lane kinds 1, 2, 4, 8, 16
-void launch_batch_force(sgk_batch *b, bool prekick = false, void *posOut = nullptr);
-void launch_batch_force_eval(sgk_batch *b);  // forces, energies and partials only: velocities untouched
+void launch_batch_force(sgk_batch *b, bool prekick = false, void *posOut = nullptr, bool closePrev = false);
+void launch_batch_force_eval(sgk_batch *b);  // forces and energies only: velocities untouched
 // prekick: the force pass also applies the next step's first half-kick (the caller guarantees that
 // nothing touches velocities or accelerations before that step's launch_lf1(kicked = true)).
 // posOut (with prekick): also drift the positions of the next step into posOut (sgk_force.hip).
@@ -269,7 +275,7 @@ void launch_lf1(sgk_ctx *c, bool bin, bool kicked = false);
 void launch_insert(sgk_ctx *c);
 void launch_lf1_next(sgk_ctx *c, bool shear);  // with the closing of a folded step (regime 1: and the insertion)
 // drifted: the previous force pass drifted the positions (posOut), so only the binning is left.
-void launch_batch_lf1(sgk_batch *b, bool kicked = false, bool drifted = false);
+void launch_batch_lf1(sgk_batch *b, bool kicked = false, bool drifted = false, bool folded = false);
 void launch_batch_finalize(sgk_batch *b);
 void launch_batch_thermostat(sgk_batch *b);
 void launch_batch_shear(sgk_batch *b);

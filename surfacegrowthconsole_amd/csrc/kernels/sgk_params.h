@@ -76,6 +76,7 @@ struct PartMap {
     __device__ int parts(int k) const { return quad && k >= nbM ? 4 : 1; }
 };
 inline __host__ __device__ PartMap plain_map(int n) { return {n, n, 0}; }
+constexpr int kFoldParts = 1024;  // most partials that one workgroup closes without k_reduce1
 
 // Device-resident run state.  A context has two: a step whose closing is folded into the next step
 // leaves its state as it is, and the next step's first kernel writes the advanced state into the

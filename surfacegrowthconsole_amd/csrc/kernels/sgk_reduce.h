@@ -88,8 +88,17 @@ __device__ __forceinline__ T half_sum(bool hi, T a, T b) {
     return keep + dpp_all<CTRL>(give);
 }
 
+// A workgroup's v^2 maximum: into its place, or joined with a replica's others (as the bits of a double,
+// which order non-negative values; a NaN is left out, as OpMax leaves it).
+template <class T>
+__device__ __forceinline__ void store_vmax(T r, T *vmax, unsigned long long *vmaxAll) {
+    if (vmax) *vmax = r;
+    if (vmaxAll && r > T(0)) atomicMax(vmaxAll, (unsigned long long)__double_as_longlong((double)r));
+}
+
 template <bool METAL, int G, class T>
-__device__ __forceinline__ void block_store_partial(Partial<T> q, Partial<T> *out, T *vmax) {
+__device__ __forceinline__ void block_store_partial(Partial<T> q, Partial<T> *out, T *vmax,
+                                                    unsigned long long *vmaxAll) {
     static_assert(sizeof(Partial<T>) == kPartFields * sizeof(T), "fields of Partial in their order");
     __shared__ Partial<T> sh[4];
     __shared__ T row[4][4][8];
@@ -151,14 +160,14 @@ __device__ __forceinline__ void block_store_partial(Partial<T> q, Partial<T> *ou
         }
     }
     ((T *)out)[f] = r;
-    if (vmax && f == kPartVmax) *vmax = r;
+    if (f == kPartVmax) store_vmax(r, vmax, vmaxAll);
 }
 
 // The same sums for a workgroup with four lanes per carbon (64 carbons), each of which holds its carbon's
 // contribution: lane l of a quad takes two fields, the quads of a row of 16 lanes are summed in it and the
 // rows in LDS.  The tree is that of one wave of block_store_partial with a carbon per lane.
 template <class T>
-__device__ __forceinline__ void block_store_quad(Partial<T> q, Partial<T> *out, T *vmax) {
+__device__ __forceinline__ void block_store_quad(Partial<T> q, Partial<T> *out, T *vmax, unsigned long long *vmaxAll) {
     __shared__ T rows[16][8];
     const int l = threadIdx.x & 3, f = threadIdx.x;
     T a = q.vmax, b = q.vs[2];
@@ -196,7 +205,7 @@ __device__ __forceinline__ void block_store_quad(Partial<T> q, Partial<T> *out, 
         r = x[0];
     }
     ((T *)out)[f] = r;
-    if (vmax && f == kPartVmax) *vmax = r;
+    if (f == kPartVmax) store_vmax(r, vmax, vmaxAll);
 }
 
 // First stage of the step reduction: one wave reduces a chunk of up to kPartChunk partials (lane k
@@ -258,7 +267,7 @@ __device__ __forceinline__ StepNext<A> step_next(const DevParams &p, const DevSt
 // Otherwise at most kSumParts partials: chunks of 64, then the chunk totals as the first 16 lanes of a wave.
 // One launch for up to 1,024 partials in place of k_reduce1 and k_finalize: a sheared step of 997 atoms
 // (FP32) 29.1 -> 26.8 us, a deposition step of 4,393 27.2 -> 25.3, kb_finalize of 64 replicas 8.0 -> 6.5.
-constexpr int kSumFours = 64, kSumParts = 1024, kSumGroups = 256 / kPartFields;
+constexpr int kSumFours = 64, kSumParts = kFoldParts, kSumGroups = 256 / kPartFields;
 
 // One field of a tree: sums add, the others keep the larger value, minima with their sign turned.
 template <class A>
@@ -553,7 +562,7 @@ __device__ __forceinline__ void close_body(const DevParams &p, const StepClose<A
     record_sums(p, P, rec, cmVelX, vvSum);
     rec.step = c.st->step;
     rec.rebuilt = c.old->nebrNow;
-    rec.nebrNow = c.st->nebrNow;
+    rec.nebrNow = step_next(p, c.old, P.vmax).nebrNow;  // its own rule's: a batch may rebuild for another replica
     rec.errors = c.st->errPrev;
     rec.dispHi = c.st->dispHi;
     rec.shear = c.st->shear;

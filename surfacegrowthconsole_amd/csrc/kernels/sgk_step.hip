@@ -99,6 +99,38 @@ __global__ __launch_bounds__(256) void kb_lf1(BatchArgs a, int kicked, int syncN
                 rep_cells(a, B), st, 1, kicked, rebuild, drifted);
 }
 
+// Batched k_bin_next: the drifted step after a folded one (StepClose, sgk_reduce.h).  The replicas' v^2
+// maxima come joined from the force pass, so that a workgroup can also tell what every other replica's
+// rule asks for (syncN > 0).  Whole step with closing launches / folded (us): 8 replicas of 22,000 atoms together
+// (FP32) 26.6 / 24.0, 64 replicas of 413,000 107.5 / 103.4.
+template <bool M>
+__global__ __launch_bounds__(256) void kb_bin_next(BatchArgs a, int syncN) {
+    using A = typename Prec<M>::A;
+    const int2 e = a.atomTab[blockIdx.x];
+    const BatchRep &B = a.reps[e.x];
+    DevState *st = a.state + e.x;
+    const DevState *old = a.stateOld + e.x;
+    auto vmax = [&](int r) { return (A)__longlong_as_double((long long)a.vmaxOld[r]); };
+    StepNext<A> s = step_next(B.p, old, vmax(e.x));
+    if (syncN > 0) {
+        __shared__ int any;
+        if (threadIdx.x < 64) {
+            int f = 0;
+            for (int r = threadIdx.x; r < syncN; r += 64) f |= step_next(a.reps[r].p, a.stateOld + r, vmax(r)).nebrNow;
+            f = __any(f) ? 1 : 0;
+            if (threadIdx.x == 0) any = f;
+        }
+        __syncthreads();
+        s.nebrNow = any;
+    }
+    if (e.y == 0 && threadIdx.x == 0)
+        advance_state(st, old, s, old->shear, deposited_next(B.p, s.step, old->nMolDeposited));
+    const int n = e.y * 256 + threadIdx.x;
+    if (!s.nebrNow || n >= B.p.nMol) return;
+    const auto r = ((const typename Prec<M>::P4 *)a.pos + B.atomOff)[n];
+    bin_atom(B.p, n, make_float3((float)r.x, (float)r.y, (float)r.z), rep_cells(a, B), s.cellbuf ^ 1, &st->errors);
+}
+
 // InsertAtomsK (SurfaceGrowth.cu:488-514) with the schedule of .cu:2148-2168, for the step `next` about
 // to run with dep atoms deposited: metal atoms of this step's group are placed at z = 0.49 Lz moving
 // down at velMagDepos; atoms not yet due are parked above the box at rest (outside every cell).
@@ -290,6 +322,7 @@ __global__ __launch_bounds__(kFinalizeThreads) void kb_finalize(BatchArgs a) {
     }
     finalize_body<A>(B.p, part, map, totals, a.state + blockIdx.x,
                      a.records + (size_t)blockIdx.x * a.recCap, a.recCap, 0);
+    if (threadIdx.x == 0) a.vmax[blockIdx.x] = 0ull;
 }
 
 // ApplyBerendsenThermostat (SurfaceGrowth.cu:455-485), kinetic energy of all atoms.
@@ -621,8 +654,13 @@ void launch_diffuse_reset(sgk_ctx *c) {
 }
 
 // ---- batched launchers -----------------------------------------------------------------------
-void launch_batch_lf1(sgk_batch *b, bool kicked, bool drifted) {
+void launch_batch_lf1(sgk_batch *b, bool kicked, bool drifted, bool folded) {
     const int syncN = b->cfg.sync_rebuilds && b->nrep > 1 ? b->nrep : 0;
+    if (folded) {
+        hipLaunchKernelGGL((b->mixed ? kb_bin_next<true> : kb_bin_next<false>), dim3(b->nAtomBlocks), dim3(256), 0,
+                           b->stream, b->args(), syncN);
+        return;
+    }
     if (b->mixed)
         hipLaunchKernelGGL(kb_lf1<true>, dim3(b->nAtomBlocks), dim3(256), 0, b->stream, b->args(), (int)kicked, syncN,
                            (int)drifted);
