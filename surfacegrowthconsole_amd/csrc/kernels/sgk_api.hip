@@ -770,7 +770,7 @@ std::string sgk::step_flag_string(sgk_ctx *c, int step0, int nsteps, int rdfEver
     return f;
 }
 
-static void enqueue_steps(sgk_ctx *c, const std::string &flags) {
+void sgk::enqueue_steps(sgk_ctx *c, const std::string &flags, StepTrace *trace) {
     sgk::launch_reset_records(c);
     // The force pass of a step also applies the next step's first half-kick when nothing touches the
     // velocities or accelerations in between (no thermostat, shear or deposition) and the step is
@@ -798,7 +798,7 @@ static void enqueue_steps(sgk_ctx *c, const std::string &flags) {
     std::vector<char> fuse(n, 0), fold(n, 0);
     int nFold = 0;
     for (size_t k = 0; k < n; ++k) {
-        if (!pre[k] || !c->posAlt) continue;
+        if (!pre[k] || !(c->posAlt || trace)) continue;
         fuse[k] = !unfuse;
         unfuse = false;
         fold[k] = fuse[k] && !((flags[k] - 'a') & ~8) && c->stateAlt && c->partVmax;  // 8 takes no sums
@@ -821,6 +821,11 @@ static void enqueue_steps(sgk_ctx *c, const std::string &flags) {
     bool kicked = false, drifted = false, folded = false, next = false;
     for (size_t k = 0; k < n; ++k) {
         const int b = flags[k] - 'a';
+        if (trace && !drifted) {  // the drift of this step is made in place: in the step's own slot
+            if (hipMemcpyAsync(trace->slot(k), c->pos, trace->stride, hipMemcpyDeviceToDevice, c->stream) != hipSuccess)
+                trace->rc = SGK_E_HIP;
+            c->pos = trace->slot(k);
+        }
         if (!next) sgk::launch_insert(c);  // regime 1 only
         if (next)
             sgk::launch_lf1_next(c, c->dp.iRegime == 2);
@@ -833,8 +838,10 @@ static void enqueue_steps(sgk_ctx *c, const std::string &flags) {
         sgk::launch_sortcells(c, false);
         sgk::launch_nl(c, false);
         sgk::launch_rho(c);
-        sgk::launch_force(c, true, !fold[k], pre[k], fuse[k] ? c->posAlt : nullptr, folded);
+        void *const drift = !fuse[k] ? nullptr : trace ? trace->slot(k + 1) : c->posAlt;
+        sgk::launch_force(c, true, !fold[k], pre[k], drift, folded);
         if (fold[k]) sgk::launch_reduce_chunks(c);
+        if (trace && trace->after && trace->rc == 0) trace->rc = trace->after(k);
         kicked = pre[k];
         drifted = fuse[k];
         folded = fold[k];
@@ -845,7 +852,10 @@ static void enqueue_steps(sgk_ctx *c, const std::string &flags) {
         if (b & 4) sgk::launch_rdf(c);
         if (b & 16) sgk::launch_diffuse(c);
         if (b & 8) sgk::launch_adh_obs(c, c->adj->d.part, c->adj->d.adh + k);
-        if (fuse[k]) std::swap(c->pos, c->posAlt);
+        if (fuse[k] && trace)
+            c->pos = drift;
+        else if (fuse[k])
+            std::swap(c->pos, c->posAlt);
         if (fold[k]) {
             std::swap(c->state, c->stateAlt);
             std::swap(c->partials, c->partialsAlt);
@@ -884,7 +894,7 @@ static int step_graph(sgk_ctx *c, const std::string &flags, hipGraphExec_t *out)
         hipGraph_t graph = nullptr;
         SGK_HIP(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
         g_capturing = true;
-        enqueue_steps(c, flags);
+        sgk::enqueue_steps(c, flags);
         g_capturing = false;
         hipError_t e = hipStreamEndCapture(c->stream, &graph);
         if (e != hipSuccess) return hip_fail(c, e, "hipStreamEndCapture");
@@ -934,7 +944,7 @@ int sgk::run_steps(sgk_ctx *c, int nsteps, int rdfEvery, sgk_record *records, do
         if (rc != SGK_OK) return rc;
         SGK_HIP(c, hipGraphLaunch(exec, c->stream));
     } else {
-        enqueue_steps(c, flags);
+        sgk::enqueue_steps(c, flags);
     }
     SGK_HIP(c, hipGetLastError());
     SGK_HIP(c, hipEventRecord(c->ev1, c->stream));

@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <functional>
 #include <map>
 #include <string>
 #include <vector>
@@ -296,6 +297,17 @@ int check_device_flags(sgk_ctx *c);
 // One character per step, 'a' + bits: 1 thermostat, 2 shear, 4 RDF, 8 adhesion energy recorded,
 // 16 diffusion sample.
 std::string step_flag_string(sgk_ctx *c, int step0, int nsteps, int rdfEvery, bool observe);
+// Where the positions of the steps are kept: after step k they lie at slot(k), and stay there.  after(k) runs
+// when step k's force pass is enqueued, before its thermostat.
+struct StepTrace {
+    char *pos = nullptr;
+    size_t stride = 0;
+    std::function<int(size_t)> after;
+    int rc = 0;
+    char *slot(size_t k) const { return pos + stride * k; }
+};
+// Enqueues the steps of the flags; with a trace, c->pos ends on its last slot.
+void enqueue_steps(sgk_ctx *c, const std::string &flags, StepTrace *trace = nullptr);
 // sgk_run with, if adh is not null, the adhesion energy of every step copied to adh[nsteps].
 int run_steps(sgk_ctx *c, int nsteps, int rdfEvery, sgk_record *records, double *adh);
 // Destroy the cached step graphs (their launches carry grids, parameters and buffer addresses).
