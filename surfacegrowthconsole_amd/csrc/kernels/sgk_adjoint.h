@@ -74,7 +74,8 @@ void launch_adj_rho(sgk_ctx *c, const AdjDev &d);
 void launch_adj_force(sgk_ctx *c, const AdjDev &d, double wE);
 void launch_adj_rho2(sgk_ctx *c, const AdjDev &d);
 void launch_adj_therm(sgk_ctx *c, const AdjDev &d, const double *velPre, int step);
-void launch_adj_pre(sgk_ctx *c, const AdjDev &d, const double *velPre);
+// Step k's end (posK, or null) and the start of the step at the context's positions, with its densities.
+void launch_adj_turn(sgk_ctx *c, const AdjDev &d, const void *posK, const double *velPre);
 void launch_adj_post(sgk_ctx *c, const AdjDev &d);
 void launch_adj_lam0(sgk_ctx *c, const AdjDev &d);
 void launch_adj_add(sgk_ctx *c, const AdjDev &d);  // G = Rb + G

@@ -244,9 +244,9 @@ struct KeepPos {
     ~KeepPos() { c->pos = pos; }
 };
 
-void enqueue_vjp(sgk_ctx *c, const AdjDev &d, double wE) {
+void enqueue_vjp(sgk_ctx *c, const AdjDev &d, double wE, bool rho = true) {
     sgk::launch_rho(c);  // the bond and near lists of the current positions
-    sgk::launch_adj_rho(c, d);
+    if (rho) sgk::launch_adj_rho(c, d);
     sgk::launch_adj_force(c, d, wE);
     sgk::launch_adj_rho2(c, d);
 }
@@ -369,18 +369,24 @@ int sgk_adjoint_backward(sgk_ctx *c, const double *w, double *grad, double *dr0,
         sgk::launch_adj_cmp(c, d, next.pos, next.vel, next.acc);
         // the step transposes in reverse
         int cur = n ? ver[n - 1] : 0;
+        const void *done = nullptr;  // positions of a step whose end is still due
         for (int k = n - 1; k >= 0; --k) {
             if (ver[k] != cur) {
                 ADJ_TRY(copy_nl(c, ver[k] == 0 ? a->ck[s].nl : a->slots[ver[k] - 1], true));
                 cur = ver[k];
             }
-            c->pos = trace.slot(k);
             const double *vp = a->thermo[base + k] == '1' ? (const double *)((char *)a->velStore + 24 * N * k) : nullptr;
-            if (vp) sgk::launch_adj_therm(c, d, vp, a->step0 + base + k + 1);
-            sgk::launch_adj_pre(c, d, vp);
-            enqueue_vjp(c, d, wE);
-            sgk::launch_adj_post(c, d);
+            if (vp) {  // the thermostat's transpose needs the end of the step behind it
+                if (done) sgk::launch_adj_post(c, d);
+                done = nullptr;
+                sgk::launch_adj_therm(c, d, vp, a->step0 + base + k + 1);
+            }
+            c->pos = trace.slot(k);
+            sgk::launch_adj_turn(c, d, done, vp);
+            enqueue_vjp(c, d, wE, false);
+            done = c->pos;
         }
+        if (done) sgk::launch_adj_post(c, d);
         ADJ_HIP(c, hipGetLastError());
     }
     // the initial acceleration a_0 = a(r_0) with the list built at r_0
