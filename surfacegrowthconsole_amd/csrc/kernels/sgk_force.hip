@@ -13,8 +13,8 @@
 //   k_force  one launch: blocks [0, nbM) are the metal pass (G lanes per atom: EAM pairs + LJ with
 //            carbon), blocks [nbM, nbM + nbC) the carbon pass (one thread per atom, or four: bond, plane
 //            and angle terms from the close list + LJ with metal).  The epilogue writes acceleration,
-//            energy, friction, applies leapfrog part 2 and leaves one Partial per block; k_finalize
-//            (sgk_step.hip), the next launch, reduces them and runs the step bookkeeping.  (A
+//            energy, friction, applies leapfrog part 2 and leaves one Partial per block; the first workgroup of
+//            the next step's launch (close_body), or k_finalize (sgk_step.hip), reduces them and closes the step.  (A
 //            last-block reduction inside k_force needs a device-scope release fence per block, which
 //            on gfx950 writes back and invalidates the XCD's L2 - it cost more than the pass itself.)
 // Precision: displacement vectors, cutoff tests and, for the stiff graphene terms, the bond-length

@@ -8,9 +8,10 @@
 //               positions with each atom's index in w (padded with a far-away point to a multiple
 //               of 8), so a list walk reads one 16-byte entry per candidate; every atom clears its
 //               cell's count in cur for the rebuild after this one.  No global counter is involved.
-//   k_nlc       the lists in the reference order from the sorted cells: lanes per metal atom, one
-//               lane per carbon in cell order (nl_scheme 3, the default; schemes 0-2: k_nl, k_nlt).
-//   commit      cellbuf = nxt (the step reduction, or k_commit).
+//   k_nl9, k_nlc  the lists in the reference order from the sorted cells: nine lanes per atom in small
+//               systems, else lanes per metal atom and one lane per carbon in cell order (nl_scheme 3,
+//               the default; schemes 0-2: k_nl, k_nlt).
+//   commit      cellbuf = nxt (the closing of the step, or k_commit).
 // The API path (sgk_bin) bins with k_bin.  In the device-resident loop the kernels return at once
 // unless state.nebrNow is set, so a captured step needs no host decision.
 //

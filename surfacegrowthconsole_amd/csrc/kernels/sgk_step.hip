@@ -2,9 +2,9 @@
 //
 // The reference copies nine reduction results to the host every step and decides on the host
 // whether to rebuild the neighbour list (SurfaceGrowth.cu:2242-2395).  Here the force kernels leave
-// one Partial per block and k_finalize (one workgroup) reduces them in a fixed order, evaluates the
-// same host arithmetic on the device, updates dispHi / nebrNow / shear and appends an sgk_record,
-// so consecutive steps run without any host round trip.
+// one Partial per block; the next step's kernels (StepClose, sgk_reduce.h) or k_finalize (one workgroup)
+// reduce them in a fixed order, evaluate the same host arithmetic on the device, update dispHi / nebrNow /
+// shear and append an sgk_record, so consecutive steps run without any host round trip.
 #include "sgk_batch.h"
 #include "sgk_cells.h"
 #include "sgk_device.h"
