@@ -18,6 +18,23 @@ __device__ __forceinline__ void partial_identity(Partial<T> &q) {
     }
 }
 
+// What an atom brings to a maximum or a minimum: its value, or the identity where that is a NaN.  A
+// comparison keeps or drops a NaN by the side it stands on, so joins in another order would decide
+// differently; with none among the values, every closing of a step takes the same maximum.
+template <class T>
+__device__ __forceinline__ T number_or(T v, T none) {
+    return v == v ? v : none;
+}
+// The metal's bounding box is joined from these.
+template <class T>
+__device__ __forceinline__ void box_of(Partial<T> &q) {
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        q.bmin[d] = number_or(q.com[d], T(3.0e38f));
+        q.bmax[d] = number_or(q.com[d], T(-3.0e38f));
+    }
+}
+
 template <class T>
 __device__ __forceinline__ void partial_combine(Partial<T> &r, const Partial<T> &s) {
     r.u += s.u;
@@ -89,7 +106,7 @@ __device__ __forceinline__ T half_sum(bool hi, T a, T b) {
 }
 
 // A workgroup's v^2 maximum: into its place, or joined with a replica's others (as the bits of a double,
-// which order non-negative values; a NaN is left out, as OpMax leaves it).
+// which order non-negative values; 0 is what a step starts from).
 template <class T>
 __device__ __forceinline__ void store_vmax(T r, T *vmax, unsigned long long *vmaxAll) {
     if (vmax) *vmax = r;
