@@ -260,6 +260,10 @@ int sgk_batch_create(int nrep, const SimParams *params, const sgk_config *cfgIn,
             return bfail(nullptr, SGK_E_UNSUPPORTED, "batched replicas must be regime 0 or 2");
         if (s.cells.x <= 0 || s.cells.y <= 0 || s.cells.z <= 0)
             return bfail(nullptr, SGK_E_ARG, "replica " + std::to_string(r) + ": empty cell grid");
+        // as prepare_ctx: the list kernels index a replica's cell-ordered positions in 32 bits
+        if ((long long)s.cells.x * s.cells.y * s.cells.z * cfg.cell_capacity >= (1ll << 31))
+            return bfail(nullptr, SGK_E_UNSUPPORTED, "replica " + std::to_string(r) +
+                                                         ": cell grid too large: cells x cell capacity must stay below 2^31");
         if (s.sizeHistRdf <= 0 || s.sizeHistRdf > 8192) return bfail(nullptr, SGK_E_ARG, "RDF bins must be 1..8192");
         if (const char *m = mismatch(s0, s))
             return bfail(nullptr, SGK_E_ARG, "replica " + std::to_string(r) + " differs from replica 0 in " + m);
