@@ -582,6 +582,9 @@ __device__ __forceinline__ void close_body(const DevParams &p, const StepClose<A
     rec.nebrNow = step_next(p, c.old, P.vmax).nebrNow;  // its own rule's: a batch may rebuild for another replica
     rec.errors = c.st->errPrev;
     rec.dispHi = c.st->dispHi;
+    // Without an increment the rule only rounds the shear to A; it needs the sums, so k_bin_next leaves it
+    // to this place.  With one, a launch that takes the sums (k_lf1_next) has applied it.
+    if (p.deltaF == 0.f) c.st->shear = shear_next(p, rec.step, c.st->shear, cmVelX);
     rec.shear = c.st->shear;
     rec.shearCount = (double)c.old->shearCount;
     rec.nMolDeposited = c.st->nMolDeposited;
