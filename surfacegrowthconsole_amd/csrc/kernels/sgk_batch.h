@@ -47,7 +47,7 @@ struct BatchArgs {
     uint4 *bondC, *bondA;
     void *partials, *partialsOld;           // Old: of the step that this one closes (a folded step)
     DevState *state, *stateOld;
-    unsigned long long *vmax, *vmaxOld;     // per replica, the step's v^2 maximum (bits of a double >= 0)
+    unsigned long long *vmax, *vmaxOld;     // per replica, a folded step's v^2 maximum (bits of a double >= 0)
     sgk_record *records;
     int recCap;
     unsigned *hist;

@@ -128,7 +128,7 @@ void enqueue_batch(sgk_batch *b, const std::string &flags) {
         sgk::launch_batch_sortcells(b);
         sgk::launch_batch_nl(b);
         sgk::launch_batch_rho(b);
-        sgk::launch_batch_force(b, pre[s], fuse[s] ? b->posAlt : nullptr, folded);
+        sgk::launch_batch_force(b, pre[s], fuse[s] ? b->posAlt : nullptr, folded, fold[s]);
         if (!fold[s]) sgk::launch_batch_finalize(b);
         kicked = pre[s];
         drifted = fuse[s];

@@ -955,7 +955,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
 }
 
 // Batched: each replica's workgroups write into its own range of partials.  With a step to close, the first
-// nClose workgroups close one replica's each.
+// nClose workgroups close one replica's each.  a.vmax only where the next step's first kernel takes the
+// maxima (a folded step): one address per replica serialises its workgroups' atomics, ~5 ns each, which a
+// replica of 1,925 workgroups (464,800 atoms, FP32) paid with 10 us a step although nothing is folded above kFoldParts.
 template <bool M, class T, int G>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void kb_force(BatchArgs a, int nClose, int integrate) {
     using R = typename Prec<M>::R;
@@ -984,7 +986,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
                          (R *)a.vel + 3 * B.atomOff, (R *)a.acc + 3 * B.atomOff, a.nlM + B.metalOff * p.nlCap,
                          a.nnM + B.metalOff, a.embF + B.metalOff, a.embDF + B.metalOff, a.fric + B.metalOff,
                          a.lj + B.carbonOff * p.ljCap, a.nlj + B.carbonOff, a.bondC + B.carbonOff,
-                         a.bondA + B.carbonOff, (Partial<A> *)a.partials + B.partOff, nullptr, a.vmax + e.x, integrate);
+                         a.bondA + B.carbonOff, (Partial<A> *)a.partials + B.partOff, nullptr, a.vmax ? a.vmax + e.x : nullptr, integrate);
 }
 
 // ---- launchers ---------------------------------------------------------------------------------
@@ -1066,13 +1068,14 @@ int batch_lane_index(int G) { return G == 1 ? 0 : G == 2 ? 1 : G == 4 ? 2 : G ==
 // One launch per lane count present: the replicas with G lanes per metal atom, through their own
 // block table (the kernel body is templated on G).
 template <bool M, class T>
-static void batch_dispatch(sgk_batch *b, bool force, int integrate, void *posOut, bool closePrev) {
+static void batch_dispatch(sgk_batch *b, bool force, int integrate, void *posOut, bool closePrev, bool fold) {
     int nClose = closePrev ? b->nrep : 0;  // in the first launch
     static const int kinds[sgk_batch::kLaneKinds] = {1, 2, 4, 8, 16};
     for (int q = 0; q < sgk_batch::kLaneKinds; ++q) {
         if (b->grpN[q] == 0) continue;
         BatchArgs a = b->args();
         a.posOut = posOut;
+        if (!fold) a.vmax = nullptr;
         a.forceTab = b->forceTab + b->grpOff[q];
         const dim3 g((force ? nClose : 0) + b->grpN[q]), t(256);
 #define SGK_B(GG)                                                                            \
@@ -1094,20 +1097,21 @@ static void batch_dispatch(sgk_batch *b, bool force, int integrate, void *posOut
     }
 }
 
-static void batch_launch(sgk_batch *b, bool force, int integrate, void *posOut = nullptr, bool closePrev = false) {
+static void batch_launch(sgk_batch *b, bool force, int integrate, void *posOut = nullptr, bool closePrev = false,
+                         bool fold = false) {
     if (b->nForceBlocks == 0) return;
     if (integrate != 2) posOut = nullptr;  // the drift follows the next step's half-kick only
     if (!b->mixed)
-        batch_dispatch<false, float>(b, force, integrate, posOut, closePrev);
+        batch_dispatch<false, float>(b, force, integrate, posOut, closePrev, fold);
     else if (b->cfg.pair_fp64)
-        batch_dispatch<true, double>(b, force, integrate, posOut, closePrev);
+        batch_dispatch<true, double>(b, force, integrate, posOut, closePrev, fold);
     else
-        batch_dispatch<true, float>(b, force, integrate, posOut, closePrev);
+        batch_dispatch<true, float>(b, force, integrate, posOut, closePrev, fold);
 }
 
 void launch_batch_rho(sgk_batch *b) { batch_launch(b, false, 0); }
-void launch_batch_force(sgk_batch *b, bool prekick, void *posOut, bool closePrev) {
-    batch_launch(b, true, prekick ? 2 : 1, posOut, closePrev);
+void launch_batch_force(sgk_batch *b, bool prekick, void *posOut, bool closePrev, bool fold) {
+    batch_launch(b, true, prekick ? 2 : 1, posOut, closePrev, fold);
 }
 void launch_batch_force_eval(sgk_batch *b) { batch_launch(b, true, 0); }
 

@@ -263,7 +263,9 @@ RdfGrid rdf_grid(const DevParams &p, int S);  // complete-range RDF grid, cells 
 void launch_rho(sgk_ctx *c);
 void launch_batch_rho(sgk_batch *b);
 int batch_lane_index(int G);  // position of G in the lane kinds 1, 2, 4, 8, 16
-void launch_batch_force(sgk_batch *b, bool prekick = false, void *posOut = nullptr, bool closePrev = false);
+// closePrev: the first workgroups close the previous step; fold: the next step closes this one (it takes the maxima).
+void launch_batch_force(sgk_batch *b, bool prekick = false, void *posOut = nullptr, bool closePrev = false,
+                        bool fold = false);
 void launch_batch_force_eval(sgk_batch *b);  // forces and energies only: velocities untouched
 // prekick: the force pass also applies the next step's first half-kick (the caller guarantees that
 // nothing touches velocities or accelerations before that step's launch_lf1(kicked = true)).

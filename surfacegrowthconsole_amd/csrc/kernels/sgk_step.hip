@@ -322,7 +322,6 @@ __global__ __launch_bounds__(kFinalizeThreads) void kb_finalize(BatchArgs a) {
     }
     finalize_body<A>(B.p, part, map, totals, a.state + blockIdx.x,
                      a.records + (size_t)blockIdx.x * a.recCap, a.recCap, 0);
-    if (threadIdx.x == 0) a.vmax[blockIdx.x] = 0ull;
 }
 
 // ApplyBerendsenThermostat (SurfaceGrowth.cu:455-485), kinetic energy of all atoms.
