@@ -107,13 +107,14 @@ void enqueue_batch(sgk_batch *b, const std::string &flags) {
     }
     // and a fused step with no sample behind it is closed by the next step's kernels, an even number again
     bool unfuseFirst = (nPre & 1) != 0;
+    const bool canFold = b->canFold && !(b->cfg.sync_rebuilds && b->nrep > kFoldSync);
     std::vector<char> fuse(n, 0), fold(n, 0);
     int nFold = 0;
     for (size_t s = 0; s < n; ++s) {
         if (!pre[s] || !b->posAlt) continue;
         fuse[s] = !unfuseFirst;
         unfuseFirst = false;
-        fold[s] = fuse[s] && flags[s] == 'a' && b->canFold;
+        fold[s] = fuse[s] && flags[s] == 'a' && canFold;
         nFold += fold[s];
     }
     for (size_t s = 0; (nFold & 1) && s < n; ++s)

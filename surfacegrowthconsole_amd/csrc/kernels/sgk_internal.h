@@ -139,6 +139,11 @@ inline int metal_blocks(long long nMe, int G, int xcdMap) {
 // without / with it (us), sheared FP32 9,417 atoms 24.8 / 21.5, 47,776 36.0 / 32.6, 119,200 43.7 / 42.0,
 // mixed 119,200 53.8 / 53.2; deposition 17,196 24.1 / 19.0, 205,100 67.9 / 53.0.
 constexpr int kCloseLf1Parts = sgk::kFoldParts;
+// Most replicas of a batch with synchronised rebuilds whose steps are folded: every workgroup of
+// kb_bin_next goes through all of them.  Whole step with closing launches / folded (us): 500 replicas of 525 atoms
+// (FP32) 64.3 / 59.9, 1,000 99.6 / 93.5, 1,500 132.1 / 130.9, 2,000 168.8 / 176.9, 4,000 363 / 454; 1,000 of 1,161
+// (mixed) 356.9 / 354.3, 2,000 740 / 766.
+constexpr int kFoldSync = 1024;
 // The force pass's partials of a step.
 inline sgk::PartMap part_map(const sgk_ctx *c) { return {c->nbM, c->nbM + c->nbC, c->carbonLanes == 4}; }
 

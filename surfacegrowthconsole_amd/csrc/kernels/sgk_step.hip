@@ -101,8 +101,9 @@ __global__ __launch_bounds__(256) void kb_lf1(BatchArgs a, int kicked, int syncN
 
 // Batched k_bin_next: the drifted step after a folded one (StepClose, sgk_reduce.h).  The replicas' v^2
 // maxima come joined from the force pass, so that a workgroup can also tell what every other replica's
-// rule asks for (syncN > 0).  Whole step with closing launches / folded (us): 8 replicas of 22,000 atoms together
-// (FP32) 26.6 / 24.0, 64 replicas of 413,000 107.5 / 103.4.
+// rule asks for (syncN > 0; what the rule reads of the parameters, all replicas share).  Whole step with
+// closing launches / folded (us): 8 replicas of 22,000 atoms together (FP32) 26.6 / 24.0, 64 replicas of
+// 413,000 107.5 / 103.4.
 template <bool M>
 __global__ __launch_bounds__(256) void kb_bin_next(BatchArgs a, int syncN) {
     using A = typename Prec<M>::A;
@@ -113,15 +114,9 @@ __global__ __launch_bounds__(256) void kb_bin_next(BatchArgs a, int syncN) {
     auto vmax = [&](int r) { return (A)__longlong_as_double((long long)a.vmaxOld[r]); };
     StepNext<A> s = step_next(B.p, old, vmax(e.x));
     if (syncN > 0) {
-        __shared__ int any;
-        if (threadIdx.x < 64) {
-            int f = 0;
-            for (int r = threadIdx.x; r < syncN; r += 64) f |= step_next(a.reps[r].p, a.stateOld + r, vmax(r)).nebrNow;
-            f = __any(f) ? 1 : 0;
-            if (threadIdx.x == 0) any = f;
-        }
-        __syncthreads();
-        s.nebrNow = any;
+        int f = 0;
+        for (int r = threadIdx.x; r < syncN; r += 256) f |= step_next(B.p, a.stateOld + r, vmax(r)).nebrNow;
+        s.nebrNow = __syncthreads_or(f) ? 1 : 0;
     }
     if (e.y == 0 && threadIdx.x == 0)
         advance_state(st, old, s, old->shear, deposited_next(B.p, s.step, old->nMolDeposited));
