@@ -409,6 +409,19 @@ __device__ __forceinline__ Partial<A> sum_parts(const Partial<A> *part, const Pa
     return total;
 }
 
+// Total of n > 256 chunk totals by one workgroup of 256, returned to thread 0: a thread joins whole partials
+// t, t + 256, ... and the workgroup's tree the threads'.  The sums are sum_parts's, bit for bit.  Its loads
+// are all in flight, where sum_parts walks a field's totals one by one; up to 256 each thread has one, and there
+// sum_parts is the quicker.  sgk_eval_props by sum_parts / so (us, mixed): 44,353 atoms (174 totals) 30.6 / 31.2,
+// 82,000 (321) 40.0 / 32.7, 163,280 (638) 49.6 / 34.6, 1.1 M (4,311) 162 / 60.
+template <class A>
+__device__ Partial<A> sum_strided(const Partial<A> *part, int n) {
+    Partial<A> q;
+    partial_identity(q);
+    for (int k = threadIdx.x; k < n; k += blockDim.x) partial_combine(q, part[k]);
+    return block_reduce_partial(q);
+}
+
 // The sums of a record, with the reference's host arithmetic (SurfaceGrowth.cu:2307-2395); returns the
 // metal's x velocity and the kinetic sum that the thermostat takes.
 template <class A>
@@ -468,11 +481,11 @@ __device__ __forceinline__ int deposited_next(const DevParams &p, int step, int 
 // reference's host arithmetic of SurfaceGrowth.cu:2307-2395 in thread 0.
 // mode 0: one step - advance the step counter, commit a rebuild, update dispHi / nebrNow / shear,
 //         append a record.  mode 1: evaluation only - write records[0], leave the state alone.
-template <class A>
+template <class A, bool STRIDED = false>
 __device__ void finalize_body(const DevParams &p, const Partial<A> *part, const PartMap &map, bool totals, DevState *st,
                               sgk_record *records, int recCap, int mode) {
     const DevState s0 = *st;  // before the sums: its latency passes meanwhile
-    const Partial<A> P = sum_parts(part, map, totals);
+    const Partial<A> P = STRIDED ? sum_strided(part, map.stored) : sum_parts(part, map, totals);
     if (threadIdx.x != 0) return;
     const int nMe = p.nMolMe;
     sgk_record rec;

@@ -290,12 +290,12 @@ __global__ __launch_bounds__(256) void k_reduce1(const Partial<typename Prec<M>:
     if (j * kPartChunk < map.count()) reduce_chunk(part, map, j, part2 + j);
 }
 
-template <bool M>
+template <bool M, bool STRIDED>
 __global__ __launch_bounds__(kFinalizeThreads) void k_finalize(DevParams p,
                                                                const Partial<typename Prec<M>::A> *__restrict__ part,
                                                                PartMap map, int totals, DevState *st,
                                                                sgk_record *records, int recCap, int mode) {
-    finalize_body<typename Prec<M>::A>(p, part, map, totals, st, records, recCap, mode);
+    finalize_body<typename Prec<M>::A, STRIDED>(p, part, map, totals, st, records, recCap, mode);
 }
 
 // Batched: one workgroup per replica, which also reduces the chunks where the partials are too many to
@@ -576,8 +576,10 @@ static void finalize_dispatch(sgk_ctx *c, int mode) {
         part += c->part2Off;
         map = plain_map(nChunks);
     }
-    hipLaunchKernelGGL(k_finalize<M>, dim3(1), dim3(kFinalizeThreads), 0, c->stream, c->dp, part, map, (int)totals,
-                       c->state, c->records, mode == 1 ? 1 : c->cfg.records_capacity, mode);
+    const bool strided = totals && map.count() > kFinalizeThreads;
+    hipLaunchKernelGGL((strided ? k_finalize<M, true> : k_finalize<M, false>), dim3(1), dim3(kFinalizeThreads), 0,
+                       c->stream, c->dp, part, map, (int)totals, c->state, c->records,
+                       mode == 1 ? 1 : c->cfg.records_capacity, mode);
 }
 
 // The first reduction stage alone, for a step whose closing is folded into the next one: chunk totals
