@@ -1,5 +1,6 @@
-"""The densities as they come back through the pinned stage, which serves the
-other transfers too, against the FP64 oracle, atom by atom.  Bound: the mixed form's densities differ from the oracle's by up to 1e-6 of the largest."""
+"""The densities as they come back through the pinned stage, which serves the other transfers too, against
+the FP64 oracle, atom by atom.  Bound: the mixed form's densities differ from the oracle's by up to 1e-6
+of the largest."""
 import ctypes
 
 import numpy as np
