@@ -297,7 +297,7 @@ int sgk_batch_create(int nrep, const SimParams *params, const sgk_config *cfgIn,
     const int G = cfg.metal_lanes;
     const bool fixedG = G == 1 || G == 2 || G == 4 || G == 8 || G == 16;
     for (int r = 0; r < nrep; ++r) b->repLanes.push_back(fixedG ? G : default_lanes(params[r].nMolMe));
-    b->nlNine = sumAtoms <= sgk::kNlNineAtoms;
+    b->nlNine = sgk::nl_nine(sumCarbons, sumAtoms - sumCarbons);
     // replica table and block tables; per-replica workgroup decomposition as in sgk_ctx
     std::vector<int2> atomTab, metalTab, nlTab, nlTabC;
     long long atomOff = 0, metalOff = 0, carbonOff = 0, cellOff = 0, ordOff = 0;

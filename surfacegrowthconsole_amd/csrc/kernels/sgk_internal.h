@@ -106,8 +106,16 @@ constexpr int kNlMetalLanes = 4;
 // one-lane build in instructions; whole steps at 900-1,000 K, one-lane / nine-lane (us): 1,161 atoms
 // 39.3 / 34.6, 44,353 49.8 / 41.0, 129,120 53.1 / 48.0, 275,880 85.7 / 84.8, 440,000 107.7 / 114.9,
 // 1.1 M 224 / 248; batches of 373,577 atoms 112.9 / 113.0, of 448,542 125.0 / 127.4.
+// A metal atom has four lanes otherwise, and a column of its cells up to 72 candidates: it pays for nine lanes only beside
+// carbons, whose one lane under a cluster is the longest chain of the launch.  A rebuild on thermal
+// positions, four lanes / nine: bulk metal 10,976 atoms 50.6 / 36.8, 19,652 52.5 / 46.7, 32,000 49.8 / 57.6, 108,000
+// 99.4 / 145, 256,000 169 / 294; clusters on a sheet, 30,000 + 3,520 C 86.2 / 52.4, 60,000 + 53,760 C 105 / 84.3,
+// 100,000 + 30,720 C 128 / 111, 150,000 + 30,720 C 147 / 150, 200,000 + 53,760 C 184 / 199.
 constexpr int kNineAtoms = 4 * 7;
-constexpr int kNlNineAtoms = 1 << 18;
+constexpr int kNlNineAtoms = 1 << 18, kNlNineMetal = 1 << 17, kNlNineBulk = 28 << 10;
+inline bool nl_nine(long long nC, long long nMe) {
+    return nC + nMe <= kNlNineAtoms && nMe <= (nC > 0 ? kNlNineMetal : kNlNineBulk);
+}
 // A system, or a batch in all, of up to so many carbons takes four lanes per carbon in the density and
 // force passes: there one lane's chain, not the chip's throughput, sets the time.  The results are the
 // same bits either way.  Whole step with one lane / four (us), FP64 pairs unless said: 1,161 atoms

@@ -859,7 +859,7 @@ __device__ __forceinline__ void nlc_body(const DevParams &p, int blk, const type
 // masks; a scan over the atom's nine lanes gives the list position of each column's first entry (the
 // columns in table order, so the lists are those of the walks above, bit for bit); each lane then
 // writes its own entries.  The columns' setup and the scans are paid per nine lanes instead of once,
-// so the walks above keep the sizes where the chip is full (kNlNineAtoms).  Bound by its two rounds
+// so the walks above keep the sizes where the chip is full (nl_nine).  Bound by its two rounds
 // of dependent loads below ~50 k atoms and by VALU issue above.
 
 // A lane's column: three cells back to back; candidate v is entry v + o of the cell-ordered positions.
@@ -1643,7 +1643,7 @@ void launch_nl(sgk_ctx *c, bool force) {
     const unsigned g = blocks_for(c->dp.nMol, 256);
     const int fromNext = force ? 0 : 1;  // step path: build from the new buffer before the commit
     if (c->dp.nlScheme == 3) {
-        const bool nine = c->dp.nMol <= kNlNineAtoms;
+        const bool nine = nl_nine(c->dp.nC, c->dp.nMolMe);
         const int nbM = nine ? (int)blocks_for(c->dp.nMolMe, kNineAtoms)
                              : (int)blocks_for((long long)c->dp.nMolMe * kNlMetalLanes, 256);
         const unsigned gc = (unsigned)nbM + blocks_for(c->dp.nC, nine ? kNineAtoms : 256);
