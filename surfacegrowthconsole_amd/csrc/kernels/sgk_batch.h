@@ -35,7 +35,7 @@ struct BatchArgs {
     const int2 *forceTab;  // (replica, block) over each replica's nbM + nbC force/density blocks
     const int2 *metalTab;  // (replica, block) over each replica's metal atoms
     const int2 *nlTab;     // (replica, block) over each replica's cell-ordered list-build blocks
-    const int2 *rdfTab;    // (replica, chunk) over each replica's metal atoms, rdf_chunk atoms each
+    const int2 *rdfTab;    // (replica, workgroup) over each replica's metal atoms, rdf_chunk atoms each
     const int *order;      // list-build order: replica r's atoms (local indices) at [atomOff, atomOff + nMol)
     void *pos, *vel, *acc;
     void *posOut;          // the force pass's fused drift writes here (null: no drift)

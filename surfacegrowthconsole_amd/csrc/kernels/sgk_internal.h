@@ -127,7 +127,12 @@ inline int carbon_lanes(long long nC) { return nC <= kQuadCarbons ? 4 : 1; }
 inline int carbon_blocks(long long nC, int lanes) { return (int)((nC + 255) / 256) * lanes; }
 // Reference-stencil RDF.
 constexpr int kRdfAtoms = 8;          // atoms a workgroup takes at once
-constexpr int kRdfBlocks = 512;       // workgroups per launch at most: each merges its bins into one histogram
+// Workgroups per launch at most: each merges its bins into one histogram, and fewer leave too few waves in
+// flight.  A sample by one lane per atom / 512 workgroups of a run of atoms each / 512 taking groups in turn / 1,024 /
+// 2,048 so (us, mixed, then FP32): clusters of 30,000 257 / 82 / 77 / 73 / 73, 238 / 72 / 68 / 61 / 71; 100,000
+// 308 / 242 / 218 / 198 / 186, 282 / 190 / 176 / 130 / 122; bulk metal of 256,000 683 / 704 / 612 / 561 / 563,
+// 514 / 592 / 510 / 367 / 339; of 864,000 1,590 / 2,087 / 1,822 / 1,573 / 1,588, 1,230 / 1,803 / 1,468 / 1,012 / 1,005.
+constexpr int kRdfBlocks = 1024;
 inline int rdf_chunk(long long nMe) {  // atoms per workgroup (at least one group)
     const long long groups = (nMe + kRdfAtoms - 1) / kRdfAtoms;
     return kRdfAtoms * (int)std::max<long long>(1, (groups + kRdfBlocks - 1) / kRdfBlocks);

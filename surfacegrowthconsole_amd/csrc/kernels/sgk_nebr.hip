@@ -1375,13 +1375,14 @@ __global__ void k_commit(DevState *st) {
 }
 
 // EvalRdfK (SurfaceGrowth.cu:1895-1999): metal-metal pairs of the 27-cell stencil of the current
-// cells, r^2 < rangeRdf^2, bin = int(sqrt(r^2) * intervalRdf), for metal atoms [i0, i1).  27 lanes per
+// cells, r^2 < rangeRdf^2, bin = int(sqrt(r^2) * intervalRdf), by workgroup blk of nBlk.  27 lanes per
 // atom, one per cell, two atoms a wave: with one lane per atom the chain of ~500 dependent loads was
-// the time whatever the size.  A sample, synchronised: 201 metal atoms 155 -> 19 us, 4,033 220 -> 26,
-// 100,000 294 -> 234.  A cell's slots ascend, so its metal atoms come first.
+// the time whatever the size.  The workgroups take groups of eight atoms in turn, so that those in flight read
+// the same stretch of the system.  A sample, synchronised: 201 metal atoms 155 -> 19 us, 4,033 220 -> 26,
+// 100,000 308 -> 198 (kRdfBlocks).  A cell's slots ascend, so its metal atoms come first.
 // Histogram in LDS, merged with one atomic per bin and block; counts are order independent.
 template <bool M>
-__device__ __forceinline__ void rdf_body(const DevParams &p, int i0, int i1, const typename Prec<M>::P4 *__restrict__ pos,
+__device__ __forceinline__ void rdf_body(const DevParams &p, int blk, int nBlk, const typename Prec<M>::P4 *__restrict__ pos,
                                          const CellBufs &bufs, const DevState *st, unsigned *__restrict__ hist,
                                          unsigned *sh, int *errors) {
     for (int b = threadIdx.x; b < p.sizeHistRdf; b += blockDim.x) sh[b] = 0;
@@ -1392,9 +1393,9 @@ __device__ __forceinline__ void rdf_body(const DevParams &p, int i0, int i1, con
     const int *slots = bufs.slotsB(cb);
     const float range2 = p.rangeRdf2;
     int edge = 0;
-    for (int base = i0; base < i1; base += kRdfAtoms) {
+    for (int base = blk * kRdfAtoms; base < p.nMolMe; base += nBlk * kRdfAtoms) {
         const int i = base + (int)(threadIdx.x >> 5);
-        const int c = i < i1 && o < 27 ? bufs.cellOfB(cb)[i] : -1;
+        const int c = i < p.nMolMe && o < 27 ? bufs.cellOfB(cb)[i] : -1;
         if (c < 0) continue;
         const int ccz = c / (p.cx * p.cy);
         const int ccy = (c - ccz * p.cx * p.cy) / p.cx;
@@ -1431,11 +1432,10 @@ __device__ __forceinline__ void rdf_body(const DevParams &p, int i0, int i1, con
 }
 
 template <bool M>
-__global__ __launch_bounds__(256) void k_rdf(DevParams p, int chunk, const typename Prec<M>::P4 *__restrict__ pos,
+__global__ __launch_bounds__(256) void k_rdf(DevParams p, const typename Prec<M>::P4 *__restrict__ pos,
                                              CellBufs bufs, DevState *st, unsigned *__restrict__ hist) {
     extern __shared__ unsigned sh[];
-    const int i0 = blockIdx.x * chunk;
-    rdf_body<M>(p, i0, min(i0 + chunk, p.nMolMe), pos, bufs, st, hist, sh, &st->errors);
+    rdf_body<M>(p, blockIdx.x, gridDim.x, pos, bufs, st, hist, sh, &st->errors);
 }
 
 // Batched: rdfTab counts workgroups of rdf_chunk atoms over each replica's metal atoms.
@@ -1444,9 +1444,8 @@ __global__ __launch_bounds__(256) void kb_rdf(BatchArgs a, int chunk) {
     extern __shared__ unsigned sh[];
     const int2 e = a.rdfTab[blockIdx.x];
     const BatchRep &B = a.reps[e.x];
-    const int i0 = e.y * chunk;
-    rdf_body<M>(B.p, i0, min(i0 + chunk, B.p.nMolMe), (const typename Prec<M>::P4 *)a.pos + B.atomOff, rep_cells(a, B),
-                a.state + e.x, a.hist + (size_t)e.x * B.p.sizeHistRdf, sh, &a.state[e.x].errors);
+    rdf_body<M>(B.p, e.y, (B.p.nMolMe + chunk - 1) / chunk, (const typename Prec<M>::P4 *)a.pos + B.atomOff,
+                rep_cells(a, B), a.state + e.x, a.hist + (size_t)e.x * B.p.sizeHistRdf, sh, &a.state[e.x].errors);
 }
 
 // ---- complete-range RDF (no counterpart in the reference) ------------------------------------
@@ -1812,11 +1811,11 @@ void launch_rdf(sgk_ctx *c) {
     const int chunk = rdf_chunk(c->dp.nMolMe);
     const dim3 gr(blocks_for(c->dp.nMolMe, chunk));
     if (c->mixed)
-        hipLaunchKernelGGL(k_rdf<true>, gr, dim3(256), shm, c->stream, c->dp, chunk, (const double4 *)c->pos,
-                           cell_bufs(c), c->state, c->hist);
+        hipLaunchKernelGGL(k_rdf<true>, gr, dim3(256), shm, c->stream, c->dp, (const double4 *)c->pos, cell_bufs(c),
+                           c->state, c->hist);
     else
-        hipLaunchKernelGGL(k_rdf<false>, gr, dim3(256), shm, c->stream, c->dp, chunk, (const float4 *)c->pos,
-                           cell_bufs(c), c->state, c->hist);
+        hipLaunchKernelGGL(k_rdf<false>, gr, dim3(256), shm, c->stream, c->dp, (const float4 *)c->pos, cell_bufs(c),
+                           c->state, c->hist);
     profile_end(c, "rdf");
 }
 
