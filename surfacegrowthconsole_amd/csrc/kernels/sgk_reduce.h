@@ -282,8 +282,8 @@ __device__ __forceinline__ StepNext<A> step_next(const DevParams &p, const DevSt
 // (fours, rows of 16, then the rows of a chunk) and so are the sums, bit for bit.
 // totals: the n are chunk totals (any number): thread t of 256 first adds totals t, t + 256, ... in order.
 // Otherwise at most kSumParts partials: chunks of 64, then the chunk totals as the first 16 lanes of a wave.
-// One launch for up to 1,024 partials in place of k_reduce1 and k_finalize: a sheared step of 997 atoms
-// (FP32) 29.1 -> 26.8 us, a deposition step of 4,393 27.2 -> 25.3, kb_finalize of 64 replicas 8.0 -> 6.5.
+// One launch in place of k_reduce1 and k_finalize, for a few partials or beside other work: a sheared step of 997
+// atoms (FP32) 29.1 -> 26.8 us, a deposition step of 4,393 27.2 -> 25.3, kb_finalize of 64 replicas 8.0 -> 6.5.
 constexpr int kSumFours = 64, kSumParts = kFoldParts, kSumGroups = 256 / kPartFields;
 
 // One field of a tree: sums add, the others keep the larger value, minima with their sign turned.

@@ -278,10 +278,14 @@ __global__ __launch_bounds__(256) void k_props(DevParams p, const typename Prec<
     if (threadIdx.x == 0) part[blockIdx.x] = r;
 }
 
-// The step reduction: k_finalize (one workgroup: the sums, then the step's bookkeeping) takes up to
-// kSumParts force-pass partials directly.  More are first reduced to chunk totals by k_reduce1 (one
-// wave per chunk of kPartChunk): a single workgroup over all partials took 26 us at 1.1 M atoms.
+// The step reduction: k_finalize (one workgroup: the sums, then the step's bookkeeping) takes a few chunks of
+// force-pass partials directly.  More are first reduced to chunk totals by k_reduce1 (one wave per chunk of
+// kPartChunk): nothing runs beside that workgroup, and reading them all outlasts a second launch.  A run of
+// one step, all partials direct / by chunk totals (us): a sheet of 997 atoms 26.8 / 29.1, of 32,013 (133
+// partials, with a sample every step) 45.5 / 49.5, of 61,453 (249) 46.3 / 46.3, of 259,085 (1,020) 72.8 / 66.4; bulk
+// metal of 8,788 atoms (280, FP32) 46.1 / 41.2, of 32,000 (1,000) 61.7 / 49.8, mixed 76.0 / 64.7.
 // mode 1 reduces k_props partials, which count as totals.
+constexpr int kFinalizeDirect = 4 * kPartChunk;
 constexpr int kFinalizeThreads = 256;
 template <bool M>
 __global__ __launch_bounds__(256) void k_reduce1(const Partial<typename Prec<M>::A> *__restrict__ part, PartMap map,
@@ -569,7 +573,7 @@ static void finalize_dispatch(sgk_ctx *c, int mode) {
     using A = typename Prec<M>::A;
     Partial<A> *part = (Partial<A> *)c->partials;
     PartMap map = mode == 1 ? plain_map(c->nbProps) : part_map(c);
-    const bool totals = mode == 1 || map.count() > kSumParts;
+    const bool totals = mode == 1 || map.count() > kFinalizeDirect;
     if (mode != 1 && totals) {
         const int nChunks = (map.count() + kPartChunk - 1) / kPartChunk;
         hipLaunchKernelGGL(k_reduce1<M>, dim3((nChunks + 3) / 4), dim3(256), 0, c->stream, part, map, part + c->part2Off);
