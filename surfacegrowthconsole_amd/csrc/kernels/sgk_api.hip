@@ -614,8 +614,8 @@ int sgk_compute_forces(sgk_ctx *c) {
 
 int sgk_get_rho(sgk_ctx *c, double *rho) {
     if (!c || !rho) return SGK_E_ARG;
-    const size_t n = (size_t)c->dp.nMolMe;
-    SGK_HIP(c, sgk::floats_to_host(c->stage, c->device, c->stream, n, c->rho, rho));
+    const sgk::XferArray x = {rho, c->rho, (size_t)c->dp.nMolMe, sgk::XferLayout::plain, false};
+    SGK_HIP(c, sgk::xfer_to_host<double>(c->stage, c->device, c->stream, &x, 1));
     return SGK_OK;
 }
 

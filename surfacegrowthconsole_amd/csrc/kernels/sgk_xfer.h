@@ -52,10 +52,6 @@ struct XferArray {
 // follows on it; on return the host's are complete, or no longer needed.
 template <class H>
 hipError_t xfer_to_host(HostStage &st, int device, hipStream_t s, const XferArray *arrays, int n);
-// n floats of the device as doubles: one copy of the floats to the stage, widened from there.  By a kernel that
-// writes doubles / so / by a pageable copy into a warm or a fresh heap (us): 2,000 floats 15.3 / 14.5 / 17.3,
-// 8,000 16.7 / 12.5 / 12.5 or 24.8, 20,000 21.0 / 17.2 / 17.1 or 43.3, 40,000 30.1 / 24.7 / 23.7, 100,000 46 / 45 / 45.
-hipError_t floats_to_host(HostStage &st, int device, hipStream_t s, size_t n, const float *dev, double *host);
 // The state of n atoms, any of the host arrays null: r 4n, v 3n, a 3n.
 template <class H>
 hipError_t state_to_host(HostStage &st, int device, hipStream_t s, size_t n, bool wide, const void *pos, const void *vel,

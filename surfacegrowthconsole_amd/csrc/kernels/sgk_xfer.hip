@@ -108,17 +108,6 @@ struct Transfer {
     }
 };
 
-// At least so many pinned bytes.
-hipError_t stage_reserve(HostStage &st, size_t bytes) {
-    if (st.bytes >= bytes) return hipSuccess;
-    if (st.pin) (void)hipHostFree(st.pin);
-    st.pin = nullptr;
-    st.bytes = 0;
-    const hipError_t e = hipHostMalloc((void **)&st.pin, bytes, 0);
-    if (e == hipSuccess) st.bytes = bytes;
-    return e;
-}
-
 template <class H, bool OUT>
 hipError_t transfer(HostStage &st, int device, hipStream_t s, const XferArray *arrays, int n) {
     Transfer<H, OUT> x = {s, arrays, n, {}, 0};
@@ -139,9 +128,16 @@ hipError_t transfer(HostStage &st, int device, hipStream_t s, const XferArray *a
     const int threads = bytes >= kXferLarge ? kXferThreads : 1;
     // A small owner keeps small slots.  Below kXferWhole one piece is quicker than two that overlap.
     const size_t slot = std::min(kXferSlot, ((bytes < kXferWhole ? bytes : bytes / 2) + 4095) / 4096 * 4096);
+    const size_t need = 2 * slot * threads;
     x.slot = slot / sizeof(H);
-    hipError_t e = stage_reserve(st, 2 * slot * threads);
-    if (e != hipSuccess) return e;
+    hipError_t e;
+    if (st.bytes < need) {
+        if (st.pin) (void)hipHostFree(st.pin);
+        st.pin = nullptr;
+        st.bytes = 0;
+        if ((e = hipHostMalloc((void **)&st.pin, need, 0)) != hipSuccess) return e;
+        st.bytes = need;
+    }
     for (int k = 0; k < 2 * threads; ++k)
         if (!st.ev[k] && (e = hipEventCreateWithFlags(&st.ev[k], hipEventDisableTiming)) != hipSuccess) return e;
     hipError_t res[kXferThreads] = {};
@@ -183,17 +179,6 @@ void stage_free(HostStage &st) {
     for (hipEvent_t e : st.ev)
         if (e) (void)hipEventDestroy(e);
     st = {};
-}
-
-hipError_t floats_to_host(HostStage &st, int device, hipStream_t s, size_t n, const float *dev, double *host) {
-    const OnDevice here(device);
-    hipError_t e = n ? stage_reserve(st, sizeof(float) * n) : hipSuccess;
-    if (e == hipSuccess && n) e = hipMemcpyAsync(st.pin, dev, sizeof(float) * n, hipMemcpyDeviceToHost, s);
-    const hipError_t done = hipStreamSynchronize(s);
-    if (e == hipSuccess) e = done;
-    const float *f = (const float *)st.pin;
-    for (size_t i = 0; e == hipSuccess && i < n; ++i) host[i] = f[i];
-    return e;
 }
 
 template <class H>
