@@ -235,7 +235,6 @@ int download_vec(sgk_ctx *c, const double *dev, double *host) {
     return SGK_OK;
 }
 
-// Force-pass transpose at the live positions and lists, cotangent already in d.Lam.
 // The context's position buffer again at the end of a scope that points it elsewhere.
 struct KeepPos {
     sgk_ctx *c;
@@ -244,6 +243,7 @@ struct KeepPos {
     ~KeepPos() { c->pos = pos; }
 };
 
+// Force-pass transpose at the live positions and lists, cotangent already in d.Lam.
 void enqueue_vjp(sgk_ctx *c, const AdjDev &d, double wE, bool rho = true) {
     sgk::launch_rho(c);  // the bond and near lists of the current positions
     if (rho) sgk::launch_adj_rho(c, d);

@@ -247,17 +247,22 @@ struct OpSum {
     template <class T>
     __device__ static __forceinline__ T f(T a, T b) { return a + b; }
 };
+// A NaN is left out beside a number (v_max, v_min), on whichever side it stands.
+__device__ __forceinline__ float max_num(float a, float b) { return __builtin_fmaxf(a, b); }
+__device__ __forceinline__ double max_num(double a, double b) { return __builtin_fmax(a, b); }
+__device__ __forceinline__ float min_num(float a, float b) { return __builtin_fminf(a, b); }
+__device__ __forceinline__ double min_num(double a, double b) { return __builtin_fmin(a, b); }
 struct OpMax {
     template <class T>
     __device__ static __forceinline__ T id() { return T(-3.0e38f); }
     template <class T>
-    __device__ static __forceinline__ T f(T a, T b) { return b > a ? b : a; }
+    __device__ static __forceinline__ T f(T a, T b) { return max_num(a, b); }
 };
 struct OpMin {
     template <class T>
     __device__ static __forceinline__ T id() { return T(3.0e38f); }
     template <class T>
-    __device__ static __forceinline__ T f(T a, T b) { return b < a ? b : a; }
+    __device__ static __forceinline__ T f(T a, T b) { return min_num(a, b); }
 };
 
 template <int CTRL>

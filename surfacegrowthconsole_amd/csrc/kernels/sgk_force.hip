@@ -400,8 +400,8 @@ __device__ __forceinline__ Partial<typename Prec<M>::A> metal_body(
         q.vs[2] = (A)vz;
         const A v2 = (A)vx * (A)vx + (A)vy * (A)vy + (A)vz * (A)vz;
         q.vv = m * v2;
-        q.vmax = number_or(v2, A(0));
-        box_of(q);
+        q.vmax = v2;
+        for (int d = 0; d < 3; ++d) q.bmin[d] = q.bmax[d] = q.com[d];
     }
     return q;
 }
@@ -541,7 +541,7 @@ __device__ __forceinline__ Partial<typename Prec<M>::A> carbon_finish(
     // written out: which product a contraction rounds would depend on the code around it
     const A v2 = fmaA((A)vz, (A)vz, fmaA((A)vx, (A)vx, (A)vy * (A)vy));
     q.vv = v2;
-    q.vmax = number_or(v2, A(0));
+    q.vmax = v2;
     return q;
 }
 

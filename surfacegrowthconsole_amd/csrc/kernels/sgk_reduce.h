@@ -18,37 +18,20 @@ __device__ __forceinline__ void partial_identity(Partial<T> &q) {
     }
 }
 
-// What an atom brings to a maximum or a minimum: its value, or the identity where that is a NaN.  A
-// comparison keeps or drops a NaN by the side it stands on, so joins in another order would decide
-// differently; with none among the values, every closing of a step takes the same maximum.
-template <class T>
-__device__ __forceinline__ T number_or(T v, T none) {
-    return v == v ? v : none;
-}
-// The metal's bounding box is joined from these.
-template <class T>
-__device__ __forceinline__ void box_of(Partial<T> &q) {
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        q.bmin[d] = number_or(q.com[d], T(3.0e38f));
-        q.bmax[d] = number_or(q.com[d], T(-3.0e38f));
-    }
-}
-
 template <class T>
 __device__ __forceinline__ void partial_combine(Partial<T> &r, const Partial<T> &s) {
     r.u += s.u;
     r.vir += s.vir;
     r.fr += s.fr;
     r.vv += s.vv;
-    r.vmax = s.vmax > r.vmax ? s.vmax : r.vmax;
+    r.vmax = OpMax::f(r.vmax, s.vmax);
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
         r.com[d] += s.com[d];
         r.cmv[d] += s.cmv[d];
         r.vs[d] += s.vs[d];
-        r.bmin[d] = s.bmin[d] < r.bmin[d] ? s.bmin[d] : r.bmin[d];
-        r.bmax[d] = s.bmax[d] > r.bmax[d] ? s.bmax[d] : r.bmax[d];
+        r.bmin[d] = OpMin::f(r.bmin[d], s.bmin[d]);
+        r.bmax[d] = OpMax::f(r.bmax[d], s.bmax[d]);
     }
 }
 
@@ -159,9 +142,9 @@ __device__ __forceinline__ void block_store_partial(Partial<T> q, Partial<T> *ou
         for (int k = 1; k < 4; ++k) {
             const T x = s[k * kPartFields + f];
             if (f >= kPartBmin && f < kPartBmax)
-                r = x < r ? x : r;
+                r = OpMin::f(r, x);
             else if (f == kPartVmax || (f >= kPartBmax && f < kPartVir))
-                r = x > r ? x : r;
+                r = OpMax::f(r, x);
             else
                 r += x;
         }
@@ -296,7 +279,7 @@ struct Field {
           id(f >= kPartBmin && f < kPartVir ? A(-3.0e38f) : A(0)) {}
     __device__ __forceinline__ A in(A x) const { return turn ? -x : x; }  // its own inverse
     __device__ __forceinline__ A join(A x, A y) const {
-        const A s = x + y, m = y > x ? y : x;
+        const A s = x + y, m = max_num(x, y);
         return sum ? s : m;
     }
     __device__ __forceinline__ A four(A a, A b, A c, A d) const { return join(join(a, b), join(c, d)); }
@@ -403,6 +386,7 @@ __device__ __forceinline__ Partial<A> sum_parts(const Partial<A> *part, const Pa
                 for (int j = 0; j < 16; j += 2 * d) x[j] = fl.join(x[j], x[j + d]);
             r = x[0];
         }
+        r = fl.sum || r == r ? r : fl.id;  // nothing but NaNs: as no atoms, like block_max
         ((A *)&total)[f] = fl.in(r);
     }
     __syncthreads();

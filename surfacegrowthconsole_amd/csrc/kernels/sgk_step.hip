@@ -252,7 +252,7 @@ __global__ __launch_bounds__(256) void k_props(DevParams p, const typename Prec<
         const A vx = (A)vel[n], vy = (A)vel[p.nMol + n], vz = (A)vel[2 * p.nMol + n];
         const A v2 = vx * vx + vy * vy + vz * vz;
         q.u = (A)r.w;
-        q.vmax = number_or(v2, A(0));
+        q.vmax = v2;
         if (n < p.nMolMe) {
             const A m = (A)p.massMe;
             q.fr = fric ? (A)fric[n] : A(0);
@@ -266,7 +266,7 @@ __global__ __launch_bounds__(256) void k_props(DevParams p, const typename Prec<
             q.vs[1] = vy;
             q.vs[2] = vz;
             q.vv = m * v2;
-            box_of(q);
+            for (int d = 0; d < 3; ++d) q.bmin[d] = q.bmax[d] = q.com[d];
         } else {
             q.vs[0] = vx;
             q.vs[1] = vy;
