@@ -74,7 +74,8 @@ Layout plan(const sgk_ctx &c, bool ownFric, bool ownVel) {
     L.fric = ownFric ? k.take(4 * nMe) : 0;
     L.zeroVelBytes = ownVel ? 3 * nMol * R : 0;
     L.zeroVel = ownVel ? k.take(L.zeroVelBytes) : 0;
-    // one per 256 atoms of each kind at 16 lanes per metal atom; a force evaluation alone stores none
+    // One per 256 atoms of each kind at 16 lanes per metal atom.  An evaluation stores none; the place is kept, so
+    // that the scratch a system needs, and with it which systems are taken, stays as callers know it.
     const size_t nParts = std::max<size_t>(((16 * (size_t)p.nMolMe + 255) / 256 + 7) / 8 * 8 + ((size_t)p.nC + 255) / 256,
                                            (nMol + 255) / 256);
     L.partials = k.take((nParts + nParts / 64 + 2) * sgk::partial_bytes_for(c.mixed));

@@ -517,7 +517,7 @@ __device__ void finalize_body(const DevParams &p, const Partial<A> *part, const 
 // launches of its own: the next step's k_bin_next takes the maximum and advances the state into the
 // other DevState, and one workgroup of the next force launch reduces the sums and writes the record
 // while the others work (the force launch, not the density one: its registers cover the reduction, and it
-// is longer than the reduction's ~11 us at 1,000 partials).  The two closing launches cost a small
+// is longer than the reduction's 9 us (FP32) or 12 (mixed) at 1,000 partials).  The two closing launches cost a small
 // step ~6 us of latency.  Whole step, closed by launches / folded (us): 1,161 atoms 34.6 / 29.0,
 // 44,353 41.4 / 35.2, 137,940 (FP32) 50.3 / 45.3, 1.1 M 224.2 / 223.5.
 //
