@@ -81,6 +81,14 @@ __device__ Partial<T> block_reduce_partial(Partial<T> q) {
 // at 44,353, 112.3 -> 110.0 for 64 replicas.
 constexpr int kPartVv = 11, kPartVmax = 12, kPartBmin = 13, kPartBmax = 16, kPartVir = 19, kPartFields = 20;
 
+// Field f of a workgroup's partial as it is stored: the identity for a maximum or minimum over nothing but NaNs.
+// No NaN is then among the values that later joins compare, and every way of closing a step takes the same maximum.
+template <class T>
+__device__ __forceinline__ T held(int f, T r) {
+    if (f < kPartVmax || f >= kPartVir || r == r) return r;
+    return f < kPartBmin ? T(0) : (f < kPartBmax ? T(3.0e38f) : T(-3.0e38f));
+}
+
 // Half of a pair of sums: a lane with `hi` keeps b and gives a away, the others the reverse.
 template <int CTRL, class T>
 __device__ __forceinline__ T half_sum(bool hi, T a, T b) {
@@ -159,6 +167,7 @@ __device__ __forceinline__ void block_store_partial(Partial<T> q, Partial<T> *ou
             }
         }
     }
+    r = held(f, r);
     ((T *)out)[f] = r;
     if (f == kPartVmax) store_vmax(r, vmax, vmaxAll);
 }
@@ -204,6 +213,7 @@ __device__ __forceinline__ void block_store_quad(Partial<T> q, Partial<T> *out, 
             for (int k = 0; k < 16; k += 2 * d) x[k] = f == kPartVmax ? OpMax::f(x[k], x[k + d]) : x[k] + x[k + d];
         r = x[0];
     }
+    r = held(f, r);
     ((T *)out)[f] = r;
     if (f == kPartVmax) store_vmax(r, vmax, vmaxAll);
 }
@@ -279,7 +289,7 @@ struct Field {
           id(f >= kPartBmin && f < kPartVir ? A(-3.0e38f) : A(0)) {}
     __device__ __forceinline__ A in(A x) const { return turn ? -x : x; }  // its own inverse
     __device__ __forceinline__ A join(A x, A y) const {
-        const A s = x + y, m = max_num(x, y);
+        const A s = x + y, m = y > x ? y : x;
         return sum ? s : m;
     }
     __device__ __forceinline__ A four(A a, A b, A c, A d) const { return join(join(a, b), join(c, d)); }
@@ -386,7 +396,6 @@ __device__ __forceinline__ Partial<A> sum_parts(const Partial<A> *part, const Pa
                 for (int j = 0; j < 16; j += 2 * d) x[j] = fl.join(x[j], x[j + d]);
             r = x[0];
         }
-        r = fl.sum || r == r ? r : fl.id;  // nothing but NaNs: as no atoms, like block_max
         ((A *)&total)[f] = fl.in(r);
     }
     __syncthreads();

@@ -114,9 +114,13 @@ __global__ __launch_bounds__(256) void kb_bin_next(BatchArgs a, int syncN) {
     auto vmax = [&](int r) { return (A)__longlong_as_double((long long)a.vmaxOld[r]); };
     StepNext<A> s = step_next(B.p, old, vmax(e.x));
     if (syncN > 0) {
+        __shared__ int any[4];
         int f = 0;
         for (int r = threadIdx.x; r < syncN; r += 256) f |= step_next(B.p, a.stateOld + r, vmax(r)).nebrNow;
-        s.nebrNow = __syncthreads_or(f) ? 1 : 0;
+        f = __any(f) ? 1 : 0;
+        if ((threadIdx.x & 63) == 0) any[threadIdx.x >> 6] = f;
+        __syncthreads();
+        s.nebrNow = any[0] | any[1] | any[2] | any[3];
     }
     if (e.y == 0 && threadIdx.x == 0)
         advance_state(st, old, s, old->shear, deposited_next(B.p, s.step, old->nMolDeposited));
@@ -274,8 +278,14 @@ __global__ __launch_bounds__(256) void k_props(DevParams p, const typename Prec<
             q.vv = v2;
         }
     }
-    const Partial<A> r = block_reduce_partial(q);
-    if (threadIdx.x == 0) part[blockIdx.x] = r;
+    Partial<A> r = block_reduce_partial(q);
+    if (threadIdx.x != 0) return;
+    r.vmax = held(kPartVmax, r.vmax);
+    for (int d = 0; d < 3; ++d) {
+        r.bmin[d] = held(kPartBmin, r.bmin[d]);
+        r.bmax[d] = held(kPartBmax, r.bmax[d]);
+    }
+    part[blockIdx.x] = r;
 }
 
 // The step reduction: k_finalize (one workgroup: the sums, then the step's bookkeeping) takes a few chunks of
